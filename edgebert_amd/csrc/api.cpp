@@ -78,6 +78,16 @@ struct HostTensor {
 struct DevLayer {
     float *wqkv, *bqkv, *wo, *bo, *ln1_g, *ln1_b, *w1, *b1, *w2, *b2, *ln2_g, *ln2_b;
     uint16_t *wqkv16, *wo16, *w116, *w216;
+    // fp32 models whose products run on fp16 pairs (PairScales): the weights
+    // in the pair format
+    uint32_t *wqkvp, *wop, *w1p, *w2p;
+};
+
+// Scales (powers of two) of a layer's pair operands: its input X, the context,
+// the FFN's input (the first LayerNorm's output), the GELU output, and the
+// four weight matrices.
+struct PairScales {
+    float x, ctx, mid, f, wqkv, wo, w1, w2;
 };
 
 struct Workspace {
@@ -137,6 +147,8 @@ struct ebh_model {
     void* wbase = nullptr;
     float *word, *pos, *type0, *emb_g, *emb_b;
     std::vector<DevLayer> layers;
+    void* wpair = nullptr;                 // the pair weights (one allocation), or null
+    std::vector<PairScales> pair_scales;   // per layer, with wpair
     // cross-encoder head (classifier.weight [H], classifier.bias), when loaded
     bool cross_encoder = false;
     float *cls_w = nullptr, *cls_b = nullptr;
@@ -358,6 +370,108 @@ int ensure_host_staging(ebh_model* m, HostSlot& hs, int64_t T, int64_t outn) {
     return EBH_OK;
 }
 
+// The last kernels of a forward: the pool over the final X (or X16), and the
+// cross-encoder's head.
+int enqueue_pool(ebh_model* m, Workspace& w, int B, int S, int normalize, float* d_out, hipStream_t s,
+                 float* d_scores, int prof_kind) {
+    const int H = m->cfg.hidden_size;
+    ProfPair pp{};
+    bool on = false;
+    prof_begin(m, prof_kind, EBH_PROF_POOL, s, pp, on);
+    HIP_TRY(m->dtype == EBH_DTYPE_BF16 ? ebh::launch_pool_b16(w.X16, w.cu, B, H, S, normalize, d_out, s)
+                                       : ebh::launch_pool(w.X, w.cu, B, H, S, normalize, w.Y, d_out, s));
+    prof_end(m, s, pp, on);
+    if (d_scores) HIP_TRY(ebh::launch_cls_head(d_out, m->cls_w, m->cls_b, B, H, d_scores, s));
+    return EBH_OK;
+}
+
+// The encoder layers and the pool of an fp32 forward whose products run on
+// fp16 pairs (after the embeddings, which wrote X and its pairs).  Every
+// operand of a product is written as pairs by the kernel that makes it (4
+// bytes an element, as in fp32); X itself stays fp32 for the residual sums.
+int enqueue_pair_layers(ebh_model* m, Workspace& w, int B, int S, int normalize, float* d_out, hipStream_t s,
+                        float* d_scores, int64_t tokens, int prof_kind, const int* seq_order) {
+    const ebh_config& c = m->cfg;
+    const int H = c.hidden_size, I = c.intermediate_size, nh = c.num_attention_heads, hd = H / nh;
+    const float eps = c.layer_norm_eps, scale = 1.0f / sqrtf((float)hd);
+    // Grids and tiles are sized by the packed rows where the host counted them,
+    // else by B * S.  Every tile sums a product's k in the same order, so only
+    // the split counts bear on the result: those always go by B * S, and the
+    // host and device entry points agree bit for bit.
+    const int T_pad = B * S;
+    const int T = tokens >= 0 && tokens < (int64_t)B * S ? (int)std::max<int64_t>(tokens, 1) : B * S;
+    uint32_t* const xp = reinterpret_cast<uint32_t*>(w.CTX);
+    // Split partials lie T * H floats apart from Y on, into QKV's buffer behind
+    // it (3 rows' worth a token), which nobody reads by then.
+    const int max_splits = (int)std::min<int64_t>(8, ((int64_t)w.y_parts + 3) * w.tok_cap / T_pad);
+    auto gemm = [&](int kind, const void* A, const uint32_t* W, const float* bias, void* C, int N, int K, int epi,
+                    bool out_pair, float acc_scale, float out_scale, const ebh::Gemm16Plan& plan) -> int {
+        ebh::Gemm16Args a{};
+        a.A = A;
+        a.W = W;
+        a.bias = bias;
+        a.C = C;
+        a.lda = a.ldw = K;
+        a.ldc = N;
+        a.M_max = T;
+        a.M_dev = w.ntok;
+        a.N = N;
+        a.K = K;
+        a.splits = plan.splits;
+        a.split_stride = (int64_t)T * N;
+        a.acc_scale = acc_scale;
+        a.out_scale = out_scale;
+        ProfPair p2{};
+        bool on2 = false;
+        prof_begin(m, prof_kind, kind, s, p2, on2);
+        hipError_t e = ebh::launch_gemm16_pair(a, epi, out_pair, plan.tile, s);
+        prof_end(m, s, p2, on2);
+        if (e != hipSuccess) return fail(EBH_ERR_HIP, "gemm launch failed: %s", hipGetErrorString(e));
+        return EBH_OK;
+    };
+    auto add_ln = [&](const float* bias, const float* g, const float* b, int parts, float xs) -> int {
+        ProfPair p2{};
+        bool on2 = false;
+        prof_begin(m, prof_kind, EBH_PROF_LAYERNORM, s, p2, on2);
+        HIP_TRY(ebh::launch_add_layernorm(w.Y, bias, w.X, g, b, T, w.ntok, H, eps, nullptr, s, parts,
+                                          (int64_t)T * H, xs > 0.0f ? xp : nullptr, xs));
+        prof_end(m, s, p2, on2);
+        return EBH_OK;
+    };
+    const int sp_out = ebh::gemm16_pair_plan(T_pad, H, H, false, 1, max_splits).splits,
+              sp_down = ebh::gemm16_pair_plan(T_pad, H, I, false, 1, max_splits).splits;
+    const ebh::Gemm16Plan p_qkv = ebh::gemm16_pair_plan(T, 3 * H, H, false, 1, 1),
+                          p_up = ebh::gemm16_pair_plan(T, I, H, true, 1, 1),
+                          p_out = ebh::gemm16_pair_plan(T, H, H, false, sp_out, sp_out),
+                          p_down = ebh::gemm16_pair_plan(T, H, I, false, sp_down, sp_down);
+    for (size_t l = 0; l < m->layers.size(); ++l) {
+        const DevLayer& L = m->layers[l];
+        const PairScales& q = m->pair_scales[l];
+        int rc;
+        if ((rc = gemm(EBH_PROF_GEMM_QKV, xp, L.wqkvp, L.bqkv, w.QKV, 3 * H, H, ebh::EPI_BIAS, false,
+                       1.0f / (q.x * q.wqkv), 0.0f, p_qkv)))
+            return rc;
+        ProfPair pp{};
+        bool on = false;
+        prof_begin(m, prof_kind, EBH_PROF_ATTENTION, s, pp, on);
+        HIP_TRY(ebh::launch_attention(w.QKV, w.cu, B, S, H, nh, hd, scale, w.CTX, s, seq_order, q.ctx));
+        prof_end(m, s, pp, on);
+        if ((rc = gemm(EBH_PROF_GEMM_OUT, w.CTX, L.wop, nullptr, w.Y, H, H, ebh::EPI_NONE, false,
+                       1.0f / (q.ctx * q.wo), 0.0f, p_out)))
+            return rc;
+        if ((rc = add_ln(L.bo, L.ln1_g, L.ln1_b, p_out.splits, q.mid))) return rc;
+        if ((rc = gemm(EBH_PROF_GEMM_FFN_UP, xp, L.w1p, L.b1, w.F, I, H, ebh::EPI_BIAS_GELU, true,
+                       1.0f / (q.mid * q.w1), q.f, p_up)))
+            return rc;
+        if ((rc = gemm(EBH_PROF_GEMM_FFN_DOWN, w.F, L.w2p, nullptr, w.Y, H, I, ebh::EPI_NONE, false,
+                       1.0f / (q.f * q.w2), 0.0f, p_down)))
+            return rc;
+        const bool last = l + 1 == m->layers.size();
+        if ((rc = add_ln(L.b2, L.ln2_g, L.ln2_b, p_down.splits, last ? 0.0f : m->pair_scales[l + 1].x))) return rc;
+    }
+    return enqueue_pool(m, w, B, S, normalize, d_out, s, d_scores, prof_kind);
+}
+
 // The kernels of one forward on stream s (ids/mask already in device memory).
 // d_scores (optional, cross-encoders): score[b] = pooled[b] . w + bias, from
 // the un-normalised pooled rows left in d_out.
@@ -380,6 +494,13 @@ int enqueue_kernels(ebh_model* m, Workspace& w, const int* d_ids, const int* d_m
     bool on = false;
     const bool bf16 = m->dtype == EBH_DTYPE_BF16;
     const bool few_pack = ebh::pack_embed_few_fits(B, S, H);
+    // fp32 products on fp16 pairs (gemm16.hpp).  Up to 64 rows a product is a
+    // chain of memory round trips, and the few-token kernels stay.
+    const bool pair = m->wpair && T > ebh::SKINNY_MAX_ROWS;
+    // The pair copy of X shares CTX's memory: X is read by the QKV product
+    // before attention writes the context there, and the context by the
+    // output product before the LayerNorm writes the next X.
+    uint32_t* const xp = pair ? reinterpret_cast<uint32_t*>(w.CTX) : nullptr;
     const int* seq_order = few_pack ? nullptr : w.order;   // written by launch_pack only
     if (few_pack) {   // a few short sentences: one launch
         prof_begin(m, prof_kind, EBH_PROF_EMBED, s, pp, on);
@@ -392,9 +513,10 @@ int enqueue_kernels(ebh_model* m, Workspace& w, const int* d_ids, const int* d_m
         prof_begin(m, prof_kind, EBH_PROF_EMBED, s, pp, on);
         HIP_TRY(ebh::launch_embed_ln(w.tok_id, w.tok_pos, w.ntok, T, m->word, m->pos, m->type0,
                                      m->emb_g, m->emb_b, c.vocab_size, H, eps, bf16 ? nullptr : w.X, w.err,
-                                     w.X16, s));
+                                     w.X16, s, xp, pair ? m->pair_scales[0].x : 0.0f));
         prof_end(m, s, pp, on);
     }
+    if (pair) return enqueue_pair_layers(m, w, B, S, normalize, d_out, s, d_scores, tokens, prof_kind, seq_order);
 
     // bf16 models keep the residual stream in bf16 (X16, written by each
     // LayerNorm; every sum and statistic stays fp32) and hand the GEMMs bf16
@@ -540,12 +662,7 @@ int enqueue_kernels(ebh_model* m, Workspace& w, const int* d_ids, const int* d_m
             prof_end(m, s, pp, on);
         }
     }
-    prof_begin(m, prof_kind, EBH_PROF_POOL, s, pp, on);
-    HIP_TRY(bf16 ? ebh::launch_pool_b16(w.X16, w.cu, B, H, S, normalize, d_out, s)
-                 : ebh::launch_pool(w.X, w.cu, B, H, S, normalize, w.Y, d_out, s));
-    prof_end(m, s, pp, on);
-    if (d_scores) HIP_TRY(ebh::launch_cls_head(d_out, m->cls_w, m->cls_b, B, H, d_scores, s));
-    return EBH_OK;
+    return enqueue_pool(m, w, B, S, normalize, d_out, s, d_scores, prof_kind);
 }
 
 // The recorded forward for this call, recording it at the key's second call;
@@ -815,9 +932,11 @@ static void release_partial_finalize(ebh_model* m) {
     (void)hipSetDevice(m->device);
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     if (m->wbase) (void)hipFree(m->wbase);
+    if (m->wpair) (void)hipFree(m->wpair);
     if (m->done) (void)hipEventDestroy(m->done);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     m->wbase = nullptr;
+    m->wpair = nullptr;
     m->noalloc_err = nullptr;
     m->done = nullptr;
     m->stream = nullptr;
@@ -832,6 +951,140 @@ int ebh_finalize(ebh_model* m, int32_t dtype) {
     const int rc = finalize_locked(m, dtype);
     if (rc != EBH_OK && !m->finalized) release_partial_finalize(m);
     return rc;
+}
+
+// The largest power of two s with s * bound <= limit, or 0 where the operand
+// is left to the fp32 kernels: bound or s not an ordinary number, or typical
+// values (typ) more than 2^13 below the bound.  Beyond its own 23 to 24 bits an
+// operand's pair is off by at most 2^-25 / s <= 2^-39 bound, which is then
+// under 2^-26 of a typical value.
+static float pair_scale(double bound, double typ, double limit) {
+    if (!(bound > 0.0) || !(bound <= 1e15) || !(bound <= 8192.0 * typ)) return 0.0f;
+    const int e = (int)std::floor(std::log2(limit / bound));
+    return e >= -40 && e <= 40 ? (float)std::ldexp(1.0, e) : 0.0f;
+}
+
+// fp32 models: the GEMM weights in the pair format beside the fp32 ones (which
+// the few-token kernels read), and a scale for every operand from what it can
+// reach.  A LayerNorm output is at most |gamma_i| sqrt(H) + |beta_i|, and its
+// 2-norm at most max |gamma| sqrt(H) + |beta|; a projection's row is at most
+// |w| |x| + |b|; the context is a mean of v rows, and |gelu(u)| <= |u|.  So no
+// input can overflow an operand.  Where a scale would leave the range in which
+// pairs are as exact as fp32 products (pair_scale), or a shape is not whole
+// 64-wide k-tiles, the model keeps the fp32 kernels throughout.
+static int prepare_pairs(ebh_model* m) {
+    const ebh_config& c = m->cfg;
+    const size_t H = c.hidden_size, I = c.intermediate_size, L = m->layers.size();
+    if (H % 64 || I % 64 || L == 0 || !ebh::row4_shape_ok((int)H)) return EBH_OK;
+    hipStream_t st = m->stream;
+    const size_t rows = 3 * H + H + I + H;               // weight rows of a layer
+    float* d_stats = nullptr;
+    HIP_TRY(hipMalloc((void**)&d_stats, L * rows * 2 * sizeof(float)));
+    std::unique_ptr<void, hipError_t (*)(void*)> stats_guard(d_stats, hipFree);
+    std::vector<float> stats(L * rows * 2);
+    for (size_t l = 0; l < L; ++l) {
+        const DevLayer& d = m->layers[l];
+        float *n2 = d_stats + l * rows * 2, *am = n2 + rows;
+        HIP_TRY(ebh::launch_row_stats(d.wqkv, 3 * (int)H, (int)H, n2, am, st));
+        HIP_TRY(ebh::launch_row_stats(d.wo, (int)H, (int)H, n2 + 3 * H, am + 3 * H, st));
+        HIP_TRY(ebh::launch_row_stats(d.w1, (int)I, (int)H, n2 + 4 * H, am + 4 * H, st));
+        HIP_TRY(ebh::launch_row_stats(d.w2, (int)H, (int)I, n2 + 4 * H + I, am + 4 * H + I, st));
+    }
+    HIP_TRY(hipMemcpyAsync(stats.data(), d_stats, stats.size() * 4, hipMemcpyDeviceToHost, st));
+    // emb g, b; per layer: bv, ln1 g, b, b1, ln2 g, b
+    const size_t per = 5 * H + I;
+    std::vector<float> v(2 * H + L * per);
+    HIP_TRY(hipMemcpyAsync(v.data(), m->emb_g, H * 4, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(v.data() + H, m->emb_b, H * 4, hipMemcpyDeviceToHost, st));
+    for (size_t l = 0; l < L; ++l) {
+        const DevLayer& d = m->layers[l];
+        float* p = v.data() + 2 * H + l * per;
+        const float* src[] = {d.bqkv + 2 * H, d.ln1_g, d.ln1_b, d.ln2_g, d.ln2_b};
+        for (int i = 0; i < 5; ++i) HIP_TRY(hipMemcpyAsync(p + i * H, src[i], H * 4, hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipMemcpyAsync(p + 5 * H, d.b1, I * 4, hipMemcpyDeviceToHost, st));
+    }
+    HIP_TRY(hipStreamSynchronize(st));
+
+    constexpr double kActLimit = 32000.0, kWeightLimit = 32768.0;   // half of fp16's range
+    auto median = [](std::vector<double> a) {
+        std::nth_element(a.begin(), a.begin() + a.size() / 2, a.end());
+        return a[a.size() / 2];
+    };
+    struct Norm { double max, typ, norm; };              // of a LayerNorm's output rows
+    auto norm_of = [&](const float* g, const float* b) {
+        double mx = 0, gm = 0, ss = 0, bb = 0;
+        std::vector<double> size(H);
+        const double root = std::sqrt((double)H);
+        for (size_t i = 0; i < H; ++i) {
+            const double gi = std::fabs((double)g[i]), bi = std::fabs((double)b[i]);
+            mx = std::max(mx, gi * root + bi);
+            gm = std::max(gm, gi);
+            ss += size[i] = std::sqrt(gi * gi + bi * bi);
+            bb += bi * bi;
+        }
+        if (!std::isfinite(ss)) return Norm{NAN, NAN, NAN};   // std::max loses a NaN
+        return Norm{mx, median(std::move(size)), gm * root + std::sqrt(bb)};
+    };
+    // Bound and typical size of the rows of x . w^T + b.
+    auto out_scale = [&](const float* n2, const float* b, size_t n, const Norm& x) {
+        double mx = 0, ss = 0;
+        std::vector<double> size(n);
+        for (size_t i = 0; i < n; ++i) {
+            const double w = std::sqrt((double)n2[i]), bi = std::fabs((double)b[i]);
+            mx = std::max(mx, w * x.norm + bi);
+            ss += size[i] = w * x.typ + bi;
+        }
+        return std::isfinite(ss) ? pair_scale(mx, median(std::move(size)), kActLimit) : 0.0f;
+    };
+    auto weight_scale = [&](const float* n2, const float* am, size_t n) {
+        double mx = 0, mn = 1e300, sum = 0;
+        for (size_t i = 0; i < n; ++i) {
+            mx = std::max(mx, (double)am[i]);
+            if (am[i] > 0) mn = std::min(mn, (double)am[i]);
+            sum += n2[i];
+        }
+        // a row far below the matrix's largest weight would lose bits
+        return std::isfinite(sum) && mx > 0 ? pair_scale(mx, mn, kWeightLimit) : 0.0f;
+    };
+    std::vector<PairScales> sc(L);
+    Norm in = norm_of(v.data(), v.data() + H);
+    for (size_t l = 0; l < L; ++l) {
+        const float *n2 = stats.data() + l * rows * 2, *am = n2 + rows, *p = v.data() + 2 * H + l * per;
+        const Norm mid = norm_of(p + H, p + 2 * H);
+        PairScales& q = sc[l];
+        q.x = pair_scale(in.max, in.typ, kActLimit);
+        q.ctx = out_scale(n2 + 2 * H, p, H, in);
+        q.mid = pair_scale(mid.max, mid.typ, kActLimit);
+        q.f = out_scale(n2 + 4 * H, p + 5 * H, I, mid);
+        q.wqkv = weight_scale(n2, am, 3 * H);
+        q.wo = weight_scale(n2 + 3 * H, am + 3 * H, H);
+        q.w1 = weight_scale(n2 + 4 * H, am + 4 * H, I);
+        q.w2 = weight_scale(n2 + 4 * H + I, am + 4 * H + I, H);
+        for (float f : {q.x, q.ctx, q.mid, q.f, q.wqkv, q.wo, q.w1, q.w2})
+            if (!(f > 0.0f)) return EBH_OK;
+        in = norm_of(p + 3 * H, p + 4 * H);
+    }
+    const size_t words = 4 * H * H + 2 * H * I;          // pair weights of a layer
+    if (hipMalloc(&m->wpair, L * words * 4) != hipSuccess) {   // no room: the fp32 kernels need none
+        (void)hipGetLastError();
+        m->wpair = nullptr;
+        return EBH_OK;
+    }
+    for (size_t l = 0; l < L; ++l) {
+        DevLayer& d = m->layers[l];
+        uint32_t* w = static_cast<uint32_t*>(m->wpair) + l * words;
+        d.wqkvp = w;
+        d.wop = w + 3 * H * H;
+        d.w1p = w + 4 * H * H;
+        d.w2p = w + 4 * H * H + H * I;
+        HIP_TRY(ebh::launch_to_pair(d.wqkv, d.wqkvp, 3 * H * H, sc[l].wqkv, st));
+        HIP_TRY(ebh::launch_to_pair(d.wo, d.wop, H * H, sc[l].wo, st));
+        HIP_TRY(ebh::launch_to_pair(d.w1, d.w1p, H * I, sc[l].w1, st));
+        HIP_TRY(ebh::launch_to_pair(d.w2, d.w2p, H * I, sc[l].w2, st));
+    }
+    HIP_TRY(hipStreamSynchronize(st));
+    m->pair_scales = std::move(sc);
+    return EBH_OK;
 }
 
 static int finalize_locked(ebh_model* m, int32_t dtype) {
@@ -974,6 +1227,7 @@ static int finalize_locked(ebh_model* m, int32_t dtype) {
         d.ln2_g = (float*)(b + o.ln2_g); d.ln2_b = (float*)(b + o.ln2_b);
         d.wqkv = d.wo = d.w1 = d.w2 = nullptr;
         d.wqkv16 = d.wo16 = d.w116 = d.w216 = nullptr;
+        d.wqkvp = d.wop = d.w1p = d.w2p = nullptr;
         if (b16) {
             d.wqkv16 = (uint16_t*)(b + o.wqkv); d.wo16 = (uint16_t*)(b + o.wo);
             d.w116 = (uint16_t*)(b + o.w1); d.w216 = (uint16_t*)(b + o.w2);
@@ -982,6 +1236,7 @@ static int finalize_locked(ebh_model* m, int32_t dtype) {
             d.w1 = (float*)(b + o.w1); d.w2 = (float*)(b + o.w2);
         }
     }
+    if (dtype == EBH_DTYPE_F32 && (rc = prepare_pairs(m))) return rc;
     m->dtype = dtype;
     m->finalized = true;
     m->host.clear();  // weights now live in HBM only (and any mapped file is released)
@@ -998,6 +1253,7 @@ void ebh_destroy(ebh_model* m) {
         drop_graphs(m);
         if (m->ws.base) (void)hipFree(m->ws.base);
         if (m->wbase) (void)hipFree(m->wbase);
+        if (m->wpair) (void)hipFree(m->wpair);
         for (HostSlot& hs : m->slots) {
             if (hs.ids) (void)hipHostFree(hs.ids);
             if (hs.mask) (void)hipHostFree(hs.mask);
@@ -1364,6 +1620,44 @@ int ebh_op_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, int64_t 
     hipError_t e = ebh::launch_gemm_bf16_act(a, epilogue, c_dtype == EBH_DTYPE_BF16,
                                              static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(EBH_ERR_HIP, "gemm launch failed: %s", hipGetErrorString(e));
+    return EBH_OK;
+}
+
+int ebh_op_gemm_pair(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t ldw, float acc_scale,
+                     const float* bias, void* C, int64_t ldc, float c_scale, int32_t M, int32_t N, int32_t K,
+                     int32_t epilogue, int32_t splits, int64_t split_stride, int32_t tile, void* stream) {
+    if (!A || !W || !C || M < 0 || N <= 0 || K <= 0 || splits < 1 || tile < -1 || tile >= ebh::GEMM16_TILES ||
+        !(acc_scale > 0.0f) || !(c_scale >= 0.0f) || epilogue < EBH_EPI_BIAS || epilogue > EBH_EPI_NONE ||
+        epilogue == EBH_EPI_BIAS_RESID || (epilogue == EBH_EPI_BIAS_GELU) != (c_scale > 0.0f) ||
+        (splits > 1 && epilogue != EBH_EPI_NONE))
+        return fail(EBH_ERR_INVALID_ARG, "bad pair gemm arguments");
+    ebh::Gemm16Args a{};
+    a.A = A;
+    a.W = W;
+    a.bias = bias;
+    a.C = C;
+    a.lda = lda;
+    a.ldw = ldw;
+    a.ldc = ldc;
+    a.M_max = M;
+    a.N = N;
+    a.K = K;
+    a.splits = splits;
+    a.split_stride = split_stride;
+    a.acc_scale = acc_scale;
+    a.out_scale = c_scale;
+    if (tile < 0) tile = ebh::gemm16_pair_plan(M, N, K, epilogue == EBH_EPI_BIAS_GELU, splits, splits).tile;
+    const hipError_t e = ebh::launch_gemm16_pair(a, epilogue, c_scale > 0.0f, tile, (hipStream_t)stream);
+    if (e == hipErrorInvalidValue) return fail(EBH_ERR_INVALID_ARG, "pair gemm shape, stride or alignment");
+    if (e != hipSuccess) return fail(EBH_ERR_HIP, "gemm launch failed: %s", hipGetErrorString(e));
+    return EBH_OK;
+}
+
+int ebh_op_to_pair(const float* x, uint32_t* y, int64_t n, float scale, void* stream) {
+    if (!x || !y || n < 0 || !(scale > 0.0f)) return fail(EBH_ERR_INVALID_ARG, "bad pair arguments");
+    const hipError_t e = ebh::launch_to_pair(x, y, n, scale, (hipStream_t)stream);
+    if (e == hipErrorInvalidValue) return fail(EBH_ERR_INVALID_ARG, "n must be a multiple of 8, x and y 16-byte aligned");
+    if (e != hipSuccess) return fail(EBH_ERR_HIP, "launch failed: %s", hipGetErrorString(e));
     return EBH_OK;
 }
 

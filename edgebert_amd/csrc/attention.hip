@@ -125,10 +125,10 @@ __device__ __forceinline__ void attend_chunk(const float* Ks, const float* Vs, c
 // workgroups per CU (c3: 69.5 -> 65.8 us per layer against one 128-key chunk);
 // longer sequences keep 128-key chunks, loaded when they are needed, three
 // workgroups per CU (c4: 53.1 against 53.9 us with 64-key chunks).
-template <int HD, int KC>
+template <int HD, int KC, bool PAIR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ? (KC == 64 ? 4 : 3) : 2))) void attention_kernel(
     const float* __restrict__ qkv, const int* __restrict__ cu_seqlens, float* __restrict__ ctx_out, int H, float scale,
-    const int* __restrict__ order) {
+    const int* __restrict__ order, float pair_scale) {
     constexpr bool PREFETCH = KC == 64;
     constexpr int KS = HD + 4;     // K row stride (floats): conflict-free 16-B reads
     constexpr int NJ = HD / 32;    // 32-wide output blocks of the context
@@ -214,7 +214,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ? 
             for (int g = 0; g < 4; ++g) {
                 const float c0 = o[j][4 * g] * inv, c1 = o[j][4 * g + 1] * inv;
                 const float c2 = o[j][4 * g + 2] * inv, c3 = o[j][4 * g + 3] * inv;
-                *reinterpret_cast<float4*>(ctx_out + at + j * 32 + 8 * g) = make_float4(c0, c1, c2, c3);
+                if constexpr (PAIR) {   // dims 8 g + 4 half ..: half of a 32-byte pair group
+                    uint2 h, l;
+                    split_f16x2(c0 * pair_scale, c1 * pair_scale, h.x, l.x);
+                    split_f16x2(c2 * pair_scale, c3 * pair_scale, h.y, l.y);
+                    uint32_t* const pr = reinterpret_cast<uint32_t*>(ctx_out) + at - 2 * half + j * 32 + 8 * g;
+                    *reinterpret_cast<uint2*>(pr) = h;
+                    *reinterpret_cast<uint2*>(pr + 4) = l;
+                } else {
+                    *reinterpret_cast<float4*>(ctx_out + at + j * 32 + 8 * g) = make_float4(c0, c1, c2, c3);
+                }
             }
     }
 }
@@ -647,22 +656,32 @@ hipError_t launch_attention_bf16(const uint16_t* qkv, const int* cu_seqlens, int
     return hipGetLastError();
 }
 
-hipError_t launch_attention(const float* qkv, const int* cu_seqlens, int B, int max_len, int H,
-                            int nh, int head_dim, float scale, float* ctx, hipStream_t s, const int* order) {
-    if (B <= 0 || max_len <= 0) return hipSuccess;
+template <bool PAIR>
+static hipError_t launch_attention_f32(const float* qkv, const int* cu_seqlens, int B, int max_len, int H,
+                                       int nh, int head_dim, float scale, float* ctx, hipStream_t s, const int* order,
+                                       float pair_scale) {
     const dim3 grid(nh, (max_len + 127) / 128, B), block(256);
     const bool short_seqs = max_len <= 128;
     if (head_dim == 32 && short_seqs)
-        hipLaunchKernelGGL((attention_kernel<32, 64>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order);
+        hipLaunchKernelGGL((attention_kernel<32, 64, PAIR>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order, pair_scale);
     else if (head_dim == 32)
-        hipLaunchKernelGGL((attention_kernel<32, 128>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order);
+        hipLaunchKernelGGL((attention_kernel<32, 128, PAIR>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order, pair_scale);
     else if (head_dim == 64 && short_seqs)
-        hipLaunchKernelGGL((attention_kernel<64, 64>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order);
+        hipLaunchKernelGGL((attention_kernel<64, 64, PAIR>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order, pair_scale);
     else if (head_dim == 64)
-        hipLaunchKernelGGL((attention_kernel<64, 128>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order);
+        hipLaunchKernelGGL((attention_kernel<64, 128, PAIR>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order, pair_scale);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();
+}
+
+hipError_t launch_attention(const float* qkv, const int* cu_seqlens, int B, int max_len, int H,
+                            int nh, int head_dim, float scale, float* ctx, hipStream_t s, const int* order,
+                            float pair_scale) {
+    if (B <= 0 || max_len <= 0) return hipSuccess;
+    return pair_scale > 0.0f
+               ? launch_attention_f32<true>(qkv, cu_seqlens, B, max_len, H, nh, head_dim, scale, ctx, s, order, pair_scale)
+               : launch_attention_f32<false>(qkv, cu_seqlens, B, max_len, H, nh, head_dim, scale, ctx, s, order, 0.0f);
 }
 
 }  // namespace ebh

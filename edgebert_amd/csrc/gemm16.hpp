@@ -1,0 +1,349 @@
+// gemm16.hpp -- GEMM tiles on the 16-bit matrix cores: fp32 products from
+// fp16 pairs, and bf16 products.
+//
+// Pair format.  An fp32 value x of a matrix with scale s (a power of two) is
+// held as two fp16 numbers h = fp16(s x) and l = fp16(s x - h), both rounded
+// to nearest even; s x - h is exact in fp32, and h + l is s x to within one
+// unit of its 24th bit.  Eight consecutive elements of a row take 32 bytes,
+// h0..h7 then l0..l7, so a row of K values takes 4 K bytes as in fp32 and an
+// MFMA operand (8 k-consecutive fp16) is one aligned 16-byte chunk.
+//
+// s a . t b = ah.bh + ah.bl + al.bh, three v_mfma_f32_16x16x32_f16 with every
+// product exact in fp32 and sums in fp32; al.bl, below 2^-22 of |a b|, is left
+// out.  Measured against float64 the relative error of such a product is 0.62
+// of the fp32 MFMA's (K = 384: 2.2e-7 against 3.5e-7; K = 3072: 6.2e-7 against
+// 9.9e-7; the same on GELU outputs and on rows with outlier features), because
+// the fp32 form rounds its sum every k and this one every 32: the pairs'
+// own rounding (2^-24 per operand) is a small part of either.  The error is
+// flat for scales from 2^4 to 2^10, so one scale per matrix, taken from a
+// bound of its values, is enough.
+//
+// The fp16 MFMA rounds its aligned terms down (towards minus infinity), so its
+// sums sit 1e-8 (K = 384) to 4e-8 (K = 1536) of their size low on average, a
+// small part of a sum's own error and nearly the same for every column, which
+// the LayerNorm after the attention-output and FFN-down products takes out.
+#pragma once
+#include <type_traits>
+
+#include "kernels.hpp"
+
+namespace ebh {
+
+typedef float g16_v4f __attribute__((ext_vector_type(4)));
+typedef int g16_v4i __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef __bf16 g16_v8bf __attribute__((ext_vector_type(8)));
+typedef unsigned int u4v_t __attribute__((ext_vector_type(4)));
+
+// Word 3 of a gfx9 buffer resource descriptor for plain dword-addressed
+// buffers; accesses at or past the descriptor's byte count return 0 (loads,
+// into LDS too) or are dropped (stores).
+constexpr int G16_RSRC_WORD3 = 0x00020000;
+
+// One lane's 16 bytes from a buffer straight into LDS at lds_addr + 16 lane
+// (buffer_load_dwordx4 ... lds; offset = voff + soff).  Issued from inline asm
+// so that the compiler does not make every LDS read wait for it; callers
+// count and wait with wait_vmcnt.
+__device__ __forceinline__ void load_lds16_buf(const g16_v4i& rsrc, uint32_t voff, uint32_t soff, uint32_t lds_addr) {
+    uint32_t saved;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %4\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %2, %3 offen lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_addr)
+        : "memory");
+}
+
+__device__ __forceinline__ g16_v4i make_rsrc(const void* base, uint32_t bytes) {
+    const uint64_t b = uniform_u64(base);
+    return g16_v4i{(int)(uint32_t)b, (int)(uint32_t)((b >> 32) & 0xffffu), __builtin_amdgcn_readfirstlane((int)bytes),
+                   G16_RSRC_WORD3};
+}
+
+enum Out16 : int { OUT_F32 = 0, OUT_PAIR = 1, OUT_BF16 = 2 };
+
+// C = epi(A . W^T + bias), one list of work items (C tiles, N-fastest, times
+// the K splits) walked by a persistent grid.  A [M, K] and W [N, K] rows are
+// K-contiguous, in pairs (PAIR) or bf16; a k-tile is 128 bytes of each row
+// (32 pairs or 64 bf16), staged unpadded in LDS with the row's eight 16-byte
+// chunks XOR-swizzled, by direct-to-LDS buffer loads whose descriptors end at
+// the last real row (rows past it read as zeros).
+//
+// Chunks 2q and 2q + 1 of a row are lane group q's operands: h and l of
+// k = 8q .. 8q + 7 (pairs), or two 8-deep runs of k (bf16).  The MFMAs take W
+// as their first operand, so lane (r, q) of a 16 x 16 block holds C row r and
+// the block's W rows 4q .. 4q + 3.  W rows are permuted on their way into LDS
+// (within each 32, LDS row 16 jj + 4q + e holds column 8q + 4 jj + e), so a lane
+// holds eight consecutive columns across two blocks: 32 bytes of fp32 or
+// of a pair chunk, stored straight from the accumulators, four lanes to a
+// 128-byte line.  The epilogue needs no LDS pass and no barrier, and the next
+// k-tile's loads are in flight ahead of its stores.
+//
+// What bounds it: the matrix cores (a 256 x 256 k-tile is 64 KB of loads for
+// 3,072 cycles of MFMAs per SIMD).  A k-tile's fragments are read a step (SB
+// row blocks) ahead and its last step's MFMAs run after the next k-tile's
+// barrier, so that the pipes work while the barrier releases and the first
+// fragments arrive; two sets of W fragments make that possible, and k-tiles
+// come in pairs so that the sets have fixed registers.
+template <bool PAIR, int BM, int BN, int WAVES_M, int WAVES_N, int NST, int EPI, int OUT>
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm16_kernel(Gemm16Args p) {
+    constexpr int NT = 64 * WAVES_M * WAVES_N, NW = WAVES_M * WAVES_N;
+    constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
+    constexpr int FM = WM / 16, FN = WN / 16;
+    static_assert(FM * 16 == WM && FN * 16 == WN && FN % 2 == 0, "wave tile of 16 x 32 blocks");
+    constexpr int SB = FM >= 8 ? 2 : 1, NS = FM / SB;
+    static_assert(NS % 2 == 0, "steps alternate between two A sets");
+    constexpr int ES = PAIR ? 4 : 2, KT = 128 / ES;
+    constexpr int RPT = NT / 8;                   // tile rows a pass of loads covers
+    constexpr int LA = BM / RPT, LW = BN / RPT, NL = LA + LW;
+    static_assert(LA * RPT == BM && LW * RPT == BN && RPT % 32 == 0, "every wave issues the same loads");
+    constexpr int STAGE = (BM + BN) * 128;        // bytes
+    constexpr int D = NST - 1;                    // k-tiles in flight ahead
+    constexpr bool HAS_BIAS = EPI != EPI_NONE;
+    constexpr int CES = OUT == OUT_BF16 ? 2 : 4;
+    constexpr int NSTO = FM * (FN / 2) * (OUT == OUT_BF16 ? 1 : 2);   // stores per lane and tile
+    constexpr int BIAS_BYTES = 1024;              // one wave's 64 x 16-byte bias chunks
+    __shared__ __attribute__((aligned(16))) char smem[NST * STAGE + (HAS_BIAS ? 2 * NW * BIAS_BYTES : 0)];
+
+    const int M = p.M_dev ? *p.M_dev : p.M_max;
+    const int N = p.N;
+    const int ntn = (N + BN - 1) / BN, ntiles = ((M + BM - 1) / BM) * ntn;
+    const int S = p.splits > 1 ? p.splits : 1;
+    const int nwork = ntiles * S, nk = p.K / KT / S;   // nk is even
+    // Workgroup b runs on XCD b % 8; each XCD's workgroups take consecutive
+    // tiles, which share A row panels in that XCD's L2.  Whole rounds: 32
+    // consecutive tiles per XCD and round; otherwise an eighth of the items
+    // per XCD, so that the last, partial round spreads over all of them.
+    const int G = gridDim.x;
+    int u0 = blockIdx.x, ustep = G, uend = nwork;
+    if ((G & 7) == 0 && nwork % G == 0) {
+        u0 = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
+    } else if ((G & 7) == 0) {
+        const int x = blockIdx.x & 7;
+        ustep = G >> 3;
+        u0 = (int)((int64_t)x * nwork / 8) + (blockIdx.x >> 3);
+        uend = (int)((int64_t)(x + 1) * nwork / 8);
+    }
+    const int my_tiles = u0 < uend ? (uend - u0 + ustep - 1) / ustep : 0;
+    const int total = my_tiles * nk;
+    if (total == 0) return;  // uniform over the workgroup
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+
+    // Lane share of a k-tile's loads: tile row r0 + i * RPT, LDS chunk tid % 8.
+    const int r0 = tid >> 3;
+    const uint32_t chunk = 16 * ((tid & 7) ^ chunk_swizzle16<8>(r0));
+    const int rw = (r0 & ~31) + 8 * ((r0 >> 2) & 3) + 4 * ((r0 >> 4) & 1) + (r0 & 3);
+    const uint32_t lda_b = (uint32_t)p.lda * ES, ldw_b = (uint32_t)p.ldw * ES;
+    const uint32_t avoff = r0 * lda_b + chunk, wvoff = rw * ldw_b + chunk;
+
+    // Load cursor: the next k-tile to load, its panels' descriptors and k offset.
+    g16_v4i arsrc, wrsrc;
+    uint32_t koff = 0;
+    const float* bias_src = nullptr;
+    int nit = 0, nkt = 0, nt_ = 0;                 // k-tile count, k-tile within the tile, tile
+    auto point_at = [&](int t) __attribute__((always_inline)) {
+        const int u = u0 + t * ustep, split = u / ntiles, tile = u - split * ntiles;
+        const int mt = tile / ntn, m0 = mt * BM, n0 = (tile - mt * ntn) * BN;
+        arsrc = make_rsrc(static_cast<const char*>(p.A) + (int64_t)m0 * p.lda * ES, (uint32_t)min(M - m0, BM) * lda_b);
+        wrsrc = make_rsrc(static_cast<const char*>(p.W) + (int64_t)n0 * p.ldw * ES, (uint32_t)min(N - n0, BN) * ldw_b);
+        koff = (uint32_t)(split * nk) * 128;
+        if (HAS_BIAS) bias_src = p.bias + min(n0 + wn * WN + 4 * lane, N - 4);
+    };
+    int vm = 0;                                    // vector memory instructions issued by this wave
+    int mark[D];                                   // vm after the loads of the next D k-tiles to enter
+#pragma unroll
+    for (int d = 0; d < D; ++d) mark[d] = 0;
+    constexpr int NPART = NS < 2 ? 1 : 2, PER = (NL + NPART - 1) / NPART;
+    auto issue_part = [&](int part) __attribute__((always_inline)) {
+        const uint32_t st = lds0 + (uint32_t)(nit % NST) * STAGE + (uint32_t)wave * 1024;
+#pragma unroll
+        for (int i = 0; i < NL; ++i)
+            if (i / PER == part) {
+                if (i < LA) load_lds16_buf(arsrc, avoff + i * RPT * lda_b, koff, st + i * RPT * 128);
+                else load_lds16_buf(wrsrc, wvoff + (i - LA) * RPT * ldw_b, koff, st + BM * 128 + (i - LA) * RPT * 128);
+                ++vm;
+            }
+        if (part == NPART - 1) {
+            if (HAS_BIAS && nkt == 0) {
+                load_lds16_async(bias_src, reinterpret_cast<const float*>(smem + NST * STAGE + ((nt_ & 1) * NW + wave) * BIAS_BYTES));
+                ++vm;
+            }
+            mark[D - 1] = vm;
+            ++nit;
+            koff += 128;
+            if (++nkt == nk) {
+                nkt = 0;
+                if (++nt_ < my_tiles) point_at(nt_);
+            }
+        }
+    };
+
+    const int r16 = lane & 15, q16 = lane >> 4;
+    const uint32_t frag = r16 * 128 + 16 * ((2 * q16) ^ chunk_swizzle16<8>(r16));
+    const uint32_t a_at = wm * WM * 128 + frag, w_at = BM * 128 + wn * WN * 128 + frag;
+    g16_v4f acc[FM][FN];
+    g16_v4f af[2][SB][2], wf[2][FN][2];
+
+    int it = 0;
+    auto enter = [&]() __attribute__((always_inline)) {
+        const int n = vm - mark[0];
+        constexpr auto c = [](int v) { return v > 63 ? 63 : v; };
+        if constexpr (D == 1) wait_vmcnt_of<c(NSTO)>(n);
+        else wait_vmcnt_of<c(NSTO + (D - 1) * NL + 1), c(NSTO + (D - 1) * NL), (D - 1) * NL + 1, (D - 1) * NL>(n);
+#pragma unroll
+        for (int d = 0; d + 1 < D; ++d) mark[d] = mark[d + 1];
+        lds_barrier();
+    };
+    auto mfma_step = [&](int s, int as, int ws) __attribute__((always_inline)) {
+        // smallest products first; consecutive MFMAs on different accumulators
+#pragma unroll
+        for (int pr = PAIR ? 0 : 1; pr < 3; ++pr)
+#pragma unroll
+            for (int i = 0; i < SB; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j) {
+                    g16_v4f& d = acc[s * SB + i][j];
+                    if constexpr (PAIR) {
+                        const g16_v4f& w = wf[ws][j][pr == 1 ? 1 : 0];
+                        const g16_v4f& a = af[as][i][pr == 0 ? 1 : 0];
+                        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, w), __builtin_bit_cast(v8h, a), d, 0, 0, 0);
+                    } else {
+                        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(g16_v8bf, wf[ws][j][pr - 1]),
+                                                                    __builtin_bit_cast(g16_v8bf, af[as][i][pr - 1]), d, 0, 0, 0);
+                    }
+                }
+    };
+    auto run_ktile = [&](auto pset, bool first) __attribute__((always_inline)) {
+        constexpr int P = decltype(pset)::value;
+        const bool refill = nit < total;
+        const char* st = smem + (it % NST) * STAGE;
+        auto rd_a = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < SB; ++i) {
+                const char* at = st + a_at + (s * SB + i) * 16 * 128;
+                af[s & 1][i][0] = *reinterpret_cast<const g16_v4f*>(at);
+                af[s & 1][i][1] = *reinterpret_cast<const g16_v4f*>(st + ((a_at ^ 16) + (s * SB + i) * 16 * 128));
+            }
+        };
+        rd_a(0);
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            wf[P][j][0] = *reinterpret_cast<const g16_v4f*>(st + w_at + j * 16 * 128);
+            wf[P][j][1] = *reinterpret_cast<const g16_v4f*>(st + (w_at ^ 16) + j * 16 * 128);
+        }
+        if (!first) mfma_step(NS - 1, 1, P ^ 1);   // the previous k-tile's last step
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            if (refill && s < NPART) issue_part(s);
+            if (s + 1 < NS) rd_a(s + 1);
+            if (s + 1 < NS) mfma_step(s, s & 1, P);
+        }
+        ++it;
+    };
+
+    auto epilogue = [&](int t) __attribute__((always_inline)) {
+        const int u = u0 + t * ustep, split = u / ntiles, tile = u - split * ntiles;
+        const int mt = tile / ntn, wrow = mt * BM + wm * WM, n0 = (tile - mt * ntn) * BN;
+        char* const cb = static_cast<char*>(p.C) + (int64_t)split * p.split_stride * CES;
+        const int64_t rowb = p.ldc * CES;
+        // lane-derived values opaque here: formed at the epilogue, not held across the k-loop
+        int el = lane;
+        asm volatile("" : "+v"(el));
+        const int er = el & 15, eq = el >> 4;
+        const char* bs = smem + NST * STAGE + ((t & 1) * NW + wave) * BIAS_BYTES + 32 * eq;
+        const float sc = p.acc_scale, so = p.out_scale;
+#pragma unroll
+        for (int jp = 0; jp < FN / 2; ++jp) {
+            g16_v4f b0 = {0, 0, 0, 0}, b1 = {0, 0, 0, 0};
+            if (HAS_BIAS) {
+                b0 = *reinterpret_cast<const g16_v4f*>(bs + jp * 128);
+                b1 = *reinterpret_cast<const g16_v4f*>(bs + jp * 128 + 16);
+            }
+            const int col = n0 + wn * WN + 32 * jp + 8 * eq;
+            const uint32_t voff = col < N ? (uint32_t)(er * (int)rowb + col * CES) : 0xFFFFFFE0u;   // N % 8 == 0
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+                float v[8];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (PAIR) {
+                        v[e] = HAS_BIAS ? fmaf(acc[i][2 * jp][e], sc, b0[e]) : acc[i][2 * jp][e] * sc;
+                        v[4 + e] = HAS_BIAS ? fmaf(acc[i][2 * jp + 1][e], sc, b1[e]) : acc[i][2 * jp + 1][e] * sc;
+                    } else {
+                        v[e] = acc[i][2 * jp][e] + b0[e];
+                        v[4 + e] = acc[i][2 * jp + 1][e] + b1[e];
+                    }
+                    if constexpr (EPI == EPI_BIAS_GELU) {
+                        v[e] = gelu_tanh_fast(v[e]);
+                        v[4 + e] = gelu_tanh_fast(v[4 + e]);
+                    }
+                }
+                const int left = __builtin_amdgcn_readfirstlane(M - wrow - 16 * i);
+                const int bytes = (left >= 16 ? 16 : (left > 0 ? left : 0)) * (int)rowb;
+                const __amdgpu_buffer_rsrc_t cr = __builtin_amdgcn_make_buffer_rsrc(
+                    cb + (int64_t)__builtin_amdgcn_readfirstlane(wrow + 16 * i) * rowb, (short)0, bytes, G16_RSRC_WORD3);
+                if constexpr (OUT == OUT_F32) {
+                    __builtin_amdgcn_raw_buffer_store_b128(
+                        u4v_t{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])}, cr, voff, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b128(
+                        u4v_t{__float_as_uint(v[4]), __float_as_uint(v[5]), __float_as_uint(v[6]), __float_as_uint(v[7])}, cr, voff + 16, 0, 0);
+                } else if constexpr (OUT == OUT_PAIR) {
+                    u4v_t h, l;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        uint32_t hw, lw;
+                        split_f16x2(v[2 * e] * so, v[2 * e + 1] * so, hw, lw);
+                        h[e] = hw;
+                        l[e] = lw;
+                    }
+                    __builtin_amdgcn_raw_buffer_store_b128(h, cr, voff, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b128(l, cr, voff + 16, 0, 0);
+                } else {
+                    __builtin_amdgcn_raw_buffer_store_b128(
+                        u4v_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])},
+                        cr, voff, 0, 2 /* nt */);
+                }
+            }
+        }
+        vm += NSTO;
+    };
+
+    point_at(0);
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        if (nit < total) {
+#pragma unroll
+            for (int part = 0; part < NPART; ++part) issue_part(part);
+        }
+        // mark[D - 1] was just set; the d-th k-tile's mark belongs at mark[d]
+        if constexpr (D > 1) mark[d] = vm;
+    }
+    typedef std::integral_constant<int, 0> set0;
+    typedef std::integral_constant<int, 1> set1;
+    for (int t = 0; t < my_tiles; ++t) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = g16_v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        enter();
+        run_ktile(set0{}, true);
+        enter();
+        run_ktile(set1{}, false);
+        for (int kt = 2; kt < nk; kt += 2) {
+            enter();
+            run_ktile(set0{}, false);
+            enter();
+            run_ktile(set1{}, false);
+        }
+        mfma_step(NS - 1, 1, 1);
+        epilogue(t);
+    }
+}
+
+}  // namespace ebh

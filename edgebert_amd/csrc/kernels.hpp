@@ -45,6 +45,42 @@ struct GemmArgs {
 // below 2^32; launch_gemm_f32 sends larger strides to the guarded kernel
 // (64-bit addresses), the other persistent launchers reject them.
 constexpr int GEMM_TILE_ROWS_MAX = 384;
+// Arguments of the 16-bit matrix-core products (gemm16.hpp): fp32 values as
+// fp16 pairs, or bf16.
+struct Gemm16Args {
+    const void* A;       // [M, K], rows of pairs (4 bytes an element) or bf16
+    const void* W;       // [N, K]
+    const float* bias;   // [N]
+    void* C;             // [M, N] fp32, pairs or bf16
+    int64_t lda, ldw, ldc;   // elements
+    int M_max;           // grid is sized for this many rows
+    const int* M_dev;    // actual rows, read on device (nullptr: M_max)
+    int N, K;
+    int splits;          // split-K, as in GemmArgs
+    int64_t split_stride;
+    float acc_scale;     // pairs: 1 / (scale of A * scale of W)
+    float out_scale;     // scale of a pair output
+};
+
+// Tile and split count the 16-bit products take for a shape: gelu is the FFN
+// up epilogue's cost; split counts from min_splits to max_splits are weighed
+// (above 1 for EPI_NONE only).  M: the row count as far as the host knows it.
+struct Gemm16Plan {
+    int tile, splits;
+};
+Gemm16Plan gemm16_pair_plan(int M, int N, int K, bool gelu, int min_splits, int max_splits);
+constexpr int GEMM16_TILES = 7;
+// N % 8 == 0, K % (64 * splits) == 0, strides multiples of 8 elements and at
+// most gemm_stride_max(4), 16-byte aligned operands (hipErrorInvalidValue
+// otherwise).  out_pair: C as pairs of scale out_scale instead of fp32, with
+// EPI_BIAS_GELU; fp32 with EPI_BIAS and EPI_NONE.
+hipError_t launch_gemm16_pair(const Gemm16Args& a, int epi, bool out_pair, int tile, hipStream_t s);
+// y = the pairs of scale * x, n a multiple of 8.
+hipError_t launch_to_pair(const float* x, uint32_t* y, int64_t n, float scale, hipStream_t s);
+// norm2[n], amax[n]: each row's sum of squares and largest magnitude (NaN if
+// the row has one), W [N, K].
+hipError_t launch_row_stats(const float* W, int N, int K, float* norm2, float* amax, hipStream_t s);
+
 // Largest row stride (elements of es bytes) the persistent kernels take:
 // GEMM_TILE_ROWS_MAX * stride * es + (one k-tile of at most 64 elements) * es
 // stays below 2^32.
@@ -76,10 +112,12 @@ hipError_t launch_gemm_bf16(const GemmArgs& a, int epi, hipStream_t s);
 // Masked multi-head attention over packed sequences: qkv [T, 3H] rows
 // (q | k | v), cu_seqlens [B+1]; ctx [T, H].  head_dim 32 or 64.  order
 // (nullable): a permutation of the B sequences, the order in which the grid
-// takes them (launch_pack writes one by decreasing length).
+// takes them (launch_pack writes one by decreasing length).  pair_scale > 0:
+// the context is written as fp16 pairs of that scale (gemm16.hpp)
+// instead of fp32 (the same 4 H bytes a row).
 hipError_t launch_attention(const float* qkv, const int* cu_seqlens, int B, int max_len,
                             int H, int nh, int head_dim, float scale, float* ctx, hipStream_t s,
-                            const int* order = nullptr);
+                            const int* order = nullptr, float pair_scale = 0.0f);
 
 // Attention with bf16 q / k / v (qkv [T, 3H] bf16 bits) and bf16 context;
 // scores, softmax and accumulation in fp32.  head_dim 32 or 64.
@@ -108,10 +146,11 @@ hipError_t launch_layernorm(const float* x, float* y, const float* g, const floa
 // nparts split-K partial products part_stride floats apart; they are summed in
 // order (((p0 + p1) + p2) + ...) before the bias.
 // x16 (optional): bf16 copy of the result (the input of bf16 GEMMs).
+// xp (optional, float4 row shapes only): the result as fp16 pairs of scale xs.
 hipError_t launch_add_layernorm(const float* y, const float* bias, float* x, const float* g,
                                 const float* b, int rows_max, const int* rows_dev, int H, float eps,
                                 uint16_t* x16, hipStream_t s, int nparts = 1,
-                                int64_t part_stride = 0);
+                                int64_t part_stride = 0, uint32_t* xp = nullptr, float xs = 0.0f);
 // The same with y stored as bf16 (bf16 models).  x == nullptr: the residual
 // stream is bf16 instead, x16 = bf16(LayerNorm((y + bias) + x16)) in place
 // (sums and statistics fp32).  Needs 8-byte aligned bf16 rows, 16-byte aligned
@@ -153,11 +192,13 @@ hipError_t launch_attn_out_few(const float* qkv, const float* wo, const int* cu,
                               hipStream_t s);
 
 // Embedding gather + position + token type 0 + LayerNorm over packed tokens,
-// into x (fp32) and / or x16 (bf16; either may be nullptr, not both).
+// into x (fp32) and / or x16 (bf16; either may be nullptr, not both); xp
+// (optional, float4 row shapes only): the result as fp16 pairs of scale xs.
 hipError_t launch_embed_ln(const int* tok_id, const int* tok_pos, const int* n_tokens,
                            int T_max, const float* word, const float* pos, const float* type0,
                            const float* g, const float* b, int V, int H, float eps, float* x,
-                           int* err, uint16_t* x16, hipStream_t s);
+                           int* err, uint16_t* x16, hipStream_t s, uint32_t* xp = nullptr,
+                           float xs = 0.0f);
 
 // Masked mean over each packed sequence, optional L2 normalisation; out [B, H].
 // Floats of `partials` the fp32 pool needs: B * ceil(S / 32) * H when it
@@ -373,6 +414,16 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
     const v2f_t v = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, v2bf_t));
+}
+
+// Two values already scaled, as (h, h) and (l, l) words of the pair format.
+__device__ __forceinline__ void split_f16x2(float a, float b, uint32_t& h, uint32_t& l) {
+    typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    const v2h hh = __builtin_convertvector((v2f{a, b}), v2h);
+    const v2h ll = __builtin_convertvector((v2f{a - (float)hh[0], b - (float)hh[1]}), v2h);
+    h = __builtin_bit_cast(uint32_t, hh);
+    l = __builtin_bit_cast(uint32_t, ll);
 }
 
 }  // namespace ebh

@@ -375,7 +375,8 @@ __device__ __forceinline__ float group_sum(float v) {
 
 template <int NV, int LPR>
 __device__ __forceinline__ void ln_row4(float4 (&v)[NV], int sub, int H, const float* g,
-                                        const float* b, float eps, float* y, uint16_t* y16) {
+                                        const float* b, float eps, float* y, uint16_t* y16,
+                                        uint32_t* yp = nullptr, float ps = 0.0f) {
     // gamma / beta are loaded first, so their memory round trip overlaps the
     // row reductions instead of following them.
     float4 g4[NV], b4[NV];
@@ -411,6 +412,14 @@ __device__ __forceinline__ void ln_row4(float4 (&v)[NV], int sub, int H, const f
             h.y = (uint32_t)f32_to_bf16_rne(o.z) | ((uint32_t)f32_to_bf16_rne(o.w) << 16);
             *reinterpret_cast<uint2*>(y16 + i) = h;
         }
+        if (yp) {   // fp16 pairs of ps * o: four h and four l of the element's 32-byte group
+            uint2 h, l;
+            split_f16x2(o.x * ps, o.y * ps, h.x, l.x);
+            split_f16x2(o.z * ps, o.w * ps, h.y, l.y);
+            uint32_t* const at = yp + (i & ~7) + ((i & 4) >> 1);
+            *reinterpret_cast<uint2*>(at) = h;
+            *reinterpret_cast<uint2*>(at + 4) = l;
+        }
     }
 }
 
@@ -424,7 +433,8 @@ __device__ __forceinline__ void add_layernorm4_row(const float* __restrict__ y, 
                                                    float* x, const float* __restrict__ g,
                                                    const float* __restrict__ bta, int rows_max,
                                                    const int* rows_dev, int H, float eps, uint16_t* x16,
-                                                   int nparts, int64_t part_stride) {
+                                                   int nparts, int64_t part_stride, uint32_t* xp = nullptr,
+                                                   float xs = 0.0f) {
     constexpr int RPB = BS / LPR;                 // rows per workgroup
     const int row = blockIdx.x * RPB + threadIdx.x / LPR, sub = threadIdx.x % LPR;
     const int rows = rows_dev ? *rows_dev : rows_max;
@@ -463,7 +473,8 @@ __device__ __forceinline__ void add_layernorm4_row(const float* __restrict__ y, 
     for (int c = 0; c < NV; ++c)
         v[c] = make_float4((a[c].x + bb[c].x) + r[c].x, (a[c].y + bb[c].y) + r[c].y,
                            (a[c].z + bb[c].z) + r[c].z, (a[c].w + bb[c].w) + r[c].w);
-    ln_row4<NV, LPR>(v, sub, H, g, bta, eps, xr, x16 ? x16 + (int64_t)row * H : nullptr);
+    ln_row4<NV, LPR>(v, sub, H, g, bta, eps, xr, x16 ? x16 + (int64_t)row * H : nullptr,
+                     xp ? xp + (int64_t)row * H : nullptr, xs);
 }
 
 #define EBH_ADD_LN4_KERNEL(NAME, PB)                                                                    \
@@ -472,9 +483,9 @@ __device__ __forceinline__ void add_layernorm4_row(const float* __restrict__ y, 
                                                 float* x, const float* __restrict__ g,                  \
                                                 const float* __restrict__ bta, int rows_max,            \
                                                 const int* rows_dev, int H, float eps, uint16_t* x16,   \
-                                                int nparts, int64_t part_stride) {                      \
+                                                int nparts, int64_t part_stride, uint32_t* xp, float xs) { \
         add_layernorm4_row<NV, LPR, PB>(y, bias, x, g, bta, rows_max, rows_dev, H, eps, x16, nparts,    \
-                                        part_stride);                                                   \
+                                        part_stride, xp, xs);                                           \
     }
 EBH_ADD_LN4_KERNEL(add_layernorm4_kernel, 0)       // one product
 EBH_ADD_LN4_KERNEL(add_layernorm4_p4_kernel, 4)    // split-K partials
@@ -551,7 +562,7 @@ __global__ __launch_bounds__(256) void embed_ln4_kernel(
     const int* __restrict__ n_tokens, const float* __restrict__ word,
     const float* __restrict__ pos, const float* __restrict__ type0, const float* __restrict__ g,
     const float* __restrict__ bta, int V, int H, float eps, float* __restrict__ x,
-    int* __restrict__ err, uint16_t* __restrict__ x16) {
+    int* __restrict__ err, uint16_t* __restrict__ x16, uint32_t* __restrict__ xp, float xs) {
     constexpr int RPB = 256 / LPR;
     const int t = blockIdx.x * RPB + threadIdx.x / LPR, sub = threadIdx.x % LPR;
     if (t >= *n_tokens) return;
@@ -572,7 +583,7 @@ __global__ __launch_bounds__(256) void embed_ln4_kernel(
         v[c] = make_float4((a.x + p4.x) + ty.x, (a.y + p4.y) + ty.y, (a.z + p4.z) + ty.z, (a.w + p4.w) + ty.w);
     }
     ln_row4<NV, LPR>(v, sub, H, g, bta, eps, x ? x + (int64_t)t * H : nullptr,
-                     x16 ? x16 + (int64_t)t * H : nullptr);
+                     x16 ? x16 + (int64_t)t * H : nullptr, xp ? xp + (int64_t)t * H : nullptr, xs);
 }
 
 // The bf16-residual block end of bf16 models with 16-byte lane accesses:
@@ -743,7 +754,8 @@ hipError_t launch_layernorm(const float* x, float* y, const float* g, const floa
 
 hipError_t launch_add_layernorm(const float* y, const float* bias, float* x, const float* g,
                                 const float* b, int rows_max, const int* rows_dev, int H, float eps,
-                                uint16_t* x16, hipStream_t s, int nparts, int64_t part_stride) {
+                                uint16_t* x16, hipStream_t s, int nparts, int64_t part_stride, uint32_t* xp,
+                                float xs) {
     if (rows_max <= 0) return hipSuccess;
     if (nparts < 1) nparts = 1;
     int lpr, nv;
@@ -751,7 +763,7 @@ hipError_t launch_add_layernorm(const float* y, const float* bias, float* x, con
     if (lpr && al16(y) && al16(bias) && al16(x) && al16(g) && al16(b) && (!x16 || ((uintptr_t)x16 & 7) == 0) &&
         part_stride % 4 == 0) {
         // Partials are read PB at a time, each group one memory round trip.
-        if (nparts > 8 && rows_max <= 64) {
+        if (nparts > 8 && rows_max <= 64 && !xp) {
 #define EBH_LN_ROW1(L)                                                                                  \
             if (lpr == L) {                                                                         \
                 switch (nv) {                                                                       \
@@ -770,12 +782,13 @@ hipError_t launch_add_layernorm(const float* y, const float* bias, float* x, con
         }
         if (nparts > 1)
             EBH_ROW4_DISPATCH(add_layernorm4_p4_kernel, lpr, nv, rows_max, s, y, bias, x, g, b, rows_max,
-                              rows_dev, H, eps, x16, nparts, part_stride);
+                              rows_dev, H, eps, x16, nparts, part_stride, xp, xs);
         else
             EBH_ROW4_DISPATCH(add_layernorm4_kernel, lpr, nv, rows_max, s, y, bias, x, g, b, rows_max,
-                              rows_dev, H, eps, x16, nparts, part_stride);
+                              rows_dev, H, eps, x16, nparts, part_stride, xp, xs);
         return hipGetLastError();
     }
+    if (xp) return hipErrorInvalidValue;
     const dim3 grid((rows_max + 3) / 4);
     EBH_ROW_DISPATCH(add_layernorm_kernel, H, grid, s, y, bias, x, g, b, rows_max, rows_dev, H, eps, x16,
                      nparts, part_stride);
@@ -820,7 +833,7 @@ hipError_t launch_add_layernorm_y16(const uint16_t* y, const float* bias, float*
 hipError_t launch_embed_ln(const int* tok_id, const int* tok_pos, const int* n_tokens,
                            int T_max, const float* word, const float* pos, const float* type0,
                            const float* g, const float* b, int V, int H, float eps, float* x,
-                           int* err, uint16_t* x16, hipStream_t s) {
+                           int* err, uint16_t* x16, hipStream_t s, uint32_t* xp, float xs) {
     if (T_max <= 0) return hipSuccess;
     int lpr, nv;
     row4_shape(H, lpr, nv);
@@ -828,9 +841,10 @@ hipError_t launch_embed_ln(const int* tok_id, const int* tok_pos, const int* n_t
     if (lpr && al16(word) && al16(pos) && al16(type0) && al16(g) && al16(b) && (!x || al16(x)) &&
         (!x16 || ((uintptr_t)x16 & 7) == 0)) {
         EBH_ROW4_DISPATCH(embed_ln4_kernel, lpr, nv, T_max, s, tok_id, tok_pos, n_tokens, word, pos,
-                          type0, g, b, V, H, eps, x, err, x16);
+                          type0, g, b, V, H, eps, x, err, x16, xp, xs);
         return hipGetLastError();
     }
+    if (xp) return hipErrorInvalidValue;
     const dim3 grid((T_max + 3) / 4);
     EBH_ROW_DISPATCH(embed_ln_kernel, H, grid, s, tok_id, tok_pos, n_tokens, word, pos, type0, g,
                      b, V, H, eps, x, err, x16);

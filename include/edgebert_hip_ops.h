@@ -52,6 +52,26 @@ EBH_API int ebh_op_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, 
                      const float* bias, void* C, int64_t ldc, int32_t c_dtype, int32_t M, int32_t N,
                      int32_t K, int32_t epilogue, void* stream);
 
+/* fp32 products from fp16 pairs, as the fp32 forward runs them above 64 tokens
+ * (src/lib.rs:691-698, 732-733, 741-747, 795-849, 958-978): A [M, K] and W
+ * [N, K] in the pair format of ebh_op_to_pair with scales sA and sW, acc_scale
+ * = 1 / (sA * sW).  c_scale 0: C [M, N] fp32, epilogue EBH_EPI_BIAS or
+ * EBH_EPI_NONE; c_scale > 0: C as pairs of that scale, EBH_EPI_BIAS_GELU.
+ * splits > 1 (EBH_EPI_NONE): split s sums k in [s K / splits, (s + 1) K /
+ * splits) into C + s * split_stride.  tile: -1, or one of 0 .. 6 (256x256,
+ * 256x192, 128x128, 128x96, 64x128, 128x64, 64x64); the result does not depend
+ * on it.  N % 8 == 0, K % (64 splits) == 0, strides (elements) multiples of 8
+ * and at most 2,796,202, 16-byte aligned operands (EBH_ERR_INVALID_ARG
+ * otherwise). */
+EBH_API int ebh_op_gemm_pair(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t ldw, float acc_scale,
+                     const float* bias, void* C, int64_t ldc, float c_scale, int32_t M, int32_t N, int32_t K,
+                     int32_t epilogue, int32_t splits, int64_t split_stride, int32_t tile, void* stream);
+
+/* The pair format: y holds, for each 8 consecutive values of scale * x, eight
+ * fp16 h = fp16(v) and eight fp16 l = fp16(v - h), round to nearest even (32
+ * bytes); scale a power of two, n a multiple of 8, x and y 16-byte aligned. */
+EBH_API int ebh_op_to_pair(const float* x, uint32_t* y, int64_t n, float scale, void* stream);
+
 /* Masked multi-head attention (src/lib.rs:700-730 with 851-956) over packed
  * sequences: qkv [T, 3*hidden] rows (q | k | v), sequence b = rows
  * cu_seqlens[b] .. cu_seqlens[b+1]-1 (every row a real token, lengths <=

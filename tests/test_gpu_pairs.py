@@ -1,0 +1,165 @@
+"""fp32 products from fp16 pairs (ebh_op_to_pair, ebh_op_gemm_pair) against float64
+on every tile, at tile edges and remainders; and models whose weights lie at
+the ends of the range the pair operands' scales are taken from, or outside it
+(those keep the fp32 kernels), against the CPU oracle."""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+EPI_BIAS, EPI_GELU, EPI_NONE = 0, 1, 3
+
+
+@pytest.fixture(scope="module")
+def env():
+    import torch
+    import edgebert_amd as eb
+    from edgebert_amd import _native as N
+    assert torch.cuda.is_available(), "gpu tests need a GPU"
+    return torch, eb, N, eb.lib()
+
+
+def vp(t):
+    return ctypes.c_void_p(t.data_ptr())
+
+
+def to_pair(torch, N, L, x, scale, s):
+    y = torch.empty_like(x)
+    N.check(L.ebh_op_to_pair(vp(x), vp(y), x.numel(), scale, s))
+    return y
+
+
+def unpair(torch, y, scale):
+    h = y.view(torch.float16).view(y.shape[0], -1, 2, 8).double()
+    return ((h[:, :, 0] + h[:, :, 1]) / scale).reshape(y.shape[0], -1)
+
+
+def test_to_pair_keeps_23_bits(env):
+    torch, eb, N, L = env
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    x = torch.randn(64, 264, device="cuda")
+    scale = 2.0 ** 12
+    got = unpair(torch, to_pair(torch, N, L, x, scale, s), scale)
+    # l is rounded to 11 bits of at most half a unit of h's 11: 2^-23 of |x|,
+    # or half of fp16's smallest step where l is subnormal
+    bound = np.maximum(2.0 ** -23 * x.abs().double().cpu().numpy(), 2.0 ** -25 / scale)
+    assert (np.abs((got - x.double()).cpu().numpy()) <= bound).all()
+    assert L.ebh_op_to_pair(vp(x), vp(x), 12, scale, s) == N.EBH_ERR_INVALID_ARG
+
+
+# rows below, at and just over every tile height; columns that are not whole
+# tiles; one, two and several k-tile pairs; splits
+SHAPES = [(1, 64, 64, 1), (63, 96, 128, 2), (65, 200, 192, 3), (129, 392, 384, 1), (257, 1152, 384, 2),
+          (300, 1536, 384, 1), (513, 384, 1536, 4), (1000, 264, 448, 1)]
+
+
+@pytest.mark.parametrize("tile", range(-1, 7))
+@pytest.mark.parametrize("M,Nn,K,S", SHAPES)
+def test_gemm_pair(env, M, Nn, K, S, tile):
+    torch, eb, N, L = env
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator(device="cuda").manual_seed(M + Nn + K)
+    lda, ldc = K + 8, Nn + 16
+    A = torch.randn(M, lda, device="cuda", generator=g)
+    A[:, 3] *= 30                                  # an outlier feature
+    W = 0.04 * torch.randn(Nn, K, device="cuda", generator=g)
+    b = torch.randn(Nn, device="cuda", generator=g)
+    sa, sw, sc = 2.0 ** 8, 2.0 ** 14, 2.0 ** 4
+    Ap, Wp = to_pair(torch, N, L, A, sa, s), to_pair(torch, N, L, W, sw, s)
+    Ad, Wd = A[:, :K].double(), W.double()
+    ref = Ad @ Wd.t()
+    # operands 2^-23 each, al.bl 2^-24, and 3 K / 32 sums each rounded (down)
+    # a few times within 2^-22 of the terms' size
+    tol = (2.0 ** -21 + 3 * K / 32 * 2.0 ** -22) * (Ad.abs() @ Wd.abs().t())
+
+    def run(epi, C, c_scale, bias, splits=1, stride=0):
+        N.check(L.ebh_op_gemm_pair(vp(Ap), lda, vp(Wp), K, 1 / (sa * sw), bias, vp(C), ldc, c_scale, M, Nn, K, epi,
+                                   splits, stride, tile, s))
+        torch.cuda.synchronize()
+
+    C = torch.full((M + 2, ldc), 7.0, device="cuda")
+    run(EPI_BIAS, C, 0.0, vp(b))
+    assert ((C[:M, :Nn].double() - ref - b.double()).abs() <= tol + 2.0 ** -23 * (ref.abs() + b.abs().double())).all()
+    assert (C[M:] == 7).all() and (C[:, Nn:] == 7).all()
+    first = C[:M, :Nn].clone()
+    if tile > 0:      # every tile sums in the same order
+        C0 = torch.empty_like(C)
+        N.check(L.ebh_op_gemm_pair(vp(Ap), lda, vp(Wp), K, 1 / (sa * sw), vp(b), vp(C0), ldc, 0.0, M, Nn, K, EPI_BIAS,
+                                   1, 0, 0, s))
+        torch.cuda.synchronize()
+        assert torch.equal(C0[:M, :Nn], first)
+    stride = (M + 1) * ldc
+    P = torch.full((S * stride,), 7.0, device="cuda")
+    if K % (64 * S) == 0:
+        run(EPI_NONE, P, 0.0, None, S, stride)
+        got = sum(P[i * stride:i * stride + M * ldc].view(M, ldc)[:, :Nn].double() for i in range(S))
+        assert ((got - ref).abs() <= tol + 2.0 ** -23 * ref.abs() * S).all()
+    D = torch.full((M + 2, ldc), 7.0, device="cuda")
+    run(EPI_GELU, D, sc, vp(b))
+    u = ref + b.double()
+    want = 0.5 * u * (1 + torch.tanh(0.7978845608028654 * (u + 0.044715 * u ** 3)))
+    got = unpair(torch, D[:M], sc)[:, :Nn]
+    # GELU's slope is below 1.13; its own error (8 ln2 |t| + 8) 2^-24 |gelu|
+    gtol = 1.13 * (tol + 2.0 ** -23 * u.abs()) + (2.0 ** -22 + 2.0 ** -20) * want.abs() + 2.0 ** -25 / sc
+    assert ((got - want).abs() <= gtol + 1e-6 * (u < -4)).all()
+    assert (D[M:] == 7).all() and (D[:, Nn:] == 7).all()
+
+
+def test_gemm_pair_refuses(env):
+    torch, eb, N, L = env
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    t = torch.zeros(1 << 16, device="cuda")
+
+    def call(M=8, Nn=64, K=64, epi=EPI_NONE, c_scale=0.0, splits=1, tile=-1, ldc=64, bias=None, A=None):
+        return L.ebh_op_gemm_pair(A or vp(t), K, vp(t), K, 1.0, bias, vp(t), ldc, c_scale, M, Nn, K, epi, splits, 64 * 8,
+                                  tile, s)
+
+    bad = N.EBH_ERR_INVALID_ARG
+    assert call(K=96) == bad and call(Nn=60) == bad and call(ldc=60) == bad and call(tile=7) == bad
+    assert call(epi=EPI_GELU) == bad and call(c_scale=2.0) == bad and call(splits=2) == bad
+    assert call(epi=EPI_BIAS) == bad                       # no bias
+    assert call(A=ctypes.c_void_p(t.data_ptr() + 4)) == bad
+    assert call(M=0) == N.EBH_OK and call() == N.EBH_OK
+    torch.cuda.synchronize()
+
+
+def _spread(w, how):
+    """Weights moved towards or past an end of the pair operands' range."""
+    w = {k: v.copy() for k, v in w.items()}
+    for k in w:
+        if how == "wide_gain" and k.endswith("LayerNorm.weight"):
+            w[k] *= 40.0
+        if how == "outlier_gain" and k == "embeddings.LayerNorm.weight":
+            w[k][5] = 5.0e3                                # one feature far above the rest: fp32 kernels
+        if how == "outlier_gain" and "layer.0.attention.self" in k and k.endswith("weight"):
+            w[k][:, 5] /= 5.0e3
+        if how == "zero_matrix" and k.endswith("attention.output.dense.weight"):
+            w[k][:] = 0.0                                  # no scale: fp32 kernels
+        if how == "tiny_row" and k.endswith("intermediate.dense.weight"):
+            w[k][3] *= 1e-7                                # a row far below the rest: fp32 kernels
+        if how == "small_weights" and k.endswith("dense.weight"):
+            w[k] *= 2.0 ** -20
+    return w
+
+
+@pytest.mark.parametrize("how", ["wide_gain", "outlier_gain", "zero_matrix", "tiny_row", "small_weights"])
+def test_models_at_the_ends_of_the_range(env, weights_for, how):
+    import oracle
+    torch, eb, N, L = env
+    cfg = eb.TINY
+    w = _spread(weights_for(cfg), how)
+    rng = np.random.default_rng(5)
+    B, S = 9, 31
+    ids = rng.integers(10, cfg.vocab_size, (B, S)).astype(np.uint32)
+    n = rng.integers(1, S + 1, B)
+    mask = (np.arange(S)[None, :] < n[:, None]).astype(np.uint32)
+    m = eb.Model.from_weights(w, cfg, "fp32")
+    try:
+        got = m.encode_ids(ids * mask, mask)
+    finally:
+        m.close()
+    want = oracle.OracleModel(cfg, w).encode_unpadded(ids * mask, mask, normalize=True)
+    assert np.isfinite(got).all()
+    assert np.abs(got - want).max() <= 1e-5

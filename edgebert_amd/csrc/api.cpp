@@ -83,11 +83,11 @@ struct DevLayer {
     uint32_t *wqkvp, *wop, *w1p, *w2p;
 };
 
-// Scales (powers of two) of a layer's pair operands: its input X, the context,
-// the FFN's input (the first LayerNorm's output), the GELU output, and the
-// four weight matrices.
+// Scales (powers of two) of a layer's pair operands: its input X, q / k / v,
+// the context, the FFN's input (the first LayerNorm's output), the GELU
+// output, and the four weight matrices.
 struct PairScales {
-    float x, ctx, mid, f, wqkv, wo, w1, w2;
+    float x, qkv, ctx, mid, f, wqkv, wo, w1, w2;
 };
 
 struct Workspace {
@@ -448,13 +448,14 @@ int enqueue_pair_layers(ebh_model* m, Workspace& w, int B, int S, int normalize,
         const DevLayer& L = m->layers[l];
         const PairScales& q = m->pair_scales[l];
         int rc;
-        if ((rc = gemm(EBH_PROF_GEMM_QKV, xp, L.wqkvp, L.bqkv, w.QKV, 3 * H, H, ebh::EPI_BIAS, false,
-                       1.0f / (q.x * q.wqkv), 0.0f, p_qkv)))
+        if ((rc = gemm(EBH_PROF_GEMM_QKV, xp, L.wqkvp, L.bqkv, w.QKV, 3 * H, H, ebh::EPI_BIAS, true,
+                       1.0f / (q.x * q.wqkv), q.qkv, p_qkv)))
             return rc;
         ProfPair pp{};
         bool on = false;
         prof_begin(m, prof_kind, EBH_PROF_ATTENTION, s, pp, on);
-        HIP_TRY(ebh::launch_attention(w.QKV, w.cu, B, S, H, nh, hd, scale, w.CTX, s, seq_order, q.ctx));
+        HIP_TRY(ebh::launch_attention_pair(reinterpret_cast<const uint32_t*>(w.QKV), w.cu, B, S, H, nh, hd, scale,
+                                           q.qkv, reinterpret_cast<uint32_t*>(w.CTX), q.ctx, s, seq_order));
         prof_end(m, s, pp, on);
         if ((rc = gemm(EBH_PROF_GEMM_OUT, w.CTX, L.wop, nullptr, w.Y, H, H, ebh::EPI_NONE, false,
                        1.0f / (q.ctx * q.wo), 0.0f, p_out)))
@@ -991,17 +992,18 @@ static int prepare_pairs(ebh_model* m) {
         HIP_TRY(ebh::launch_row_stats(d.w2, (int)H, (int)I, n2 + 4 * H + I, am + 4 * H + I, st));
     }
     HIP_TRY(hipMemcpyAsync(stats.data(), d_stats, stats.size() * 4, hipMemcpyDeviceToHost, st));
-    // emb g, b; per layer: bv, ln1 g, b, b1, ln2 g, b
-    const size_t per = 5 * H + I;
+    // emb g, b; per layer: ln1 g, b, ln2 g, b, bqkv, b1
+    const size_t per = 7 * H + I;
     std::vector<float> v(2 * H + L * per);
     HIP_TRY(hipMemcpyAsync(v.data(), m->emb_g, H * 4, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipMemcpyAsync(v.data() + H, m->emb_b, H * 4, hipMemcpyDeviceToHost, st));
     for (size_t l = 0; l < L; ++l) {
         const DevLayer& d = m->layers[l];
         float* p = v.data() + 2 * H + l * per;
-        const float* src[] = {d.bqkv + 2 * H, d.ln1_g, d.ln1_b, d.ln2_g, d.ln2_b};
-        for (int i = 0; i < 5; ++i) HIP_TRY(hipMemcpyAsync(p + i * H, src[i], H * 4, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipMemcpyAsync(p + 5 * H, d.b1, I * 4, hipMemcpyDeviceToHost, st));
+        const float* src[] = {d.ln1_g, d.ln1_b, d.ln2_g, d.ln2_b};
+        for (int i = 0; i < 4; ++i) HIP_TRY(hipMemcpyAsync(p + i * H, src[i], H * 4, hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipMemcpyAsync(p + 4 * H, d.bqkv, 3 * H * 4, hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipMemcpyAsync(p + 7 * H, d.b1, I * 4, hipMemcpyDeviceToHost, st));
     }
     HIP_TRY(hipStreamSynchronize(st));
 
@@ -1050,19 +1052,20 @@ static int prepare_pairs(ebh_model* m) {
     Norm in = norm_of(v.data(), v.data() + H);
     for (size_t l = 0; l < L; ++l) {
         const float *n2 = stats.data() + l * rows * 2, *am = n2 + rows, *p = v.data() + 2 * H + l * per;
-        const Norm mid = norm_of(p + H, p + 2 * H);
+        const Norm mid = norm_of(p, p + H);
         PairScales& q = sc[l];
         q.x = pair_scale(in.max, in.typ, kActLimit);
-        q.ctx = out_scale(n2 + 2 * H, p, H, in);
+        q.qkv = out_scale(n2, p + 4 * H, 3 * H, in);
+        q.ctx = out_scale(n2 + 2 * H, p + 6 * H, H, in);
         q.mid = pair_scale(mid.max, mid.typ, kActLimit);
-        q.f = out_scale(n2 + 4 * H, p + 5 * H, I, mid);
+        q.f = out_scale(n2 + 4 * H, p + 7 * H, I, mid);
         q.wqkv = weight_scale(n2, am, 3 * H);
         q.wo = weight_scale(n2 + 3 * H, am + 3 * H, H);
         q.w1 = weight_scale(n2 + 4 * H, am + 4 * H, I);
         q.w2 = weight_scale(n2 + 4 * H + I, am + 4 * H + I, H);
-        for (float f : {q.x, q.ctx, q.mid, q.f, q.wqkv, q.wo, q.w1, q.w2})
+        for (float f : {q.x, q.qkv, q.ctx, q.mid, q.f, q.wqkv, q.wo, q.w1, q.w2})
             if (!(f > 0.0f)) return EBH_OK;
-        in = norm_of(p + 3 * H, p + 4 * H);
+        in = norm_of(p + 2 * H, p + 3 * H);
     }
     const size_t words = 4 * H * H + 2 * H * I;          // pair weights of a layer
     if (hipMalloc(&m->wpair, L * words * 4) != hipSuccess) {   // no room: the fp32 kernels need none
@@ -1628,7 +1631,7 @@ int ebh_op_gemm_pair(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t 
                      int32_t epilogue, int32_t splits, int64_t split_stride, int32_t tile, void* stream) {
     if (!A || !W || !C || M < 0 || N <= 0 || K <= 0 || splits < 1 || tile < -1 || tile >= ebh::GEMM16_TILES ||
         !(acc_scale > 0.0f) || !(c_scale >= 0.0f) || epilogue < EBH_EPI_BIAS || epilogue > EBH_EPI_NONE ||
-        epilogue == EBH_EPI_BIAS_RESID || (epilogue == EBH_EPI_BIAS_GELU) != (c_scale > 0.0f) ||
+        epilogue == EBH_EPI_BIAS_RESID || (epilogue != EBH_EPI_NONE) != (c_scale > 0.0f) ||
         (splits > 1 && epilogue != EBH_EPI_NONE))
         return fail(EBH_ERR_INVALID_ARG, "bad pair gemm arguments");
     ebh::Gemm16Args a{};
@@ -1673,6 +1676,25 @@ int ebh_op_attention(const float* qkv, const int32_t* cu_seqlens, int32_t B, int
     const float scale = 1.0f / sqrtf((float)hd);
     HIP_TRY(ebh::launch_attention(qkv, cu_seqlens, B, max_len, hidden, num_heads, hd, scale, ctx,
                                   static_cast<hipStream_t>(stream)));
+    return EBH_OK;
+}
+
+int ebh_op_attention_pair(const uint32_t* qkv, float qkv_scale, const int32_t* cu_seqlens, int32_t B,
+                          int32_t max_len, int32_t hidden, int32_t num_heads, uint32_t* ctx, float ctx_scale,
+                          void* stream) {
+    if (!qkv || !cu_seqlens || !ctx || B < 0 || max_len < 0 || hidden <= 0 || num_heads <= 0 || hidden % num_heads ||
+        !(qkv_scale > 0.0f) || !(ctx_scale > 0.0f))
+        return fail(EBH_ERR_INVALID_ARG, "bad attention arguments");
+    const int hd = hidden / num_heads;
+    if (hd != 32 && hd != 64) return fail(EBH_ERR_INVALID_ARG, "head_dim %d is not 32 or 64", hd);
+    if ((uintptr_t)qkv & 15 || (uintptr_t)ctx & 7)
+        return fail(EBH_ERR_INVALID_ARG, "qkv must be 16-byte and ctx 8-byte aligned");
+    // the kernel's byte offsets within a sequence are 32-bit
+    if ((int64_t)(max_len + 64) * 3 * hidden * 4 >= (int64_t)1 << 32)
+        return fail(EBH_ERR_RANGE, "max_len %d too long for hidden %d", max_len, hidden);
+    const float scale = 1.0f / sqrtf((float)hd);
+    HIP_TRY(ebh::launch_attention_pair(qkv, cu_seqlens, B, max_len, hidden, num_heads, hd, scale, qkv_scale, ctx,
+                                       ctx_scale, (hipStream_t)stream));
     return EBH_OK;
 }
 

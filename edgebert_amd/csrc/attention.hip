@@ -125,10 +125,10 @@ __device__ __forceinline__ void attend_chunk(const float* Ks, const float* Vs, c
 // workgroups per CU (c3: 69.5 -> 65.8 us per layer against one 128-key chunk);
 // longer sequences keep 128-key chunks, loaded when they are needed, three
 // workgroups per CU (c4: 53.1 against 53.9 us with 64-key chunks).
-template <int HD, int KC, bool PAIR>
+template <int HD, int KC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ? (KC == 64 ? 4 : 3) : 2))) void attention_kernel(
     const float* __restrict__ qkv, const int* __restrict__ cu_seqlens, float* __restrict__ ctx_out, int H, float scale,
-    const int* __restrict__ order, float pair_scale) {
+    const int* __restrict__ order) {
     constexpr bool PREFETCH = KC == 64;
     constexpr int KS = HD + 4;     // K row stride (floats): conflict-free 16-B reads
     constexpr int NJ = HD / 32;    // 32-wide output blocks of the context
@@ -214,16 +214,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ? 
             for (int g = 0; g < 4; ++g) {
                 const float c0 = o[j][4 * g] * inv, c1 = o[j][4 * g + 1] * inv;
                 const float c2 = o[j][4 * g + 2] * inv, c3 = o[j][4 * g + 3] * inv;
-                if constexpr (PAIR) {   // dims 8 g + 4 half ..: half of a 32-byte pair group
-                    uint2 h, l;
-                    split_f16x2(c0 * pair_scale, c1 * pair_scale, h.x, l.x);
-                    split_f16x2(c2 * pair_scale, c3 * pair_scale, h.y, l.y);
-                    uint32_t* const pr = reinterpret_cast<uint32_t*>(ctx_out) + at - 2 * half + j * 32 + 8 * g;
-                    *reinterpret_cast<uint2*>(pr) = h;
-                    *reinterpret_cast<uint2*>(pr + 4) = l;
-                } else {
-                    *reinterpret_cast<float4*>(ctx_out + at + j * 32 + 8 * g) = make_float4(c0, c1, c2, c3);
-                }
+                *reinterpret_cast<float4*>(ctx_out + at + j * 32 + 8 * g) = make_float4(c0, c1, c2, c3);
             }
     }
 }
@@ -630,6 +621,226 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
 }
 
+// ---------------------------------------------------------------------------
+// fp32 attention on fp16 pairs (the fp32 forward above 64 tokens): Q, K, V and
+// the context in the pair format (gemm16.hpp; a head's row is 4 HD bytes, as in
+// fp32), every product from three v_mfma_f32_32x32x16_f16 with fp32 sums.
+//
+// Work split: workgroup = (head, 128-query block, sequence), 4 waves of 32
+// queries; 64-key chunks of K and V in two LDS stages, chunk c + 1 on its way
+// (direct-to-LDS buffer loads; rows past the sequence read as zeros) while
+// chunk c is computed.  A lane's query goes straight to registers.
+//
+// The layouts are those of the kernels above: S^T = K . Q^T, so a lane owns one
+// query's scores; the probabilities, scaled by 2^12 in the exponent (so that l of
+// small ones stays out of fp16's subnormals) and split in registers, are the B
+// operand of O^T = V^T . P^T, whose A operand comes from row-major V through
+// ds_read_b64_tr_b16.  K chunks are swizzled as GEMM rows are.  A half-wave's
+// transposing read takes the h (or l) chunks, every other 16 bytes, of four
+// rows; V's swizzle moves rows r and r + 2 (128-byte rows) or all four
+// (256-byte rows) to different banks.
+//
+// What bounds it: HBM at c3 (201 MB a layer), the softmax's VALU work (the
+// split of P included, it outweighs the twelve MFMAs per 32 x 32 block) on long
+// sequences.  Unlike fp32 MFMAs, fp16 ones leave the VALU free meanwhile.
+// Against the fp32 kernel above, in the forward, per layer: 256 sequences of
+// 128 tokens 76 -> 47 us (4.3 TB/s), 16 of 256-512 53 -> 26 us, 32 of 8-128
+// 12.4 -> 8.3 us; heads of 64, 48 of 16-128 24.9 -> 15.2 us.
+// ---------------------------------------------------------------------------
+template <int HD>
+__device__ __forceinline__ int v_pair_swizzle(int r) {
+    return HD == 32 ? ((r >> 1) & 1) : (r & 1) | ((r >> 1) & 1) << 3;
+}
+
+template <int HD>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ? 4 : 2))) void attention_pair_kernel(
+    const uint32_t* __restrict__ qkv, const int* __restrict__ cu_seqlens, uint32_t* __restrict__ ctx, int H,
+    float c2, float out_mul, const int* __restrict__ order) {
+    constexpr int KC = 64, NB = KC / 32;    // keys per chunk, 32-key blocks
+    constexpr int CPR = HD / 4;             // 16-byte chunks per K / V row
+    constexpr int RB = 4 * HD;              // bytes per K / V row
+    constexpr int NLD = KC * CPR / 256;     // 16-byte loads per thread for K (and for V)
+    constexpr int NJ = HD / 32, NS = HD / 16;
+    constexpr float P_LOG2 = 12.0f;         // probabilities are held times 2^12
+    __shared__ __attribute__((aligned(16))) char Ks[2][KC * RB];
+    __shared__ __attribute__((aligned(16))) char Vs[2][KC * RB];
+
+    const int head = blockIdx.x, qb = blockIdx.y, b = order ? order[blockIdx.z] : (int)blockIdx.z;
+    const int start = cu_seqlens[b];
+    const int len = cu_seqlens[b + 1] - start;
+    if (qb * 128 >= len) return;  // uniform over the workgroup
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, half = lane >> 5;
+    const int64_t ld = 3 * (int64_t)H;
+    const uint32_t ldb = (uint32_t)ld * 4;
+
+    const g16_v4i rsrc = make_rsrc(qkv + (int64_t)start * ld, (uint32_t)len * ldb);
+    uint32_t kvo[NLD], vvo[NLD];
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+        const int P = i * 256 + tid, r = P / CPR, pc = P % CPR;
+        kvo[i] = r * ldb + (H + head * HD) * 4 + 16 * (pc ^ chunk_swizzle16<CPR>(r));
+        vvo[i] = r * ldb + (2 * H + head * HD) * 4 + 16 * (pc ^ v_pair_swizzle<HD>(r));
+    }
+    auto issue = [&](int c) __attribute__((always_inline)) {
+        const uint32_t at = (uint32_t)c * KC * ldb;
+        const uint32_t ks = (uint32_t)(uintptr_t)&Ks[c & 1][0] + wave * 1024, vs = (uint32_t)(uintptr_t)&Vs[c & 1][0] + wave * 1024;
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) load_lds16_buf(rsrc, kvo[i] + at, 0, ks + i * 4096);
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) load_lds16_buf(rsrc, vvo[i] + at, 0, vs + i * 4096);
+    };
+
+    // This lane's query: dims 16 s + 8 half .. +7, h and l.
+    const int q0 = qb * 128 + wave * 32;
+    v8h qh[NS], ql[NS];
+    {
+        const uint32_t* qr = qkv + (int64_t)(start + min(q0 + l32, len - 1)) * ld + head * HD + 8 * half;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            qh[s] = *reinterpret_cast<const v8h*>(qr + 16 * s);
+            ql[s] = *reinterpret_cast<const v8h*>(qr + 16 * s + 4);
+        }
+    }
+    issue(0);
+
+    v16f o[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[j][r] = 0.0f;
+    float m_run = -INFINITY, l_run = 0.0f;
+    const bool active = q0 < len;   // a wave past the sequence's queries only helps load
+    const int g16 = lane >> 4, i16 = lane & 15;
+    const int vrow = i16 >> 2, vdim = 16 * (g16 & 1) + 4 * (i16 & 3);
+    const int nchunks = (len + KC - 1) / KC;
+    for (int c = 0; c < nchunks; ++c) {
+        wait_vmcnt(0);
+        lds_barrier();   // chunk c is here, and everyone is done with chunk c - 1
+        if (c + 1 < nchunks) issue(c + 1);
+        if (!active) continue;
+        const char *K = Ks[c & 1], *V = Vs[c & 1];
+        const int lim = len - c * KC, nkb = min(NB, (lim + 31) / 32);
+        v16f sc[NB];
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sc[kb][r] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int kb = 0; kb < NB; ++kb)
+                if (kb < nkb) {
+                    const int kr = kb * 32 + l32, ch = (2 * (2 * s + half)) ^ chunk_swizzle16<CPR>(kr);
+                    const v8h kh = *reinterpret_cast<const v8h*>(K + kr * RB + 16 * ch);
+                    const v8h kl = *reinterpret_cast<const v8h*>(K + kr * RB + 16 * (ch ^ 1));
+                    sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl, qh[s], sc[kb], 0, 0, 0);
+                    sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, ql[s], sc[kb], 0, 0, 0);
+                    sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qh[s], sc[kb], 0, 0, 0);
+                }
+        // Key-padding mask (src/lib.rs:887-891), only in the block that
+        // straddles the sequence end; the max is taken over the raw scores.
+        float cmax = -INFINITY;
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb)
+            if (kb < nkb) {
+                if ((kb + 1) * 32 > lim) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        if (kb * 32 + 8 * (r >> 2) + 4 * half + (r & 3) >= lim) sc[kb][r] = -INFINITY;
+                }
+#pragma unroll
+                for (int r = 0; r < 16; ++r) cmax = fmaxf(cmax, sc[kb][r]);
+            }
+        cmax = fmaxf(cmax, __shfl_xor(cmax, 32));
+        // 2^12 exp(scale (s - m)) as 2^(s c2 + (12 - m c2)); c2 holds the
+        // scale, log2 e and the operands' scales.
+        const float m_new = fmaxf(m_run, cmax), mc = m_new * c2, off = P_LOG2 - mc;
+        const float alpha = __builtin_amdgcn_exp2f(m_run * c2 - mc);   // 0 on the first chunk
+        float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb)
+            if (kb < nkb) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float pr = __builtin_amdgcn_exp2f(fmaf(sc[kb][r], c2, off));
+                    sc[kb][r] = pr;
+                    ps[r & 3] += pr;
+                }
+            }
+        l_run = l_run * alpha + ((ps[0] + ps[1]) + (ps[2] + ps[3]));
+        m_run = m_new;
+        if (c > 0) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[j][r] *= alpha;
+        }
+        // context^T += V^T . P^T, 16 keys a step: lane half h of P holds keys
+        // 16 mm + 4 h + 0..3 and 16 mm + 8 + 4 h + 0..3.
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb)
+            if (kb < nkb) {
+#pragma unroll
+                for (int mm = 0; mm < 2; ++mm) {
+                    uint32_t hw[4], lw[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) split_f16x2(sc[kb][8 * mm + 2 * e], sc[kb][8 * mm + 2 * e + 1], hw[e], lw[e]);
+                    const v8h ph = __builtin_bit_cast(v8h, make_uint4(hw[0], hw[1], hw[2], hw[3]));
+                    const v8h pl = __builtin_bit_cast(v8h, make_uint4(lw[0], lw[1], lw[2], lw[3]));
+                    const int ra = kb * 32 + 16 * mm + 4 * (g16 >> 1) + vrow, rb = ra + 8;
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) {
+                        const int d = j * 32 + vdim, ch = 2 * (d >> 3), in = 2 * (d & 7);
+                        auto rd = [&](int r, int part) __attribute__((always_inline)) {
+                            return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                (__attribute__((address_space(3))) v4s_t*)(V + r * RB + 16 * ((ch + part) ^ v_pair_swizzle<HD>(r)) + in));
+                        };
+                        const v4s_t ha = rd(ra, 0), hb = rd(rb, 0), la = rd(ra, 1), lb = rd(rb, 1);
+                        const v8h vh = __builtin_bit_cast(v8h, (v8s_t){ha[0], ha[1], ha[2], ha[3], hb[0], hb[1], hb[2], hb[3]});
+                        const v8h vl = __builtin_bit_cast(v8h, (v8s_t){la[0], la[1], la[2], la[3], lb[0], lb[1], lb[2], lb[3]});
+                        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, ph, o[j], 0, 0, 0);
+                        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl, o[j], 0, 0, 0);
+                        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph, o[j], 0, 0, 0);
+                    }
+                }
+            }
+    }
+
+    // Lane holds dims j*32 + 8*g + 4*half + 0..3 (g = r / 4) of query l32.
+    const float l_tot = l_run + __shfl_xor(l_run, 32);
+    const int q = q0 + l32;
+    if (q < len) {
+        const float inv = out_mul / l_tot;   // ctx scale / qkv scale; the 2^12 cancels
+        uint32_t* dst = ctx + (int64_t)(start + q) * H + head * HD + 2 * half;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                uint2 h, l;
+                split_f16x2(o[j][4 * g] * inv, o[j][4 * g + 1] * inv, h.x, l.x);
+                split_f16x2(o[j][4 * g + 2] * inv, o[j][4 * g + 3] * inv, h.y, l.y);
+                *reinterpret_cast<uint2*>(dst + j * 32 + 8 * g) = h;
+                *reinterpret_cast<uint2*>(dst + j * 32 + 8 * g + 4) = l;
+            }
+    }
+}
+
+hipError_t launch_attention_pair(const uint32_t* qkv, const int* cu_seqlens, int B, int max_len, int H, int nh,
+                                 int head_dim, float scale, float qkv_scale, uint32_t* ctx, float ctx_scale,
+                                 hipStream_t s, const int* order) {
+    if (B <= 0 || max_len <= 0) return hipSuccess;
+    const dim3 grid(nh, (max_len + 127) / 128, B), block(256);
+    const float c2 = scale * 1.4426950408889634f / (qkv_scale * qkv_scale), mul = ctx_scale / qkv_scale;
+    if (head_dim == 32)
+        hipLaunchKernelGGL(attention_pair_kernel<32>, grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, mul, order);
+    else if (head_dim == 64)
+        hipLaunchKernelGGL(attention_pair_kernel<64>, grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, mul, order);
+    else
+        return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
 hipError_t launch_attention_bf16(const uint16_t* qkv, const int* cu_seqlens, int B, int max_len,
                                  int H, int nh, int head_dim, float scale, uint16_t* ctx,
                                  hipStream_t s, const int* order) {
@@ -656,32 +867,22 @@ hipError_t launch_attention_bf16(const uint16_t* qkv, const int* cu_seqlens, int
     return hipGetLastError();
 }
 
-template <bool PAIR>
-static hipError_t launch_attention_f32(const float* qkv, const int* cu_seqlens, int B, int max_len, int H,
-                                       int nh, int head_dim, float scale, float* ctx, hipStream_t s, const int* order,
-                                       float pair_scale) {
+hipError_t launch_attention(const float* qkv, const int* cu_seqlens, int B, int max_len, int H,
+                            int nh, int head_dim, float scale, float* ctx, hipStream_t s, const int* order) {
+    if (B <= 0 || max_len <= 0) return hipSuccess;
     const dim3 grid(nh, (max_len + 127) / 128, B), block(256);
     const bool short_seqs = max_len <= 128;
     if (head_dim == 32 && short_seqs)
-        hipLaunchKernelGGL((attention_kernel<32, 64, PAIR>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order, pair_scale);
+        hipLaunchKernelGGL((attention_kernel<32, 64>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order);
     else if (head_dim == 32)
-        hipLaunchKernelGGL((attention_kernel<32, 128, PAIR>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order, pair_scale);
+        hipLaunchKernelGGL((attention_kernel<32, 128>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order);
     else if (head_dim == 64 && short_seqs)
-        hipLaunchKernelGGL((attention_kernel<64, 64, PAIR>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order, pair_scale);
+        hipLaunchKernelGGL((attention_kernel<64, 64>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order);
     else if (head_dim == 64)
-        hipLaunchKernelGGL((attention_kernel<64, 128, PAIR>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order, pair_scale);
+        hipLaunchKernelGGL((attention_kernel<64, 128>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();
-}
-
-hipError_t launch_attention(const float* qkv, const int* cu_seqlens, int B, int max_len, int H,
-                            int nh, int head_dim, float scale, float* ctx, hipStream_t s, const int* order,
-                            float pair_scale) {
-    if (B <= 0 || max_len <= 0) return hipSuccess;
-    return pair_scale > 0.0f
-               ? launch_attention_f32<true>(qkv, cu_seqlens, B, max_len, H, nh, head_dim, scale, ctx, s, order, pair_scale)
-               : launch_attention_f32<false>(qkv, cu_seqlens, B, max_len, H, nh, head_dim, scale, ctx, s, order, 0.0f);
 }
 
 }  // namespace ebh

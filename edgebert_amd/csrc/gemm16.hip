@@ -110,8 +110,8 @@ static hipError_t launch_pair_tile(const Gemm16Args& a, int epi, bool out_pair, 
     const int64_t items = (int64_t)((a.M_max + BM - 1) / BM) * ((a.N + BN - 1) / BN) * (a.splits > 1 ? a.splits : 1);
     if (items == 0) return hipSuccess;
     const dim3 grid((unsigned)std::min<int64_t>(items, (int64_t)device_cu_count() * wpc)), block(64 * WAVES_M * WAVES_N);
-    if (epi == EPI_BIAS && !out_pair)
-        hipLaunchKernelGGL((gemm16_kernel<true, BM, BN, WAVES_M, WAVES_N, NST, EPI_BIAS, OUT_F32>), grid, block, 0, s, a);
+    if (epi == EPI_BIAS && out_pair)
+        hipLaunchKernelGGL((gemm16_kernel<true, BM, BN, WAVES_M, WAVES_N, NST, EPI_BIAS, OUT_PAIR>), grid, block, 0, s, a);
     else if (epi == EPI_NONE && !out_pair)
         hipLaunchKernelGGL((gemm16_kernel<true, BM, BN, WAVES_M, WAVES_N, NST, EPI_NONE, OUT_F32>), grid, block, 0, s, a);
     else if (epi == EPI_BIAS_GELU && out_pair)

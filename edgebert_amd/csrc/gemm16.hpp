@@ -30,38 +30,8 @@
 namespace ebh {
 
 typedef float g16_v4f __attribute__((ext_vector_type(4)));
-typedef int g16_v4i __attribute__((ext_vector_type(4)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef __bf16 g16_v8bf __attribute__((ext_vector_type(8)));
 typedef unsigned int u4v_t __attribute__((ext_vector_type(4)));
-
-// Word 3 of a gfx9 buffer resource descriptor for plain dword-addressed
-// buffers; accesses at or past the descriptor's byte count return 0 (loads,
-// into LDS too) or are dropped (stores).
-constexpr int G16_RSRC_WORD3 = 0x00020000;
-
-// One lane's 16 bytes from a buffer straight into LDS at lds_addr + 16 lane
-// (buffer_load_dwordx4 ... lds; offset = voff + soff).  Issued from inline asm
-// so that the compiler does not make every LDS read wait for it; callers
-// count and wait with wait_vmcnt.
-__device__ __forceinline__ void load_lds16_buf(const g16_v4i& rsrc, uint32_t voff, uint32_t soff, uint32_t lds_addr) {
-    uint32_t saved;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %4\n\t"
-        "s_nop 0\n\t"
-        "buffer_load_dwordx4 %1, %2, %3 offen lds\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_addr)
-        : "memory");
-}
-
-__device__ __forceinline__ g16_v4i make_rsrc(const void* base, uint32_t bytes) {
-    const uint64_t b = uniform_u64(base);
-    return g16_v4i{(int)(uint32_t)b, (int)(uint32_t)((b >> 32) & 0xffffu), __builtin_amdgcn_readfirstlane((int)bytes),
-                   G16_RSRC_WORD3};
-}
 
 enum Out16 : int { OUT_F32 = 0, OUT_PAIR = 1, OUT_BF16 = 2 };
 

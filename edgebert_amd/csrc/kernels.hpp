@@ -72,8 +72,8 @@ Gemm16Plan gemm16_pair_plan(int M, int N, int K, bool gelu, int min_splits, int 
 constexpr int GEMM16_TILES = 7;
 // N % 8 == 0, K % (64 * splits) == 0, strides multiples of 8 elements and at
 // most gemm_stride_max(4), 16-byte aligned operands (hipErrorInvalidValue
-// otherwise).  out_pair: C as pairs of scale out_scale instead of fp32, with
-// EPI_BIAS_GELU; fp32 with EPI_BIAS and EPI_NONE.
+// otherwise).  out_pair: C as pairs of scale out_scale, with EPI_BIAS and
+// EPI_BIAS_GELU; fp32 with EPI_NONE.
 hipError_t launch_gemm16_pair(const Gemm16Args& a, int epi, bool out_pair, int tile, hipStream_t s);
 // y = the pairs of scale * x, n a multiple of 8.
 hipError_t launch_to_pair(const float* x, uint32_t* y, int64_t n, float scale, hipStream_t s);
@@ -112,12 +112,17 @@ hipError_t launch_gemm_bf16(const GemmArgs& a, int epi, hipStream_t s);
 // Masked multi-head attention over packed sequences: qkv [T, 3H] rows
 // (q | k | v), cu_seqlens [B+1]; ctx [T, H].  head_dim 32 or 64.  order
 // (nullable): a permutation of the B sequences, the order in which the grid
-// takes them (launch_pack writes one by decreasing length).  pair_scale > 0:
-// the context is written as fp16 pairs of that scale (gemm16.hpp)
-// instead of fp32 (the same 4 H bytes a row).
+// takes them (launch_pack writes one by decreasing length).
 hipError_t launch_attention(const float* qkv, const int* cu_seqlens, int B, int max_len,
                             int H, int nh, int head_dim, float scale, float* ctx, hipStream_t s,
-                            const int* order = nullptr, float pair_scale = 0.0f);
+                            const int* order = nullptr);
+
+// The same on fp16 pairs (gemm16.hpp): qkv [T, 3H] pairs of scale qkv_scale,
+// ctx [T, H] pairs of scale ctx_scale; scores, softmax and sums fp32.  qkv
+// 16-byte, ctx 8-byte aligned.
+hipError_t launch_attention_pair(const uint32_t* qkv, const int* cu_seqlens, int B, int max_len, int H, int nh,
+                                 int head_dim, float scale, float qkv_scale, uint32_t* ctx, float ctx_scale,
+                                 hipStream_t s, const int* order = nullptr);
 
 // Attention with bf16 q / k / v (qkv [T, 3H] bf16 bits) and bf16 context;
 // scores, softmax and accumulation in fp32.  head_dim 32 or 64.
@@ -341,6 +346,37 @@ __device__ __forceinline__ void load_lds16_sbase(uint64_t sbase, uint32_t voff, 
 }
 __device__ __forceinline__ void load_lds16_sbase(uint64_t sbase, uint32_t voff, const float* lds) {
     load_lds16_sbase(sbase, voff, (uint32_t)(uintptr_t)lds);
+}
+
+typedef int g16_v4i __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+// Word 3 of a gfx9 buffer resource descriptor for plain dword-addressed
+// buffers; accesses at or past the descriptor's byte count return 0 (loads,
+// into LDS too) or are dropped (stores).
+constexpr int G16_RSRC_WORD3 = 0x00020000;
+
+// One lane's 16 bytes from a buffer straight into LDS at lds_addr + 16 lane
+// (buffer_load_dwordx4 ... lds; offset = voff + soff).  Issued from inline asm
+// so that the compiler does not make every LDS read wait for it; callers
+// count and wait with wait_vmcnt.
+__device__ __forceinline__ void load_lds16_buf(const g16_v4i& rsrc, uint32_t voff, uint32_t soff, uint32_t lds_addr) {
+    uint32_t saved;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %4\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %2, %3 offen lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_addr)
+        : "memory");
+}
+
+__device__ __forceinline__ g16_v4i make_rsrc(const void* base, uint32_t bytes) {
+    const uint64_t b = uniform_u64(base);
+    return g16_v4i{(int)(uint32_t)b, (int)(uint32_t)((b >> 32) & 0xffffu), __builtin_amdgcn_readfirstlane((int)bytes),
+                   G16_RSRC_WORD3};
 }
 
 // At most n vector-memory operations of this wave outstanding (n is

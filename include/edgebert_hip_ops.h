@@ -55,8 +55,8 @@ EBH_API int ebh_op_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, 
 /* fp32 products from fp16 pairs, as the fp32 forward runs them above 64 tokens
  * (src/lib.rs:691-698, 732-733, 741-747, 795-849, 958-978): A [M, K] and W
  * [N, K] in the pair format of ebh_op_to_pair with scales sA and sW, acc_scale
- * = 1 / (sA * sW).  c_scale 0: C [M, N] fp32, epilogue EBH_EPI_BIAS or
- * EBH_EPI_NONE; c_scale > 0: C as pairs of that scale, EBH_EPI_BIAS_GELU.
+ * = 1 / (sA * sW).  c_scale > 0: C [M, N] as pairs of that scale, epilogue
+ * EBH_EPI_BIAS or EBH_EPI_BIAS_GELU; c_scale 0: C fp32, EBH_EPI_NONE.
  * splits > 1 (EBH_EPI_NONE): split s sums k in [s K / splits, (s + 1) K /
  * splits) into C + s * split_stride.  tile: -1, or one of 0 .. 6 (256x256,
  * 256x192, 128x128, 128x96, 64x128, 128x64, 64x64); the result does not depend
@@ -80,6 +80,14 @@ EBH_API int ebh_op_to_pair(const float* x, uint32_t* y, int64_t n, float scale, 
  * scale is 1/sqrt(head_dim) as the reference computes it (src/lib.rs:196-197). */
 EBH_API int ebh_op_attention(const float* qkv, const int32_t* cu_seqlens, int32_t B, int32_t max_len,
                      int32_t hidden, int32_t num_heads, float* ctx, void* stream);
+
+/* The same attention on fp16 pairs (ebh_op_to_pair), as the fp32 forward runs it
+ * above 64 tokens: qkv [T, 3*hidden] pairs of scale qkv_scale (16-byte
+ * aligned), ctx [T, hidden] pairs of scale ctx_scale (8-byte aligned); scores,
+ * softmax and sums fp32. */
+EBH_API int ebh_op_attention_pair(const uint32_t* qkv, float qkv_scale, const int32_t* cu_seqlens, int32_t B,
+                          int32_t max_len, int32_t hidden, int32_t num_heads, uint32_t* ctx, float ctx_scale,
+                          void* stream);
 
 /* The same attention for bf16 models: qkv [T, 3*hidden] and ctx [T, hidden]
  * hold bf16 bit patterns (qkv 16-byte, ctx 8-byte aligned); q.k^T, softmax and the P.V

@@ -79,17 +79,21 @@ def test_gemm_pair(env, M, Nn, K, S, tile):
                                    splits, stride, tile, s))
         torch.cuda.synchronize()
 
+    def padding_kept(D):
+        return (D[M:] == 7).all() and (D[:M, Nn:] == 7).all()
+
     C = torch.full((M + 2, ldc), 7.0, device="cuda")
-    run(EPI_BIAS, C, 0.0, vp(b))
-    assert ((C[:M, :Nn].double() - ref - b.double()).abs() <= tol + 2.0 ** -23 * (ref.abs() + b.abs().double())).all()
-    assert (C[M:] == 7).all() and (C[:, Nn:] == 7).all()
-    first = C[:M, :Nn].clone()
+    run(EPI_BIAS, C, sc, vp(b))
+    got = unpair(torch, C[:M], sc)[:, :Nn]
+    u = ref + b.double()
+    assert ((got - u).abs() <= tol + 2.0 ** -22 * (ref.abs() + b.abs().double()) + 2.0 ** -25 / sc).all()
+    assert padding_kept(C)
     if tile > 0:      # every tile sums in the same order
-        C0 = torch.empty_like(C)
-        N.check(L.ebh_op_gemm_pair(vp(Ap), lda, vp(Wp), K, 1 / (sa * sw), vp(b), vp(C0), ldc, 0.0, M, Nn, K, EPI_BIAS,
+        C0 = torch.full((M + 2, ldc), 7.0, device="cuda")
+        N.check(L.ebh_op_gemm_pair(vp(Ap), lda, vp(Wp), K, 1 / (sa * sw), vp(b), vp(C0), ldc, sc, M, Nn, K, EPI_BIAS,
                                    1, 0, 0, s))
         torch.cuda.synchronize()
-        assert torch.equal(C0[:M, :Nn], first)
+        assert torch.equal(C0.view(torch.int32), C.view(torch.int32))
     stride = (M + 1) * ldc
     P = torch.full((S * stride,), 7.0, device="cuda")
     if K % (64 * S) == 0:
@@ -98,13 +102,12 @@ def test_gemm_pair(env, M, Nn, K, S, tile):
         assert ((got - ref).abs() <= tol + 2.0 ** -23 * ref.abs() * S).all()
     D = torch.full((M + 2, ldc), 7.0, device="cuda")
     run(EPI_GELU, D, sc, vp(b))
-    u = ref + b.double()
     want = 0.5 * u * (1 + torch.tanh(0.7978845608028654 * (u + 0.044715 * u ** 3)))
     got = unpair(torch, D[:M], sc)[:, :Nn]
     # GELU's slope is below 1.13; its own error (8 ln2 |t| + 8) 2^-24 |gelu|
     gtol = 1.13 * (tol + 2.0 ** -23 * u.abs()) + (2.0 ** -22 + 2.0 ** -20) * want.abs() + 2.0 ** -25 / sc
     assert ((got - want).abs() <= gtol + 1e-6 * (u < -4)).all()
-    assert (D[M:] == 7).all() and (D[:, Nn:] == 7).all()
+    assert padding_kept(D)
 
 
 def test_gemm_pair_refuses(env):
@@ -119,10 +122,46 @@ def test_gemm_pair_refuses(env):
     bad = N.EBH_ERR_INVALID_ARG
     assert call(K=96) == bad and call(Nn=60) == bad and call(ldc=60) == bad and call(tile=7) == bad
     assert call(epi=EPI_GELU) == bad and call(c_scale=2.0) == bad and call(splits=2) == bad
-    assert call(epi=EPI_BIAS) == bad                       # no bias
+    assert call(epi=EPI_BIAS, c_scale=2.0) == bad          # no bias
     assert call(A=ctypes.c_void_p(t.data_ptr() + 4)) == bad
     assert call(M=0) == N.EBH_OK and call() == N.EBH_OK
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("H,nh", [(384, 12), (768, 12), (64, 1)])
+@pytest.mark.parametrize("lens", [[1], [31, 32, 33, 0, 64, 65], [127, 128, 129, 7], [192, 193, 512, 300]])
+def test_attention_pair(env, H, nh, lens):
+    """Against float64, every length around the 32-key blocks, 64-key chunks and
+    128-query blocks; rows past the last sequence stay untouched."""
+    torch, eb, N, L = env
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator(device="cuda").manual_seed(sum(lens) + H)
+    T, hd = sum(lens), H // nh
+    cu = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32, device="cuda")
+    qkv = torch.randn(T, 3 * H, device="cuda", generator=g)
+    qkv[:, :H] *= 2.0                                # peaked rows too
+    sq, sc = 2.0 ** 9, 2.0 ** 10
+    pairs = to_pair(torch, N, L, qkv, sq, s)
+    ctx = torch.full((T + 3, H), 7.0, device="cuda")
+    N.check(L.ebh_op_attention_pair(vp(pairs), sq, vp(cu), len(lens), max(lens), H, nh, vp(ctx), sc, s))
+    torch.cuda.synchronize()
+    got = unpair(torch, ctx[:T], sc)
+    at = 0
+    for n in lens:
+        x = qkv[at:at + n].double().view(n, 3, nh, hd).permute(1, 2, 0, 3).contiguous()
+        score = torch.matmul(x[0], x[1].transpose(1, 2).contiguous()) / np.sqrt(hd)
+        p = torch.softmax(score, -1)
+        want = torch.matmul(p, x[2]).transpose(0, 1).reshape(n, H)
+        # a score is off by its products' 2^-21 |q||k| sum and the exponent's
+        # few 2^-24 |s c|; that moves a probability by as much, relatively; the
+        # products with V and their split add 2^-21
+        big = (torch.matmul(x[0].abs(), x[1].abs().transpose(1, 2).contiguous()) / np.sqrt(hd)).amax(-1) if n else None
+        if n:
+            rel = 2.0 ** -20 * (1 + big).transpose(0, 1).repeat_interleave(hd, 1)
+            size = torch.matmul(p, x[2].abs()).transpose(0, 1).reshape(n, H)
+            assert ((got[at:at + n] - want).abs() <= rel * size + 2.0 ** -25 / sc).all()
+        at += n
+    assert (ctx[T:] == 7).all()
 
 
 def _spread(w, how):

@@ -438,12 +438,13 @@ int enqueue_pair_layers(ebh_model* m, Workspace& w, int B, int S, int normalize,
         prof_end(m, s, p2, on2);
         return EBH_OK;
     };
-    const int sp_out = ebh::gemm16_pair_plan(T_pad, H, H, false, 1, max_splits).splits,
-              sp_down = ebh::gemm16_pair_plan(T_pad, H, I, false, 1, max_splits).splits;
-    const ebh::Gemm16Plan p_qkv = ebh::gemm16_pair_plan(T, 3 * H, H, false, 1, 1),
-                          p_up = ebh::gemm16_pair_plan(T, I, H, true, 1, 1),
-                          p_out = ebh::gemm16_pair_plan(T, H, H, false, sp_out, sp_out),
-                          p_down = ebh::gemm16_pair_plan(T, H, I, false, sp_down, sp_down);
+    const bool exact = tokens >= 0;
+    const int sp_out = ebh::gemm16_pair_plan(T_pad, false, H, H, false, 1, max_splits).splits,
+              sp_down = ebh::gemm16_pair_plan(T_pad, false, H, I, false, 1, max_splits).splits;
+    const ebh::Gemm16Plan p_qkv = ebh::gemm16_pair_plan(T, exact, 3 * H, H, false, 1, 1),
+                          p_up = ebh::gemm16_pair_plan(T, exact, I, H, true, 1, 1),
+                          p_out = ebh::gemm16_pair_plan(T, exact, H, H, false, sp_out, sp_out),
+                          p_down = ebh::gemm16_pair_plan(T, exact, H, I, false, sp_down, sp_down);
     for (size_t l = 0; l < m->layers.size(); ++l) {
         const DevLayer& L = m->layers[l];
         const PairScales& q = m->pair_scales[l];
@@ -1649,7 +1650,7 @@ int ebh_op_gemm_pair(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t 
     a.split_stride = split_stride;
     a.acc_scale = acc_scale;
     a.out_scale = c_scale;
-    if (tile < 0) tile = ebh::gemm16_pair_plan(M, N, K, epilogue == EBH_EPI_BIAS_GELU, splits, splits).tile;
+    if (tile < 0) tile = ebh::gemm16_pair_plan(M, true, N, K, epilogue == EBH_EPI_BIAS_GELU, splits, splits).tile;
     const hipError_t e = ebh::launch_gemm16_pair(a, epilogue, c_scale > 0.0f, tile, (hipStream_t)stream);
     if (e == hipErrorInvalidValue) return fail(EBH_ERR_INVALID_ARG, "pair gemm shape, stride or alignment");
     if (e != hipSuccess) return fail(EBH_ERR_HIP, "gemm launch failed: %s", hipGetErrorString(e));

@@ -1880,6 +1880,8 @@ hipError_t launch_gemm_bf16_act(const GemmArgs& a, int epi, bool c_bf16, hipStre
     if (c_bf16 && a.N % 8 == 0 && a.ldc % 8 == 0 && (epi == EPI_NONE || aligned16(a.bias))) {
         const int64_t tiles = (int64_t)((a.M_max + 255) / 256) * ((a.N + 255) / 256);
         if (tiles == 0) return hipSuccess;
+        hipError_t err;
+        if (launch_gemm16_bf16(a, epi, s, &err)) return err;   // too few 256 x 256 tiles for the ring kernel
         const dim3 grid((unsigned)std::min<int64_t>(tiles, cu_count())), block(512);
         switch (epi) {
             case EPI_BIAS: hipLaunchKernelGGL(gemm_bf16_ring_kernel<EPI_BIAS>, grid, block, 0, s, a); break;

@@ -3,6 +3,7 @@
 #include "gemm16.hpp"
 
 #include <algorithm>
+#include <cmath>
 
 namespace ebh {
 
@@ -61,47 +62,74 @@ hipError_t launch_row_stats(const float* W, int N, int K, float* norm2, float* a
 // with n items on the busiest CU, wpc of them resident at a time,
 //   launch + sum over rounds of (k-tiles * kt[resident] + resident * epi),
 // the constants (us) fitted to a sweep on MI355X of the four products of
-// MiniLM and BERT-base at 96 .. 49,152 rows and 1 .. 8 splits (rms error of a
-// fit 8-13%; the tile it picks takes 1.03 times the best one's time on
-// average over that sweep).  What the numbers say: a 256-wide tile runs its
-// k-loop fastest but pays a long epilogue (its C is all of a CU's stores), so
-// it wins on many rounds or a long K; small tiles keep a small job on all CUs.
-// Each split beyond the first costs the LayerNorm that follows a read of
-// M * N floats (at 4 TB/s).
+// MiniLM and BERT-base at 96 .. 49,152 rows (bf16: .. 131,072) and 1 .. 8
+// splits (rms error of a fit 6-14%; the tile picked takes 1.025 times the best
+// one's time on average over that sweep).  What the numbers say: a 256-wide
+// tile runs its k-loop fastest but pays a long epilogue (its C is all of a CU's
+// stores), so it wins on many rounds or a long K; small tiles keep a small
+// job on all CUs.  Each split beyond the first costs the LayerNorm that
+// follows a read of M * N floats (at 4 TB/s).
+//
+// Device-buffer calls know only the padded rows, of which a ragged batch fills
+// a part: there the estimate is summed over fills from half to all (all counts
+// twice).  Over the sweep that choice takes 1.08 times the best tile's time on
+// ragged batches and 1.06 on full ones, against 1.13 and 1.025 for one that
+// takes every batch as full.
 // ---------------------------------------------------------------------------
 struct TileCost {
     int bm, bn, wpc;
     float launch, epi, epi_gelu, kt[4];
 };
 static const TileCost kPairTiles[GEMM16_TILES] = {
-    {256, 256, 1, 0.0f, 11.0f, 2.37f, {1.653f}},
-    {256, 192, 1, 0.0f, 9.78f, 1.70f, {1.312f}},
-    {128, 128, 2, 0.96f, 3.27f, 0.17f, {0.703f, 1.144f}},
-    {128, 96, 2, 1.16f, 2.27f, 0.16f, {0.692f, 1.044f}},
-    {64, 128, 2, 2.45f, 1.33f, 0.33f, {0.430f, 0.713f}},
-    {128, 64, 3, 1.84f, 1.53f, 1.11f, {0.455f, 0.692f, 1.079f}},
-    {64, 64, 4, 2.19f, 0.64f, 0.14f, {0.374f, 0.535f, 0.703f, 0.860f}},
+    {256, 256, 1, 0.0f, 10.41f, 1.69f, {1.673f}},
+    {256, 192, 1, 0.0f, 9.06f, 1.40f, {1.330f}},
+    {128, 128, 2, 2.08f, 2.35f, 0.07f, {0.719f, 1.141f}},
+    {128, 96, 2, 1.85f, 1.80f, 0.30f, {0.693f, 1.001f}},
+    {64, 128, 2, 2.98f, 1.00f, 0.44f, {0.429f, 0.709f}},
+    {128, 64, 3, 2.45f, 0.99f, 1.22f, {0.467f, 0.705f, 1.095f}},
+    {64, 64, 4, 2.48f, 0.50f, 0.18f, {0.374f, 0.536f, 0.684f, 0.840f}},
+};
+// bf16; the first is gemm_bf16_ring_kernel (gemm.hip).
+constexpr int BF16_TILES = 6;
+static const TileCost kBf16Tiles[BF16_TILES] = {
+    {256, 256, 1, 0.0f, 4.98f, 2.84f, {1.268f}},
+    {256, 192, 1, 0.0f, 4.94f, 1.50f, {1.050f}},
+    {128, 128, 2, 2.51f, 0.40f, 0.60f, {0.604f, 0.972f}},
+    {128, 96, 2, 2.46f, 0.40f, 0.55f, {0.563f, 0.829f}},
+    {64, 128, 2, 2.94f, 0.20f, 0.44f, {0.396f, 0.600f}},
+    {64, 64, 2, 2.81f, 0.25f, 0.19f, {0.284f, 0.399f}},
 };
 
-Gemm16Plan gemm16_pair_plan(int M, int N, int K, bool gelu, int min_splits, int max_splits) {
+static double tile_us(const TileCost& t, double M, int N, int nk, bool gelu, int S) {
+    const int cus = device_cu_count();
+    const int64_t rows = std::max<int64_t>(1, (int64_t)std::ceil(M / t.bm));
+    const int64_t items = rows * ((N + t.bn - 1) / t.bn) * S, per = (items + cus - 1) / cus;
+    const int64_t full = per / t.wpc, rem = per % t.wpc;
+    const double k = (double)nk / S, e = t.epi + (gelu ? t.epi_gelu : 0.0f);
+    double us = t.launch + full * (k * t.kt[t.wpc - 1] + e * t.wpc) + (S - 1) * (M * N * 4e-6 / 4.0);
+    if (rem) us += k * t.kt[rem - 1] + e * rem;
+    return us;
+}
+
+static double tile_us_of(const TileCost& t, int M, bool exact, int N, int nk, bool gelu, int S) {
+    if (exact) return tile_us(t, M, N, nk, gelu, S);
+    double us = 0.0;
+    for (double fill : {0.5, 0.6, 0.7, 0.8, 0.9, 1.0, 1.0}) us += tile_us(t, fill * M, N, nk, gelu, S);
+    return us;
+}
+
+Gemm16Plan gemm16_pair_plan(int M, bool exact, int N, int K, bool gelu, int min_splits, int max_splits) {
     Gemm16Plan best{0, 1};
     double best_us = 1e30;
-    const int cus = device_cu_count();
-    for (int i = 0; i < GEMM16_TILES; ++i) {
-        const TileCost& t = kPairTiles[i];
+    for (int i = 0; i < GEMM16_TILES; ++i)
         for (int S : {1, 2, 3, 4, 6, 8}) {
             if (S < min_splits || S > std::max(max_splits, 1) || K % (64 * S)) continue;
-            const int64_t items = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * S;
-            const int64_t per = (items + cus - 1) / cus, full = per / t.wpc, rem = per % t.wpc;
-            const double nk = K / 32.0 / S, e = t.epi + (gelu ? t.epi_gelu : 0.0f);
-            double us = t.launch + full * (nk * t.kt[t.wpc - 1] + e * t.wpc) + (S - 1) * ((double)M * N * 4e-6 / 4.0);
-            if (rem) us += nk * t.kt[rem - 1] + e * rem;
+            const double us = tile_us_of(kPairTiles[i], M, exact, N, K / 32, gelu, S);
             if (us < best_us) {
                 best_us = us;
                 best = Gemm16Plan{i, S};
             }
         }
-    }
     return best;
 }
 
@@ -139,6 +167,60 @@ hipError_t launch_gemm16_pair(const Gemm16Args& a, int epi, bool out_pair, int t
         case 5: return launch_pair_tile<128, 64, 2, 2, 2>(a, epi, out_pair, 3, s);
         case 6: return launch_pair_tile<64, 64, 2, 2, 2>(a, epi, out_pair, 4, s);
         default: return hipErrorInvalidValue;
+    }
+}
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, int NST>
+static hipError_t launch_bf16_tile(const Gemm16Args& a, int epi, int wpc, hipStream_t s) {
+    const int64_t items = (int64_t)((a.M_max + BM - 1) / BM) * ((a.N + BN - 1) / BN);
+    const dim3 grid((unsigned)std::min<int64_t>(items, (int64_t)device_cu_count() * wpc)), block(64 * WAVES_M * WAVES_N);
+    switch (epi) {
+        case EPI_BIAS:
+            hipLaunchKernelGGL((gemm16_kernel<false, BM, BN, WAVES_M, WAVES_N, NST, EPI_BIAS, OUT_BF16>), grid, block, 0, s, a);
+            break;
+        case EPI_BIAS_GELU:
+            hipLaunchKernelGGL((gemm16_kernel<false, BM, BN, WAVES_M, WAVES_N, NST, EPI_BIAS_GELU, OUT_BF16>), grid, block, 0, s, a);
+            break;
+        case EPI_NONE:
+            hipLaunchKernelGGL((gemm16_kernel<false, BM, BN, WAVES_M, WAVES_N, NST, EPI_NONE, OUT_BF16>), grid, block, 0, s, a);
+            break;
+        default:
+            return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+bool launch_gemm16_bf16(const GemmArgs& g, int epi, hipStream_t s, hipError_t* err) {
+    if (g.M_max <= 0 || g.K % 128 || g.lda < g.K || g.ldw < g.K || g.ldc < g.N || g.ldc > gemm_stride_max(4)) return false;
+    int best = 0;
+    double best_us = 1e30;
+    for (int i = 0; i < BF16_TILES; ++i) {
+        const double us = tile_us_of(kBf16Tiles[i], g.M_max, g.M_dev == nullptr, g.N, g.K / 64, epi == EPI_BIAS_GELU, 1);
+        if (us < best_us) {
+            best_us = us;
+            best = i;
+        }
+    }
+    Gemm16Args a{};
+    a.A = g.A;
+    a.W = g.W;
+    a.bias = g.bias;
+    a.C = g.C;
+    a.lda = g.lda;
+    a.ldw = g.ldw;
+    a.ldc = g.ldc;
+    a.M_max = g.M_max;
+    a.M_dev = g.M_dev;
+    a.N = g.N;
+    a.K = g.K;
+    a.splits = 1;
+    switch (best) {
+        case 1: *err = launch_bf16_tile<256, 192, 4, 2, 2>(a, epi, 1, s); return true;
+        case 2: *err = launch_bf16_tile<128, 128, 2, 2, 2>(a, epi, 2, s); return true;
+        case 3: *err = launch_bf16_tile<128, 96, 4, 1, 2>(a, epi, 2, s); return true;
+        case 4: *err = launch_bf16_tile<64, 128, 2, 2, 3>(a, epi, 2, s); return true;
+        case 5: *err = launch_bf16_tile<64, 64, 2, 2, 4>(a, epi, 2, s); return true;
+        default: return false;   // the ring kernel
     }
 }
 

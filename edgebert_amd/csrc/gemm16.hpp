@@ -228,17 +228,23 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm16_kernel(Gemm1
         const int er = el & 15, eq = el >> 4;
         const char* bs = smem + NST * STAGE + ((t & 1) * NW + wave) * BIAS_BYTES + 32 * eq;
         const float sc = p.acc_scale, so = p.out_scale;
+        g16_v4f bb0[FN / 2], bb1[FN / 2]; uint32_t vo[FN / 2];
 #pragma unroll
         for (int jp = 0; jp < FN / 2; ++jp) {
-            g16_v4f b0 = {0, 0, 0, 0}, b1 = {0, 0, 0, 0};
+            bb0[jp] = bb1[jp] = g16_v4f{0, 0, 0, 0};
             if (HAS_BIAS) {
-                b0 = *reinterpret_cast<const g16_v4f*>(bs + jp * 128);
-                b1 = *reinterpret_cast<const g16_v4f*>(bs + jp * 128 + 16);
+                bb0[jp] = *reinterpret_cast<const g16_v4f*>(bs + jp * 128);
+                bb1[jp] = *reinterpret_cast<const g16_v4f*>(bs + jp * 128 + 16);
             }
             const int col = n0 + wn * WN + 32 * jp + 8 * eq;
-            const uint32_t voff = col < N ? (uint32_t)(er * (int)rowb + col * CES) : 0xFFFFFFE0u;   // N % 8 == 0
+            vo[jp] = col < N ? (uint32_t)(er * (int)rowb + col * CES) : 0xFFFFFFE0u;   // N % 8 == 0
+        }
 #pragma unroll
-            for (int i = 0; i < FM; ++i) {
+        for (int i = 0; i < FM; ++i) {
+#pragma unroll
+            for (int jp = 0; jp < FN / 2; ++jp) {
+                const g16_v4f b0 = bb0[jp], b1 = bb1[jp];
+                const uint32_t voff = vo[jp];
                 float v[8];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {

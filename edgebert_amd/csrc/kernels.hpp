@@ -64,17 +64,22 @@ struct Gemm16Args {
 
 // Tile and split count the 16-bit products take for a shape: gelu is the FFN
 // up epilogue's cost; split counts from min_splits to max_splits are weighed
-// (above 1 for EPI_NONE only).  M: the row count as far as the host knows it.
+// (above 1 for EPI_NONE only).  exact: M is the row count; else it is the
+// padded one, of which a ragged batch fills a part.
 struct Gemm16Plan {
     int tile, splits;
 };
-Gemm16Plan gemm16_pair_plan(int M, int N, int K, bool gelu, int min_splits, int max_splits);
+Gemm16Plan gemm16_pair_plan(int M, bool exact, int N, int K, bool gelu, int min_splits, int max_splits);
 constexpr int GEMM16_TILES = 7;
 // N % 8 == 0, K % (64 * splits) == 0, strides multiples of 8 elements and at
 // most gemm_stride_max(4), 16-byte aligned operands (hipErrorInvalidValue
 // otherwise).  out_pair: C as pairs of scale out_scale, with EPI_BIAS and
 // EPI_BIAS_GELU; fp32 with EPI_NONE.
 hipError_t launch_gemm16_pair(const Gemm16Args& a, int epi, bool out_pair, int tile, hipStream_t s);
+// The bf16 products of launch_gemm_bf16_act (bf16 C, N and ldc multiples of 8,
+// aligned operands) on the tiles of gemm16.hpp: false, and nothing launched,
+// where the shape is left to the 256 x 256 ring kernel.
+bool launch_gemm16_bf16(const GemmArgs& a, int epi, hipStream_t s, hipError_t* err);
 // y = the pairs of scale * x, n a multiple of 8.
 hipError_t launch_to_pair(const float* x, uint32_t* y, int64_t n, float scale, hipStream_t s);
 // norm2[n], amax[n]: each row's sum of squares and largest magnitude (NaN if

@@ -1,5 +1,6 @@
 """fp32 products from fp16 pairs (ebh_op_to_pair, ebh_op_gemm_pair) against float64
-on every tile, at tile edges and remainders; and models whose weights lie at
+on every tile, at tile edges and remainders; bf16 products at the sizes between
+which their tile changes; and models whose weights lie at
 the ends of the range the pair operands' scales are taken from, or outside it
 (those keep the fp32 kernels), against the CPU oracle."""
 import ctypes
@@ -126,6 +127,30 @@ def test_gemm_pair_refuses(env):
     assert call(A=ctypes.c_void_p(t.data_ptr() + 4)) == bad
     assert call(M=0) == N.EBH_OK and call() == N.EBH_OK
     torch.cuda.synchronize()
+
+
+# the dispatch takes 64x64, 64x128, 128x96, 128x128 and 256x192 tiles and the
+# ring kernel over these sizes; rows and columns end inside a tile
+@pytest.mark.parametrize("M,Nn,K", [(1, 64, 128), (65, 264, 256), (130, 768, 3072), (1300, 2304, 768), (2050, 3072, 768),
+                                    (4353, 768, 3072), (8200, 1544, 384), (8191, 3072, 768), (20481, 2304, 768)])
+@pytest.mark.parametrize("epi", [EPI_BIAS, EPI_GELU, EPI_NONE])
+def test_gemm_bf16_tiles(env, M, Nn, K, epi):
+    torch, eb, N, L = env
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator(device="cuda").manual_seed(M + Nn + K)
+    A = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    W = (0.04 * torch.randn(Nn, K, device="cuda", generator=g)).bfloat16()
+    b = torch.randn(Nn, device="cuda", generator=g)
+    C = torch.full((M + 1, Nn), 7.0, device="cuda", dtype=torch.bfloat16)
+    N.check(L.ebh_op_gemm_bf16(vp(A), K, vp(W), K, vp(b) if epi != EPI_NONE else None, vp(C), Nn, N.EBH_DTYPE_BF16, M,
+                               Nn, K, epi, s))
+    torch.cuda.synchronize()
+    u = A.float() @ W.float().t() + (b if epi != EPI_NONE else 0.0)    # 24-bit sums of exact products
+    want = torch.nn.functional.gelu(u, approximate="tanh") if epi == EPI_GELU else u
+    # the result rounded to bf16, and two differently ordered fp32 sums
+    tol = 2.0 ** -8 * want.abs() + 4e-6 * np.sqrt(K) + 1e-6
+    assert ((C[:M].float() - want).abs() <= tol).all()
+    assert (C[M:] == 7).all()
 
 
 @pytest.mark.parametrize("H,nh", [(384, 12), (768, 12), (64, 1)])

@@ -1690,9 +1690,6 @@ int ebh_op_attention_pair(const uint32_t* qkv, float qkv_scale, const int32_t* c
     if (hd != 32 && hd != 64) return fail(EBH_ERR_INVALID_ARG, "head_dim %d is not 32 or 64", hd);
     if ((uintptr_t)qkv & 15 || (uintptr_t)ctx & 7)
         return fail(EBH_ERR_INVALID_ARG, "qkv must be 16-byte and ctx 8-byte aligned");
-    // the kernel's byte offsets within a sequence are 32-bit
-    if ((int64_t)(max_len + 64) * 3 * hidden * 4 >= (int64_t)1 << 32)
-        return fail(EBH_ERR_RANGE, "max_len %d too long for hidden %d", max_len, hidden);
     const float scale = 1.0f / sqrtf((float)hd);
     HIP_TRY(ebh::launch_attention_pair(qkv, cu_seqlens, B, max_len, hidden, num_heads, hd, scale, qkv_scale, ctx,
                                        ctx_scale, (hipStream_t)stream));

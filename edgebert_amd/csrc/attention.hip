@@ -219,210 +219,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ? 
     }
 }
 
-// ---------------------------------------------------------------------------
-// bf16 variant (models whose GEMMs run in bf16): Q, K, V and the context are
-// bf16; scores, softmax, row sums and the P.V accumulation are fp32.
-//
-// S^T = K . Q^T on v_mfma_f32_32x32x16_bf16: lane (l%32, half h) supplies
-// K row (key) l%32 and Q row (query) l%32, dims 16s + 8h .. +7 of slice s, so
-// the score layout is that of the fp32 kernel (lane owns query l%32; keys
-// 8*(r/4) + 4h + r%4 of each 32-key block).  For P.V, MFMA m (m = 0, 1) of a
-// 32-key block takes r in [8m, 8m+8): lane half h then holds keys
-// 16m + 4h + 0..3 and 16m + 8 + 4h + 0..3, which together cover the 16 keys
-// of that MFMA, so P goes to the A operand straight from registers (rounded to
-// bf16).  The B operand needs, per lane, the same 8 keys at one head dim, so V
-// is staged transposed in LDS (Vt[dim][key], two keys per 32-bit word) and
-// read as two 8-byte runs.
-// ---------------------------------------------------------------------------
 typedef short v8s_t __attribute__((ext_vector_type(8)));
 typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ float bf16_bits_to_f32(uint32_t h) { return __uint_as_float(h << 16); }
-
-template <int HD>
-__global__ __launch_bounds__(256) void attention_bf16_kernel(const uint16_t* __restrict__ qkv,
-                                                             const int* __restrict__ cu_seqlens,
-                                                             uint16_t* __restrict__ ctx, int H,
-                                                             float scale, const int* __restrict__ order) {
-    constexpr int KC = 128;                 // keys per LDS chunk
-    constexpr int KRS = HD + 8;             // K row stride (bf16): 16-byte padding, conflict-free b128 reads
-    constexpr int VTS = KC + 8;             // Vt row stride (bf16): one row per head dim
-    constexpr int NJ = HD / 32;             // 32-wide blocks of the context
-    constexpr int NS = HD / 16;             // 16-dim slices of q.k
-    __shared__ __attribute__((aligned(16))) uint16_t Ks[KC * KRS];
-    __shared__ __attribute__((aligned(16))) uint16_t Vt[HD * VTS];
-
-    const int head = blockIdx.x, qb = blockIdx.y, b = order ? order[blockIdx.z] : (int)blockIdx.z;
-    const int start = cu_seqlens[b];
-    const int len = cu_seqlens[b + 1] - start;
-    if (qb * 128 >= len) return;  // uniform over the workgroup
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int l32 = lane & 31, half = lane >> 5;
-    const int64_t ld = 3 * (int64_t)H;
-    const uint16_t* Qg = qkv + (int64_t)start * ld + head * HD;
-    const uint16_t* Kg = Qg + H;
-    const uint16_t* Vg = Qg + 2 * H;
-
-    // This lane's query as the B operand: dims 16s + 8*half .. +7.
-    const int q0 = qb * 128 + wave * 32;
-    const int qi = min(q0 + l32, len - 1);
-    v8s_t qf[NS];
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-        qf[s] = *reinterpret_cast<const v8s_t*>(Qg + (int64_t)qi * ld + 16 * s + 8 * half);
-
-    v16f o[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[j][r] = 0.0f;
-    float m_run = -INFINITY, l_run = 0.0f;
-
-    const int nchunks = (len + KC - 1) / KC;
-    for (int c = 0; c < nchunks; ++c) {
-        const int kbase = c * KC;
-        __syncthreads();  // previous chunk fully consumed
-        // Every K and V load of the chunk is issued before the first LDS
-        // write (one memory round trip per chunk).  K: 16-byte pieces (8
-        // dims) straight into the padded row layout.  V transposed: a thread
-        // takes keys (2p, 2p+1) x 8 dims and writes 8 words Vt[d][2p .. 2p+1].
-        constexpr int KP = KC * HD / 8, KPT = KP / 256;
-        constexpr int VP = (KC / 2) * (HD / 8), VPT = VP / 256;
-        static_assert(KPT * 256 == KP && VPT * 256 == VP, "whole pieces per thread");
-        uint4 kv[KPT], va[VPT], vb2[VPT];
-#pragma unroll
-        for (int pi = 0; pi < KPT; ++pi) {
-            const int i = tid + 256 * pi, key = kbase + i / (HD / 8), cc = i % (HD / 8);
-            kv[pi] = make_uint4(0, 0, 0, 0);
-            if (key < len) kv[pi] = *reinterpret_cast<const uint4*>(Kg + (int64_t)key * ld + cc * 8);
-        }
-#pragma unroll
-        for (int pi = 0; pi < VPT; ++pi) {
-            const int i = tid + 256 * pi, pr = i % (KC / 2), cc = i / (KC / 2);
-            const int k0 = kbase + 2 * pr;
-            va[pi] = vb2[pi] = make_uint4(0, 0, 0, 0);
-            if (k0 < len) va[pi] = *reinterpret_cast<const uint4*>(Vg + (int64_t)k0 * ld + cc * 8);
-            if (k0 + 1 < len) vb2[pi] = *reinterpret_cast<const uint4*>(Vg + (int64_t)(k0 + 1) * ld + cc * 8);
-        }
-#pragma unroll
-        for (int pi = 0; pi < KPT; ++pi) {
-            const int i = tid + 256 * pi, r = i / (HD / 8), cc = i % (HD / 8);
-            *reinterpret_cast<uint4*>(&Ks[r * KRS + cc * 8]) = kv[pi];
-        }
-#pragma unroll
-        for (int pi = 0; pi < VPT; ++pi) {
-            const int i = tid + 256 * pi, pr = i % (KC / 2), cc = i / (KC / 2);
-            const uint32_t av[4] = {va[pi].x, va[pi].y, va[pi].z, va[pi].w};
-            const uint32_t bv[4] = {vb2[pi].x, vb2[pi].y, vb2[pi].z, vb2[pi].w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int d = cc * 8 + 2 * e;
-                *reinterpret_cast<uint32_t*>(&Vt[d * VTS + 2 * pr]) = (av[e] & 0xFFFFu) | (bv[e] << 16);
-                *reinterpret_cast<uint32_t*>(&Vt[(d + 1) * VTS + 2 * pr]) = (av[e] >> 16) | (bv[e] & 0xFFFF0000u);
-            }
-        }
-        __syncthreads();
-        // A wave whose 32 queries all lie past the sequence end only helps
-        // load K and V.
-        if (q0 >= len) continue;
-
-        const int nkb = min(4, (len - kbase + 31) / 32);  // 32-key blocks holding real keys
-        v16f sc[4];
-        float cmax = -INFINITY;
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            if (kb < nkb) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) sc[kb][r] = 0.0f;
-                const uint16_t* kr = Ks + (kb * 32 + l32) * KRS + 8 * half;
-#pragma unroll
-                for (int s = 0; s < NS; ++s) {
-                    const v8s_t kf = *reinterpret_cast<const v8s_t*>(kr + 16 * s);
-                    sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf_t, kf),
-                                                                      __builtin_bit_cast(v8bf_t, qf[s]),
-                                                                      sc[kb], 0, 0, 0);
-                }
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int key = kbase + kb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-                    float t = sc[kb][r] * scale;         // scale after q.k^T (src/lib.rs:714)
-                    if (key >= len) t = -INFINITY;       // key-padding mask (src/lib.rs:887-891)
-                    sc[kb][r] = t;
-                    cmax = fmaxf(cmax, t);
-                }
-            }
-        }
-        cmax = fmaxf(cmax, __shfl_xor(cmax, 32));
-        const float m_new = fmaxf(m_run, cmax);
-        const float alpha = fast_exp(m_run - m_new);  // 0 on the first chunk
-        float psum = 0.0f;
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            if (kb < nkb) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float pr = fast_exp(sc[kb][r] - m_new);
-                    sc[kb][r] = pr;
-                    psum += pr;
-                }
-            }
-        }
-        l_run = l_run * alpha + psum;
-        m_run = m_new;
-        if (c > 0) {
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[j][r] *= alpha;
-        }
-        // context^T += V^T . P^T over this chunk, two 16-key MFMAs per 32-key
-        // block: A = V^T (row = dim l32, this lane half's 8 keys), B = P^T.
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            if (kb < nkb) {
-#pragma unroll
-                for (int mm = 0; mm < 2; ++mm) {
-                    const float* pf = reinterpret_cast<const float*>(&sc[kb]) + 8 * mm;
-                    const v8s_t pa = __builtin_bit_cast(
-                        v8s_t, make_uint4(pack_bf16x2(pf[0], pf[1]), pack_bf16x2(pf[2], pf[3]),
-                                          pack_bf16x2(pf[4], pf[5]), pack_bf16x2(pf[6], pf[7])));
-                    const int kl = kb * 32 + 16 * mm + 4 * half;   // first of this lane's two 4-key runs
-#pragma unroll
-                    for (int j = 0; j < NJ; ++j) {
-                        const uint16_t* vr = Vt + (j * 32 + l32) * VTS + kl;
-                        const uint2 lo = *reinterpret_cast<const uint2*>(vr);
-                        const uint2 hi = *reinterpret_cast<const uint2*>(vr + 8);
-                        v8s_t vb;
-                        vb[0] = (short)(lo.x & 0xFFFF); vb[1] = (short)(lo.x >> 16);
-                        vb[2] = (short)(lo.y & 0xFFFF); vb[3] = (short)(lo.y >> 16);
-                        vb[4] = (short)(hi.x & 0xFFFF); vb[5] = (short)(hi.x >> 16);
-                        vb[6] = (short)(hi.y & 0xFFFF); vb[7] = (short)(hi.y >> 16);
-                        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf_t, vb),
-                                                                        __builtin_bit_cast(v8bf_t, pa),
-                                                                        o[j], 0, 0, 0);
-                    }
-                }
-            }
-        }
-    }
-
-    // Lane holds dims j*32 + 8*g + 4*half + 0..3 (g = r / 4) of query l32.
-    const float l_tot = l_run + __shfl_xor(l_run, 32);
-    const int q = q0 + l32;
-    if (q < len) {
-        const float inv = 1.0f / l_tot;
-        uint16_t* dst = ctx + (int64_t)(start + q) * H + head * HD + 4 * half;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                *reinterpret_cast<uint2*>(dst + j * 32 + 8 * g) =
-                    make_uint2(pack_bf16x2(o[j][4 * g] * inv, o[j][4 * g + 1] * inv),
-                               pack_bf16x2(o[j][4 * g + 2] * inv, o[j][4 * g + 3] * inv));
-            }
-    }
-}
 
 // ---------------------------------------------------------------------------
 // bf16 attention for sequences of at most 128 tokens: one key chunk and one
@@ -622,9 +420,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 }
 
 // ---------------------------------------------------------------------------
-// fp32 attention on fp16 pairs (the fp32 forward above 64 tokens): Q, K, V and
-// the context in the pair format (gemm16.hpp; a head's row is 4 HD bytes, as in
-// fp32), every product from three v_mfma_f32_32x32x16_f16 with fp32 sums.
+// Attention that streams K and V through LDS, for any length.
+//  * PAIR: the fp32 forward above 64 tokens.  Q, K, V and the context in the
+//    pair format (gemm16.hpp; a head's row is 4 HD bytes, as in fp32), every
+//    product from three v_mfma_f32_32x32x16_f16 with fp32 sums.
+//  * otherwise bf16 models' sequences of more than 128 tokens (the kernel above
+//    takes the shorter ones): Q, K, V, the context and the probabilities bf16,
+//    scores, softmax and sums fp32.
 //
 // Work split: workgroup = (head, 128-query block, sequence), 4 waves of 32
 // queries; 64-key chunks of K and V in two LDS stages, chunk c + 1 on its way
@@ -632,36 +434,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // chunk c is computed.  A lane's query goes straight to registers.
 //
 // The layouts are those of the kernels above: S^T = K . Q^T, so a lane owns one
-// query's scores; the probabilities, scaled by 2^12 in the exponent (so that l of
-// small ones stays out of fp16's subnormals) and split in registers, are the B
-// operand of O^T = V^T . P^T, whose A operand comes from row-major V through
-// ds_read_b64_tr_b16.  K chunks are swizzled as GEMM rows are.  A half-wave's
-// transposing read takes the h (or l) chunks, every other 16 bytes, of four
-// rows; V's swizzle moves rows r and r + 2 (128-byte rows) or all four
-// (256-byte rows) to different banks.
+// query's scores; the probabilities (pairs: scaled by 2^12 in the exponent, so
+// that l of small ones stays out of fp16's subnormals, and split in registers)
+// are the B operand of O^T = V^T . P^T, whose A operand comes from row-major V
+// through ds_read_b64_tr_b16.  K chunks are swizzled as GEMM rows are.  A
+// half-wave's transposing read takes the h (or l) chunks, every other 16 bytes,
+// of four rows (bf16: all chunks of 32 dims); V's swizzle moves rows that share
+// banks (r and r + 2 of 128-byte rows, all four of 256-byte ones) apart.
 //
 // What bounds it: HBM at c3 (201 MB a layer), the softmax's VALU work (the
 // split of P included, it outweighs the twelve MFMAs per 32 x 32 block) on long
 // sequences.  Unlike fp32 MFMAs, fp16 ones leave the VALU free meanwhile.
 // Against the fp32 kernel above, in the forward, per layer: 256 sequences of
 // 128 tokens 76 -> 47 us (4.3 TB/s), 16 of 256-512 53 -> 26 us, 32 of 8-128
-// 12.4 -> 8.3 us; heads of 64, 48 of 16-128 24.9 -> 15.2 us.
+// 12.4 -> 8.3 us; heads of 64, 48 of 16-128 24.9 -> 15.2 us.  bf16 (heads of
+// 64, 40 sequences of 200-512): 72 -> 43 us against 128-key chunks staged
+// through registers with V transposed on its way.
 // ---------------------------------------------------------------------------
 template <int HD>
 __device__ __forceinline__ int v_pair_swizzle(int r) {
     return HD == 32 ? ((r >> 1) & 1) : (r & 1) | ((r >> 1) & 1) << 3;
 }
 
-template <int HD>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ? 4 : 2))) void attention_pair_kernel(
-    const uint32_t* __restrict__ qkv, const int* __restrict__ cu_seqlens, uint32_t* __restrict__ ctx, int H,
-    float c2, float out_mul, const int* __restrict__ order) {
+template <int HD, bool PAIR>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 || !PAIR ? 4 : 2))) void attention_stream_kernel(
+    const void* __restrict__ qkv_, const int* __restrict__ cu_seqlens, void* __restrict__ ctx_, int H, float c2,
+    float out_mul, const int* __restrict__ order) {
     constexpr int KC = 64, NB = KC / 32;    // keys per chunk, 32-key blocks
-    constexpr int CPR = HD / 4;             // 16-byte chunks per K / V row
-    constexpr int RB = 4 * HD;              // bytes per K / V row
+    constexpr int ES = PAIR ? 4 : 2;        // bytes per element
+    constexpr int RB = ES * HD;             // bytes per K / V row
+    constexpr int CPR = RB / 16;            // 16-byte chunks per K / V row
+    const char* qkv = static_cast<const char*>(qkv_);
     constexpr int NLD = KC * CPR / 256;     // 16-byte loads per thread for K (and for V)
     constexpr int NJ = HD / 32, NS = HD / 16;
-    constexpr float P_LOG2 = 12.0f;         // probabilities are held times 2^12
+    constexpr float P_LOG2 = PAIR ? 12.0f : 0.0f;   // pairs: probabilities are held times 2^12
     __shared__ __attribute__((aligned(16))) char Ks[2][KC * RB];
     __shared__ __attribute__((aligned(16))) char Vs[2][KC * RB];
 
@@ -671,35 +477,44 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ? 
     if (qb * 128 >= len) return;  // uniform over the workgroup
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
-    const int64_t ld = 3 * (int64_t)H;
-    const uint32_t ldb = (uint32_t)ld * 4;
+    const uint32_t ldb = 3 * (uint32_t)H * ES;
+    auto v_swz = [](int r) { return PAIR ? v_pair_swizzle<HD>(r) : v_swizzle<HD>(r); };
 
-    const g16_v4i rsrc = make_rsrc(qkv + (int64_t)start * ld, (uint32_t)len * ldb);
     uint32_t kvo[NLD], vvo[NLD];
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         const int P = i * 256 + tid, r = P / CPR, pc = P % CPR;
-        kvo[i] = r * ldb + (H + head * HD) * 4 + 16 * (pc ^ chunk_swizzle16<CPR>(r));
-        vvo[i] = r * ldb + (2 * H + head * HD) * 4 + 16 * (pc ^ v_pair_swizzle<HD>(r));
+        kvo[i] = r * ldb + (H + head * HD) * ES + 16 * (pc ^ chunk_swizzle16<CPR>(r));
+        vvo[i] = r * ldb + (2 * H + head * HD) * ES + 16 * (pc ^ v_swz(r));
     }
     auto issue = [&](int c) __attribute__((always_inline)) {
-        const uint32_t at = (uint32_t)c * KC * ldb;
+        const g16_v4i rsrc = make_rsrc(qkv + (int64_t)(start + c * KC) * ldb, (uint32_t)min(len - c * KC, KC) * ldb);
         const uint32_t ks = (uint32_t)(uintptr_t)&Ks[c & 1][0] + wave * 1024, vs = (uint32_t)(uintptr_t)&Vs[c & 1][0] + wave * 1024;
 #pragma unroll
-        for (int i = 0; i < NLD; ++i) load_lds16_buf(rsrc, kvo[i] + at, 0, ks + i * 4096);
+        for (int i = 0; i < NLD; ++i) load_lds16_buf(rsrc, kvo[i], 0, ks + i * 4096);
 #pragma unroll
-        for (int i = 0; i < NLD; ++i) load_lds16_buf(rsrc, vvo[i] + at, 0, vs + i * 4096);
+        for (int i = 0; i < NLD; ++i) load_lds16_buf(rsrc, vvo[i], 0, vs + i * 4096);
     };
 
-    // This lane's query: dims 16 s + 8 half .. +7, h and l.
+    // One 32 x 32 x 16 product step: PAIR, of (h, l) operands; else of h alone.
+    auto mul = [](const v8h& ah, const v8h& al, const v8h& bh, const v8h& bl, v16f d) __attribute__((always_inline)) {
+        if constexpr (PAIR) {
+            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, d, 0, 0, 0);
+            return __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, d, 0, 0, 0);
+        } else {
+            return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf_t, ah), __builtin_bit_cast(v8bf_t, bh), d, 0, 0, 0);
+        }
+    };
+    // This lane's query: dims 16 s + 8 half .. +7 (h and l).
     const int q0 = qb * 128 + wave * 32;
     v8h qh[NS], ql[NS];
     {
-        const uint32_t* qr = qkv + (int64_t)(start + min(q0 + l32, len - 1)) * ld + head * HD + 8 * half;
+        const char* qr = qkv + (int64_t)(start + min(q0 + l32, len - 1)) * ldb + (head * HD + 8 * half) * ES;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            qh[s] = *reinterpret_cast<const v8h*>(qr + 16 * s);
-            ql[s] = *reinterpret_cast<const v8h*>(qr + 16 * s + 4);
+            qh[s] = *reinterpret_cast<const v8h*>(qr + 16 * ES * s);
+            ql[s] = PAIR ? *reinterpret_cast<const v8h*>(qr + 16 * ES * s + 16) : qh[s];
         }
     }
     issue(0);
@@ -731,12 +546,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ? 
 #pragma unroll
             for (int kb = 0; kb < NB; ++kb)
                 if (kb < nkb) {
-                    const int kr = kb * 32 + l32, ch = (2 * (2 * s + half)) ^ chunk_swizzle16<CPR>(kr);
+                    const int kr = kb * 32 + l32, ch = ((PAIR ? 2 : 1) * (2 * s + half)) ^ chunk_swizzle16<CPR>(kr);
                     const v8h kh = *reinterpret_cast<const v8h*>(K + kr * RB + 16 * ch);
-                    const v8h kl = *reinterpret_cast<const v8h*>(K + kr * RB + 16 * (ch ^ 1));
-                    sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl, qh[s], sc[kb], 0, 0, 0);
-                    sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, ql[s], sc[kb], 0, 0, 0);
-                    sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qh[s], sc[kb], 0, 0, 0);
+                    const v8h kl = PAIR ? *reinterpret_cast<const v8h*>(K + kr * RB + 16 * (ch ^ 1)) : kh;
+                    sc[kb] = mul(kh, kl, qh[s], ql[s], sc[kb]);
                 }
         // Key-padding mask (src/lib.rs:887-891), only in the block that
         // straddles the sequence end; the max is taken over the raw scores.
@@ -753,8 +566,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ? 
                 for (int r = 0; r < 16; ++r) cmax = fmaxf(cmax, sc[kb][r]);
             }
         cmax = fmaxf(cmax, __shfl_xor(cmax, 32));
-        // 2^12 exp(scale (s - m)) as 2^(s c2 + (12 - m c2)); c2 holds the
-        // scale, log2 e and the operands' scales.
+        // exp(scale (s - m)) as 2^(s c2 - m c2) (pairs: times 2^12); c2 holds
+        // the scale, log2 e and the operands' scales.
         const float m_new = fmaxf(m_run, cmax), mc = m_new * c2, off = P_LOG2 - mc;
         const float alpha = __builtin_amdgcn_exp2f(m_run * c2 - mc);   // 0 on the first chunk
         float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -785,23 +598,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ? 
                 for (int mm = 0; mm < 2; ++mm) {
                     uint32_t hw[4], lw[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) split_f16x2(sc[kb][8 * mm + 2 * e], sc[kb][8 * mm + 2 * e + 1], hw[e], lw[e]);
+                    for (int e = 0; e < 4; ++e) {
+                        const float p0 = sc[kb][8 * mm + 2 * e], p1 = sc[kb][8 * mm + 2 * e + 1];
+                        if constexpr (PAIR) split_f16x2(p0, p1, hw[e], lw[e]);
+                        else hw[e] = lw[e] = pack_bf16x2(p0, p1);
+                    }
                     const v8h ph = __builtin_bit_cast(v8h, make_uint4(hw[0], hw[1], hw[2], hw[3]));
                     const v8h pl = __builtin_bit_cast(v8h, make_uint4(lw[0], lw[1], lw[2], lw[3]));
                     const int ra = kb * 32 + 16 * mm + 4 * (g16 >> 1) + vrow, rb = ra + 8;
 #pragma unroll
                     for (int j = 0; j < NJ; ++j) {
-                        const int d = j * 32 + vdim, ch = 2 * (d >> 3), in = 2 * (d & 7);
+                        const int d = j * 32 + vdim, ch = (PAIR ? 2 : 1) * (d >> 3), in = 2 * (d & 7);
                         auto rd = [&](int r, int part) __attribute__((always_inline)) {
                             return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                (__attribute__((address_space(3))) v4s_t*)(V + r * RB + 16 * ((ch + part) ^ v_pair_swizzle<HD>(r)) + in));
+                                (__attribute__((address_space(3))) v4s_t*)(V + r * RB + 16 * ((ch + part) ^ v_swz(r)) + in));
                         };
-                        const v4s_t ha = rd(ra, 0), hb = rd(rb, 0), la = rd(ra, 1), lb = rd(rb, 1);
+                        const v4s_t ha = rd(ra, 0), hb = rd(rb, 0);
                         const v8h vh = __builtin_bit_cast(v8h, (v8s_t){ha[0], ha[1], ha[2], ha[3], hb[0], hb[1], hb[2], hb[3]});
-                        const v8h vl = __builtin_bit_cast(v8h, (v8s_t){la[0], la[1], la[2], la[3], lb[0], lb[1], lb[2], lb[3]});
-                        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, ph, o[j], 0, 0, 0);
-                        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl, o[j], 0, 0, 0);
-                        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph, o[j], 0, 0, 0);
+                        v8h vl = vh;
+                        if constexpr (PAIR) {
+                            const v4s_t la = rd(ra, 1), lb = rd(rb, 1);
+                            vl = __builtin_bit_cast(v8h, (v8s_t){la[0], la[1], la[2], la[3], lb[0], lb[1], lb[2], lb[3]});
+                        }
+                        o[j] = mul(vh, vl, ph, pl, o[j]);
                     }
                 }
             }
@@ -811,17 +630,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ? 
     const float l_tot = l_run + __shfl_xor(l_run, 32);
     const int q = q0 + l32;
     if (q < len) {
-        const float inv = out_mul / l_tot;   // ctx scale / qkv scale; the 2^12 cancels
-        uint32_t* dst = ctx + (int64_t)(start + q) * H + head * HD + 2 * half;
+        const float inv = out_mul / l_tot;   // pairs: ctx scale / qkv scale; the 2^12 cancels
+        char* dst = static_cast<char*>(ctx_) + ((int64_t)(start + q) * H + head * HD) * ES + 8 * half;
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
+                if constexpr (!PAIR) {
+                    *reinterpret_cast<uint2*>(dst + 64 * j + 16 * g) =
+                        make_uint2(pack_bf16x2(o[j][4 * g] * inv, o[j][4 * g + 1] * inv),
+                                   pack_bf16x2(o[j][4 * g + 2] * inv, o[j][4 * g + 3] * inv));
+                    continue;
+                }
                 uint2 h, l;
                 split_f16x2(o[j][4 * g] * inv, o[j][4 * g + 1] * inv, h.x, l.x);
                 split_f16x2(o[j][4 * g + 2] * inv, o[j][4 * g + 3] * inv, h.y, l.y);
-                *reinterpret_cast<uint2*>(dst + j * 32 + 8 * g) = h;
-                *reinterpret_cast<uint2*>(dst + j * 32 + 8 * g + 4) = l;
+                *reinterpret_cast<uint2*>(dst + 128 * j + 32 * g) = h;
+                *reinterpret_cast<uint2*>(dst + 128 * j + 32 * g + 16) = l;
             }
     }
 }
@@ -833,9 +658,9 @@ hipError_t launch_attention_pair(const uint32_t* qkv, const int* cu_seqlens, int
     const dim3 grid(nh, (max_len + 127) / 128, B), block(256);
     const float c2 = scale * 1.4426950408889634f / (qkv_scale * qkv_scale), mul = ctx_scale / qkv_scale;
     if (head_dim == 32)
-        hipLaunchKernelGGL(attention_pair_kernel<32>, grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, mul, order);
+        hipLaunchKernelGGL((attention_stream_kernel<32, true>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, mul, order);
     else if (head_dim == 64)
-        hipLaunchKernelGGL(attention_pair_kernel<64>, grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, mul, order);
+        hipLaunchKernelGGL((attention_stream_kernel<64, true>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, mul, order);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();
@@ -858,10 +683,11 @@ hipError_t launch_attention_bf16(const uint16_t* qkv, const int* cu_seqlens, int
         return hipGetLastError();
     }
     const dim3 grid(nh, (max_len + 127) / 128, B), block(256);
+    const float c2 = scale * 1.4426950408889634f;
     if (head_dim == 32)
-        hipLaunchKernelGGL(attention_bf16_kernel<32>, grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order);
+        hipLaunchKernelGGL((attention_stream_kernel<32, false>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, 1.0f, order);
     else if (head_dim == 64)
-        hipLaunchKernelGGL(attention_bf16_kernel<64>, grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order);
+        hipLaunchKernelGGL((attention_stream_kernel<64, false>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, 1.0f, order);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();

@@ -58,7 +58,7 @@ __device__ __forceinline__ v4f_t mfma4(v4f_t a, v4f_t b, v4f_t c) {
 // over three times as many compute units.
 __global__ __launch_bounds__(64 * FEW_NW) void attn_out_few_kernel(
     const float* __restrict__ qkv, const float* __restrict__ Wo, const int* __restrict__ cu,
-    const int* __restrict__ ntok, int B, int H, float scale, float* __restrict__ Y, int64_t part_stride) {
+    const int* __restrict__ ntok, int B, int T_max, int H, float scale, float* __restrict__ Y, int64_t part_stride) {
     constexpr int QS = 3 * FEW_HD + 4;   // q | k | v row stride in LDS (floats)
     constexpr int PS = FEW_T + 1;        // score row stride
     constexpr int CS = FEW_HD + 4;       // context row stride
@@ -74,7 +74,8 @@ __global__ __launch_bounds__(64 * FEW_NW) void attn_out_few_kernel(
 
     // Every global load goes out before the first wait: this wave's 16
     // output-projection rows (columns h*32 .. +31), the head's q | k | v rows
-    // and the sequence bounds.
+    // and the sequence bounds.  Rows are bounded by T_max, which the buffer has
+    // room for, so that no load waits for the packed count.
     const int n0 = third * (H / 3) + wave * 16;
     v4f_t wf[2];
 #pragma unroll
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(64 * FEW_NW) void attn_out_few_kernel(
     for (int k = 0; k < PPT; ++k) {
         const int e = tid + 64 * FEW_NW * k, t = e / (3 * FEW_HD / 4), c4 = e % (3 * FEW_HD / 4);
         const int part = c4 / (FEW_HD / 4), d4 = c4 % (FEW_HD / 4);
-        if (t < M) pv[k] = ld4(qkv + (int64_t)t * 3 * H + part * H + h * FEW_HD + 4 * d4);
+        if (t < T_max) pv[k] = ld4(qkv + (int64_t)t * 3 * H + part * H + h * FEW_HD + 4 * d4);
     }
     int cb0 = 0, cb1 = 0;
     if (tid < B) {
@@ -96,7 +97,7 @@ __global__ __launch_bounds__(64 * FEW_NW) void attn_out_few_kernel(
 #pragma unroll
     for (int k = 0; k < PPT; ++k) {
         const int e = tid + 64 * FEW_NW * k, t = e / (3 * FEW_HD / 4), c4 = e % (3 * FEW_HD / 4);
-        if (t < M) *reinterpret_cast<v4f_t*>(qkv_s + t * QS + 4 * c4) = pv[k];
+        if (t < T_max) *reinterpret_cast<v4f_t*>(qkv_s + t * QS + 4 * c4) = pv[k];
     }
     // Sequence of each packed token (B <= 64 <= the workgroup's threads).
     if (tid < B)
@@ -108,9 +109,9 @@ __global__ __launch_bounds__(64 * FEW_NW) void attn_out_few_kernel(
 
     // Scores of query t against key jj of its own sequence, scaled after q.k
     // (src/lib.rs:713-714); keys past the sequence are masked out below.
-    for (int e = tid; e < FEW_T * FEW_T; e += 64 * FEW_NW) {
+    for (int e = tid; e < M * FEW_T; e += 64 * FEW_NW) {
         const int t = e / FEW_T, jj = e % FEW_T;
-        if (t >= M || jj >= seq_len[t]) continue;
+        if (jj >= seq_len[t]) continue;
         const float* qr = qkv_s + t * QS;
         const float* kr = qkv_s + (seq_start[t] + jj) * QS + FEW_HD;
         float d = 0.0f;
@@ -140,8 +141,9 @@ __global__ __launch_bounds__(64 * FEW_NW) void attn_out_few_kernel(
         if (lane == 0) inv_s[t] = 1.0f / l;
     }
     __syncthreads();
-    // Context = P . V / row sum (src/lib.rs:723); rows past M are zero.
-    for (int e = tid; e < FEW_T * FEW_HD; e += 64 * FEW_NW) {
+    // Context = P . V / row sum (src/lib.rs:723); rows past M, up to the next
+    // 16, are zero.
+    for (int e = tid; e < ((M + 15) & ~15) * FEW_HD; e += 64 * FEW_NW) {
         const int t = e / FEW_HD, d = e % FEW_HD;
         float c = 0.0f;
         if (t < M) {
@@ -180,8 +182,8 @@ hipError_t launch_attn_out_few(const float* qkv, const float* wo, const int* cu,
                               hipStream_t s) {
     if (!few_attn_fits(T_max, H, nh) || B <= 0 || B > FEW_T || part_stride < (int64_t)T_max * H)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(attn_out_few_kernel, dim3(nh, 3), dim3(64 * FEW_NW), 0, s, qkv, wo, cu, ntok, B, H, scale,
-                       Y, part_stride);
+    hipLaunchKernelGGL(attn_out_few_kernel, dim3(nh, 3), dim3(64 * FEW_NW), 0, s, qkv, wo, cu, ntok, B, T_max, H,
+                       scale, Y, part_stride);
     return hipGetLastError();
 }
 

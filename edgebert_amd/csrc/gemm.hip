@@ -1519,7 +1519,10 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs p) {
 // i, i = 0..3, of column l % 16.  The wave sums are added through LDS in wave
 // order, then either the bias (+ GELU) is applied (one split), or split s is
 // stored at C + s * split_stride (EPI_NONE: the LayerNorm that follows adds
-// the splits in order).
+// the splits in order).  Loads are bounded by M_max, the rows A has room for,
+// and only the stores look at the packed row count: that count is a load of its
+// own from device memory, and waiting for it before A and W put one more
+// round trip in front of every product.
 // ---------------------------------------------------------------------------
 template <int EPI, int NSTEP, int NW>
 __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(GemmArgs p) {
@@ -1531,12 +1534,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(GemmArgs p) {
     const int nslices = N / 32;
     const int blk = blockIdx.x, nb = blk % nslices, m0 = (blk / nslices) * 16, n0 = nb * 32;
     const int split = blockIdx.y;
-    if (m0 >= M) return;  // uniform over the workgroup
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, q = lane >> 4;
     const int KW = K / (NW * S);
     const int kb = split * (K / S) + wave * KW + 4 * q;
-    const float* Ar = static_cast<const float*>(p.A) + (int64_t)min(m0 + r, M - 1) * p.lda + kb;
+    const float* Ar = static_cast<const float*>(p.A) + (int64_t)min(m0 + r, p.M_max - 1) * p.lda + kb;
     const float* W0 = static_cast<const float*>(p.W) + (int64_t)(n0 + r) * p.ldw + kb;
     const float* W1 = W0 + 16 * p.ldw;
     v4f_t acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;

@@ -81,6 +81,7 @@ _SIGS = {
                                 _vp]),
     "ebh_op_gemm_pair": (_i32, [_vp, _i64, _vp, _i64, _f32, _vp, _vp, _i64, _f32, _i32, _i32, _i32, _i32, _i32,
                                 _i64, _i32, _vp]),
+    "ebh_op_ffn_pair": (_i32, [_vp, _vp, _vp, _vp, _f32, _f32, _f32, _vp, _i32, _i32, _i32, _i64, _vp]),
     "ebh_op_attention_pair": (_i32, [_vp, _f32, _vp, _i32, _i32, _i32, _i32, _vp, _f32, _vp]),
     "ebh_op_to_pair": (_i32, [_vp, _vp, _i64, _f32, _vp]),
     "ebh_op_attention": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _vp, _vp]),

@@ -440,11 +440,10 @@ int enqueue_pair_layers(ebh_model* m, Workspace& w, int B, int S, int normalize,
     };
     const bool exact = tokens >= 0;
     const int sp_out = ebh::gemm16_pair_plan(T_pad, false, H, H, false, 1, max_splits).splits,
-              sp_down = ebh::gemm16_pair_plan(T_pad, false, H, I, false, 1, max_splits).splits;
+              sp_down = ebh::ffn_pair_plan(T_pad, false, H, I, 1, max_splits).splits;
     const ebh::Gemm16Plan p_qkv = ebh::gemm16_pair_plan(T, exact, 3 * H, H, false, 1, 1),
-                          p_up = ebh::gemm16_pair_plan(T, exact, I, H, true, 1, 1),
-                          p_out = ebh::gemm16_pair_plan(T, exact, H, H, false, sp_out, sp_out),
-                          p_down = ebh::gemm16_pair_plan(T, exact, H, I, false, sp_down, sp_down);
+                          p_out = ebh::gemm16_pair_plan(T, exact, H, H, false, sp_out, sp_out);
+    const ebh::FfnPairPlan p_ffn = ebh::ffn_pair_plan(T, exact, H, I, sp_down, sp_down);
     for (size_t l = 0; l < m->layers.size(); ++l) {
         const DevLayer& L = m->layers[l];
         const PairScales& q = m->pair_scales[l];
@@ -462,14 +461,34 @@ int enqueue_pair_layers(ebh_model* m, Workspace& w, int B, int S, int normalize,
                        1.0f / (q.ctx * q.wo), 0.0f, p_out)))
             return rc;
         if ((rc = add_ln(L.bo, L.ln1_g, L.ln1_b, p_out.splits, q.mid))) return rc;
-        if ((rc = gemm(EBH_PROF_GEMM_FFN_UP, xp, L.w1p, L.b1, w.F, I, H, ebh::EPI_BIAS_GELU, true,
-                       1.0f / (q.mid * q.w1), q.f, p_up)))
-            return rc;
-        if ((rc = gemm(EBH_PROF_GEMM_FFN_DOWN, w.F, L.w2p, nullptr, w.Y, H, I, ebh::EPI_NONE, false,
-                       1.0f / (q.f * q.w2), 0.0f, p_down)))
-            return rc;
+        if (p_ffn.fused) {   // timed as the FFN down product
+            ebh::FfnPairArgs a{};
+            a.X = xp;
+            a.W1 = L.w1p;
+            a.W2 = L.w2p;
+            a.b1 = L.b1;
+            a.Y = w.Y;
+            a.M_max = T;
+            a.M_dev = w.ntok;
+            a.I = I;
+            a.splits = p_ffn.splits;
+            a.split_stride = (int64_t)T * H;
+            a.scale1 = 1.0f / (q.mid * q.w1);
+            a.scale_g = q.f;
+            a.scale2 = 1.0f / (q.f * q.w2);
+            prof_begin(m, prof_kind, EBH_PROF_GEMM_FFN_DOWN, s, pp, on);
+            HIP_TRY(ebh::launch_ffn_pair(a, s));
+            prof_end(m, s, pp, on);
+        } else {
+            if ((rc = gemm(EBH_PROF_GEMM_FFN_UP, xp, L.w1p, L.b1, w.F, I, H, ebh::EPI_BIAS_GELU, true,
+                           1.0f / (q.mid * q.w1), q.f, p_ffn.up)))
+                return rc;
+            if ((rc = gemm(EBH_PROF_GEMM_FFN_DOWN, w.F, L.w2p, nullptr, w.Y, H, I, ebh::EPI_NONE, false,
+                           1.0f / (q.f * q.w2), 0.0f, p_ffn.down)))
+                return rc;
+        }
         const bool last = l + 1 == m->layers.size();
-        if ((rc = add_ln(L.b2, L.ln2_g, L.ln2_b, p_down.splits, last ? 0.0f : m->pair_scales[l + 1].x))) return rc;
+        if ((rc = add_ln(L.b2, L.ln2_g, L.ln2_b, p_ffn.splits, last ? 0.0f : m->pair_scales[l + 1].x))) return rc;
     }
     return enqueue_pool(m, w, B, S, normalize, d_out, s, d_scores, prof_kind);
 }
@@ -1654,6 +1673,30 @@ int ebh_op_gemm_pair(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t 
     const hipError_t e = ebh::launch_gemm16_pair(a, epilogue, c_scale > 0.0f, tile, (hipStream_t)stream);
     if (e == hipErrorInvalidValue) return fail(EBH_ERR_INVALID_ARG, "pair gemm shape, stride or alignment");
     if (e != hipSuccess) return fail(EBH_ERR_HIP, "gemm launch failed: %s", hipGetErrorString(e));
+    return EBH_OK;
+}
+
+int ebh_op_ffn_pair(const uint32_t* X, const uint32_t* W1, const float* b1, const uint32_t* W2, float scale1,
+                    float g_scale, float scale2, float* Y, int32_t M, int32_t I, int32_t splits,
+                    int64_t split_stride, void* stream) {
+    if (!X || !W1 || !b1 || !W2 || !Y || M < 0 || !(scale1 > 0.0f) || !(g_scale > 0.0f) || !(scale2 > 0.0f))
+        return fail(EBH_ERR_INVALID_ARG, "bad ffn arguments");
+    ebh::FfnPairArgs a{};
+    a.X = X;
+    a.W1 = W1;
+    a.W2 = W2;
+    a.b1 = b1;
+    a.Y = Y;
+    a.M_max = M;
+    a.I = I;
+    a.splits = splits;
+    a.split_stride = split_stride;
+    a.scale1 = scale1;
+    a.scale_g = g_scale;
+    a.scale2 = scale2;
+    const hipError_t e = ebh::launch_ffn_pair(a, (hipStream_t)stream);
+    if (e == hipErrorInvalidValue) return fail(EBH_ERR_INVALID_ARG, "ffn shape, split count or alignment");
+    if (e != hipSuccess) return fail(EBH_ERR_HIP, "ffn launch failed: %s", hipGetErrorString(e));
     return EBH_OK;
 }
 

@@ -111,14 +111,21 @@ static double tile_us(const TileCost& t, double M, int N, int nk, bool gelu, int
     return us;
 }
 
-static double tile_us_of(const TileCost& t, int M, bool exact, int N, int nk, bool gelu, int S) {
-    if (exact) return tile_us(t, M, N, nk, gelu, S);
+// The estimate at M rows, or summed over the fills of M that a device-buffer
+// call may meet.
+template <class F>
+static double over_fills(int M, bool exact, F&& us_at) {
+    if (exact) return us_at((double)M);
     double us = 0.0;
-    for (double fill : {0.5, 0.6, 0.7, 0.8, 0.9, 1.0, 1.0}) us += tile_us(t, fill * M, N, nk, gelu, S);
+    for (double fill : {0.5, 0.6, 0.7, 0.8, 0.9, 1.0, 1.0}) us += us_at(fill * M);
     return us;
 }
 
-Gemm16Plan gemm16_pair_plan(int M, bool exact, int N, int K, bool gelu, int min_splits, int max_splits) {
+static double tile_us_of(const TileCost& t, int M, bool exact, int N, int nk, bool gelu, int S) {
+    return over_fills(M, exact, [&](double m) { return tile_us(t, m, N, nk, gelu, S); });
+}
+
+Gemm16Plan gemm16_pair_plan(int M, bool exact, int N, int K, bool gelu, int min_splits, int max_splits, double* us_out) {
     Gemm16Plan best{0, 1};
     double best_us = 1e30;
     for (int i = 0; i < GEMM16_TILES; ++i)
@@ -130,6 +137,47 @@ Gemm16Plan gemm16_pair_plan(int M, bool exact, int N, int K, bool gelu, int min_
                 best = Gemm16Plan{i, S};
             }
         }
+    if (us_out) *us_out = best_us;
+    return best;
+}
+
+// ffn_pair_kernel: rounds of one workgroup per CU; a chunk of 128 intermediate
+// columns takes 12.6 us with up to half of the CUs at work and 16.6 us with all
+// (measured at 256 .. 40,000 rows, 1 .. 12 splits; a product kernel per step takes
+// as long or longer where these rounds are filled, e.g. 14,355 rows: 105 us in 2
+// splits against 108).  The estimate is weighed at 0.9: the two products' own
+// takes the best tile for granted, which a call that knows only the padded
+// rows often misses (the same rows of 24,750 padded ones, in a forward: 138 us).
+static double ffn_us(double M, int I, int S) {
+    const int cus = device_cu_count();
+    const int64_t items = std::max<int64_t>(1, (int64_t)std::ceil(M / 128)) * S;
+    const double chunks = (double)(I / 128) / S;
+    auto round = [&](int64_t n) {
+        return 3.0 + chunks * 12.6 * (1.0 + 0.64 * std::max(0.0, (double)n / cus - 0.5));
+    };
+    double us = (double)(items / cus) * round(cus) + (S - 1) * (M * 384 * 4e-6 / 4.0);
+    if (items % cus) us += round(items % cus);
+    return us;
+}
+
+FfnPairPlan ffn_pair_plan(int M, bool exact, int H, int I, int min_splits, int max_splits) {
+    FfnPairPlan best{};
+    double up_us = 0.0, best_us = 1e30;
+    best.up = gemm16_pair_plan(M, exact, I, H, true, 1, 1, &up_us);
+    best.down = gemm16_pair_plan(M, exact, H, I, false, min_splits, max_splits, &best_us);
+    best_us += up_us;
+    best.fused = false;
+    best.splits = best.down.splits;
+    if (!ffn_pair_shape_ok(H, I)) return best;
+    for (int S : {1, 2, 3, 4, 6}) {
+        if (S < min_splits || S > std::max(max_splits, 1) || (I / 128) % S) continue;
+        const double us = 0.9 * over_fills(M, exact, [&](double m) { return ffn_us(m, I, S); });
+        if (us < best_us) {
+            best_us = us;
+            best.fused = true;
+            best.splits = S;
+        }
+    }
     return best;
 }
 

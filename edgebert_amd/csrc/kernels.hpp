@@ -69,13 +69,39 @@ struct Gemm16Args {
 struct Gemm16Plan {
     int tile, splits;
 };
-Gemm16Plan gemm16_pair_plan(int M, bool exact, int N, int K, bool gelu, int min_splits, int max_splits);
+Gemm16Plan gemm16_pair_plan(int M, bool exact, int N, int K, bool gelu, int min_splits, int max_splits,
+                            double* us = nullptr);
 constexpr int GEMM16_TILES = 7;
 // N % 8 == 0, K % (64 * splits) == 0, strides multiples of 8 elements and at
 // most gemm_stride_max(4), 16-byte aligned operands (hipErrorInvalidValue
 // otherwise).  out_pair: C as pairs of scale out_scale, with EPI_BIAS and
 // EPI_BIAS_GELU; fp32 with EPI_NONE.
 hipError_t launch_gemm16_pair(const Gemm16Args& a, int epi, bool out_pair, int tile, hipStream_t s);
+// FFN up + GELU + FFN down on fp16 pairs in one launch (ffn.hip), H = 384, I a
+// multiple of 128: partial sums of gelu(X . W1^T + b1) . W2^T, split s over the
+// s-th of `splits` ranges of I (which divides I / 128), at Y + s * split_stride.
+struct FfnPairArgs {
+    const uint32_t* X;    // [M, 384] pairs
+    const uint32_t* W1;   // [I, 384] pairs
+    const uint32_t* W2;   // [384, I] pairs
+    const float* b1;      // [I]
+    float* Y;             // [splits][M, 384]
+    int M_max;
+    const int* M_dev;
+    int I, splits;
+    int64_t split_stride;
+    float scale1, scale_g, scale2;   // 1 / (sX sW1), the GELU output's scale, 1 / (scale_g sW2)
+};
+bool ffn_pair_shape_ok(int H, int I);
+// Whether the FFN runs fused or as its two products, and in how many splits (the
+// result depends on the splits alone).
+struct FfnPairPlan {
+    bool fused;
+    int splits;
+    Gemm16Plan up, down;   // not fused
+};
+FfnPairPlan ffn_pair_plan(int M, bool exact, int H, int I, int min_splits, int max_splits);
+hipError_t launch_ffn_pair(const FfnPairArgs& a, hipStream_t s);
 // The bf16 products of launch_gemm_bf16_act (bf16 C, N and ldc multiples of 8,
 // aligned operands) on the tiles of gemm16.hpp: false, and nothing launched,
 // where the shape is left to the 256 x 256 ring kernel.

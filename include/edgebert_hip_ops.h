@@ -67,6 +67,17 @@ EBH_API int ebh_op_gemm_pair(const uint32_t* A, int64_t lda, const uint32_t* W, 
                      const float* bias, void* C, int64_t ldc, float c_scale, int32_t M, int32_t N, int32_t K,
                      int32_t epilogue, int32_t splits, int64_t split_stride, int32_t tile, void* stream);
 
+/* FFN up + GELU + FFN down in one launch (src/lib.rs:739-750, 958-978), as the
+ * fp32 forward of models of hidden size 384 may run it: split s (of `splits`,
+ * which divides I / 128) of gelu(X.W1^T + b1).W2^T over its range of I, fp32,
+ * without the second bias, to Y + s * split_stride ([M, 384]).  X [M, 384], W1
+ * [I, 384], W2 [384, I] in the pair format, scale1 = 1 / (sX * sW1), g_scale the
+ * scale (a power of two) the GELU output is held at, scale2 = 1 / (g_scale *
+ * sW2).  I % 128 == 0, 16-byte aligned operands. */
+EBH_API int ebh_op_ffn_pair(const uint32_t* X, const uint32_t* W1, const float* b1, const uint32_t* W2, float scale1,
+                    float g_scale, float scale2, float* Y, int32_t M, int32_t I, int32_t splits,
+                    int64_t split_stride, void* stream);
+
 /* The pair format: y holds, for each 8 consecutive values of scale * x, eight
  * fp16 h = fp16(v) and eight fp16 l = fp16(v - h), round to nearest even (32
  * bytes); scale a power of two, n a multiple of 8, x and y 16-byte aligned. */

@@ -111,6 +111,39 @@ def test_gemm_pair(env, M, Nn, K, S, tile):
     assert padding_kept(D)
 
 
+@pytest.mark.parametrize("M,I,S", [(1, 128, 1), (127, 256, 2), (129, 384, 1), (300, 1536, 3), (1000, 1536, 12), (2600, 1536, 1)])
+def test_ffn_pair(env, M, I, S):
+    """Against float64, and bit for bit against the two products that it stands
+    for (the same fragments in the same order), split by split."""
+    torch, eb, N, L = env
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator(device="cuda").manual_seed(M + I)
+    X = torch.randn(M, 384, device="cuda", generator=g)
+    W1 = 0.04 * torch.randn(I, 384, device="cuda", generator=g)
+    W2 = 0.04 * torch.randn(384, I, device="cuda", generator=g)
+    b1 = 0.1 * torch.randn(I, device="cuda", generator=g)
+    sx, sw, sg = 2.0 ** 9, 2.0 ** 15, 2.0 ** 10
+    Xp, W1p, W2p = (to_pair(torch, N, L, t, sc, s) for t, sc in ((X, sx), (W1, sw), (W2, sw)))
+    stride = M * 384 + 64
+    Y = torch.full((S * stride,), 7.0, device="cuda")
+    N.check(L.ebh_op_ffn_pair(vp(Xp), vp(W1p), vp(b1), vp(W2p), 1 / (sx * sw), sg, 1 / (sg * sw), vp(Y), M, I, S, stride, s))
+    F = torch.empty(M, I, device="cuda")
+    N.check(L.ebh_op_gemm_pair(vp(Xp), 384, vp(W1p), 384, 1 / (sx * sw), vp(b1), vp(F), I, sg, M, I, 384, EPI_GELU, 1, 0, -1, s))
+    P = torch.full((S * stride,), 7.0, device="cuda")
+    N.check(L.ebh_op_gemm_pair(vp(F), I, vp(W2p), I, 1 / (sg * sw), None, vp(P), 384, 0.0, M, 384, I, EPI_NONE, S, stride, -1, s))
+    torch.cuda.synchronize()
+    assert torch.equal(Y, P)
+    u = X.double() @ W1.double().t() + b1.double()
+    f = 0.5 * u * (1 + torch.tanh(0.7978845608028654 * (u + 0.044715 * u ** 3)))
+    want = f @ W2.double().t()
+    got = sum(Y[i * stride:i * stride + M * 384].view(M, 384).double() for i in range(S))
+    assert ((got - want).norm() / want.norm()).item() <= 8e-7     # an fp32 MFMA chain over 1,536 is at 7e-7
+    bad = N.EBH_ERR_INVALID_ARG
+    args = (1 / (sx * sw), sg, 1 / (sg * sw), vp(Y), M)
+    assert L.ebh_op_ffn_pair(vp(Xp), vp(W1p), vp(b1), vp(W2p), *args, I, 5, stride, s) == bad
+    assert L.ebh_op_ffn_pair(vp(Xp), vp(W1p), vp(b1), vp(W2p), *args, I + 64, 1, stride, s) == bad
+
+
 def test_gemm_pair_refuses(env):
     torch, eb, N, L = env
     s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)

@@ -394,8 +394,8 @@ int enqueue_pair_layers(ebh_model* m, Workspace& w, int B, int S, int normalize,
     const ebh_config& c = m->cfg;
     const int H = c.hidden_size, I = c.intermediate_size, nh = c.num_attention_heads, hd = H / nh;
     const float eps = c.layer_norm_eps, scale = 1.0f / sqrtf((float)hd);
-    // Grids and tiles are sized by the packed rows where the host counted them,
-    // else by B * S.  Every tile sums a product's k in the same order, so only
+    // Grids and tile families are sized by the packed rows where the host
+    // counted them, else by B * S.  Every tile sums a product's k in the same order, so only
     // the split counts bear on the result: those always go by B * S, and the
     // host and device entry points agree bit for bit.
     const int T_pad = B * S;
@@ -421,10 +421,11 @@ int enqueue_pair_layers(ebh_model* m, Workspace& w, int B, int S, int normalize,
         a.split_stride = (int64_t)T * N;
         a.acc_scale = acc_scale;
         a.out_scale = out_scale;
+        a.tile = -1;
         ProfPair p2{};
         bool on2 = false;
         prof_begin(m, prof_kind, kind, s, p2, on2);
-        hipError_t e = ebh::launch_gemm16_pair(a, epi, out_pair, plan.tile, s);
+        hipError_t e = ebh::launch_gemm16_pair(a, epi, out_pair, plan.family, s);
         prof_end(m, s, p2, on2);
         if (e != hipSuccess) return fail(EBH_ERR_HIP, "gemm launch failed: %s", hipGetErrorString(e));
         return EBH_OK;
@@ -1669,8 +1670,10 @@ int ebh_op_gemm_pair(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t 
     a.split_stride = split_stride;
     a.acc_scale = acc_scale;
     a.out_scale = c_scale;
-    if (tile < 0) tile = ebh::gemm16_pair_plan(M, true, N, K, epilogue == EBH_EPI_BIAS_GELU, splits, splits).tile;
-    const hipError_t e = ebh::launch_gemm16_pair(a, epilogue, c_scale > 0.0f, tile, (hipStream_t)stream);
+    a.tile = tile < 0 ? -1 : tile % 4;
+    const int family = tile < 0 ? ebh::gemm16_pair_plan(M, true, N, K, epilogue == EBH_EPI_BIAS_GELU, splits, splits).family
+                                : tile / 4;
+    const hipError_t e = ebh::launch_gemm16_pair(a, epilogue, c_scale > 0.0f, family, (hipStream_t)stream);
     if (e == hipErrorInvalidValue) return fail(EBH_ERR_INVALID_ARG, "pair gemm shape, stride or alignment");
     if (e != hipSuccess) return fail(EBH_ERR_HIP, "gemm launch failed: %s", hipGetErrorString(e));
     return EBH_OK;

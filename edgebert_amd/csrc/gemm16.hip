@@ -3,7 +3,6 @@
 #include "gemm16.hpp"
 
 #include <algorithm>
-#include <cmath>
 
 namespace ebh {
 
@@ -58,80 +57,86 @@ hipError_t launch_row_stats(const float* W, int N, int K, float* norm2, float* a
 }
 
 // ---------------------------------------------------------------------------
-// Tile choice.  Each tile's time on a shape is estimated from its work items:
-// with n items on the busiest CU, wpc of them resident at a time,
-//   launch + sum over rounds of (k-tiles * kt[resident] + resident * epi),
-// the constants (us) fitted to a sweep on MI355X of the four products of
-// MiniLM and BERT-base at 96 .. 49,152 rows (bf16: .. 131,072) and 1 .. 8
-// splits (rms error of a fit 6-14%; the tile picked takes 1.025 times the best
-// one's time on average over that sweep).  What the numbers say: a 256-wide
-// tile runs its k-loop fastest but pays a long epilogue (its C is all of a CU's
-// stores), so it wins on many rounds or a long K; small tiles keep a small
-// job on all CUs.  Each split beyond the first costs the LayerNorm that
-// follows a read of M * N floats (at 4 TB/s).
+// Family and tile choice: the cost model of gemm16.hpp with constants fitted to
+// a sweep on MI355X of the four products of MiniLM and BERT-base at 96 ..
+// 40,000 rows (bf16: .. 131,072) and 1 .. 6 splits (rms error of a fit 5-10%).
+// What the numbers say: a 256-wide tile runs its k-loop fastest but pays a long
+// epilogue (its C is all of a CU's stores), so it wins on many rounds or a long
+// K; small tiles, two workgroups per CU, keep a small job on all CUs.  Each split
+// beyond the first costs the LayerNorm that follows a read of M * N floats
+// (at 4 TB/s).
 //
 // Device-buffer calls know only the padded rows, of which a ragged batch fills
-// a part: there the estimate is summed over fills from half to all (all counts
-// twice).  Over the sweep that choice takes 1.08 times the best tile's time on
-// ragged batches and 1.06 on full ones, against 1.13 and 1.025 for one that
-// takes every batch as full.
+// a part: the family is the one that is best over fills from half to all (all
+// counts twice), and the kernel picks the tile by the rows it finds.  Over the
+// sweep that takes 1.03 times the best tile's time on ragged batches and 1.025
+// on full ones; a tile picked by the host in the same way took 1.09 and 1.02
+// (3,456 of 6,144 rows of BERT-base: QKV 57, FFN up 58 and FFN down 71 us, on
+// the best tiles 36, 46 and 47).
 // ---------------------------------------------------------------------------
-struct TileCost {
-    int bm, bn, wpc;
-    float launch, epi, epi_gelu, kt[4];
+constexpr int FAMILIES = 2;
+static const TileFamily kPairFamilies[FAMILIES] = {
+    {{{256, 256, 1, 0.0f, 11.02f, 2.07f, {1.714f}},
+      {256, 192, 1, 0.0f, 10.15f, 1.64f, {1.274f}},
+      {256, 128, 1, 0.0f, 7.44f, 1.01f, {1.002f}},
+      {128, 128, 1, 1.39f, 3.54f, 0.68f, {0.677f}}}},
+    {{{128, 128, 2, 2.21f, 2.96f, 0.29f, {0.636f, 1.152f}},
+      {128, 96, 2, 2.30f, 2.12f, 0.38f, {0.556f, 0.968f}},
+      {64, 128, 2, 2.61f, 1.35f, 0.38f, {0.465f, 0.739f}},
+      {64, 64, 2, 2.83f, 0.66f, 0.31f, {0.326f, 0.489f}}}},
 };
-static const TileCost kPairTiles[GEMM16_TILES] = {
-    {256, 256, 1, 0.0f, 10.41f, 1.69f, {1.673f}},
-    {256, 192, 1, 0.0f, 9.06f, 1.40f, {1.330f}},
-    {128, 128, 2, 2.08f, 2.35f, 0.07f, {0.719f, 1.141f}},
-    {128, 96, 2, 1.85f, 1.80f, 0.30f, {0.693f, 1.001f}},
-    {64, 128, 2, 2.98f, 1.00f, 0.44f, {0.429f, 0.709f}},
-    {128, 64, 3, 2.45f, 0.99f, 1.22f, {0.467f, 0.705f, 1.095f}},
-    {64, 64, 4, 2.48f, 0.50f, 0.18f, {0.374f, 0.536f, 0.684f, 0.840f}},
+static const TileFamily kBf16Families[FAMILIES] = {
+    {{{256, 256, 1, 0.0f, 6.71f, 2.50f, {1.127f}},
+      {256, 192, 1, 0.0f, 5.30f, 1.54f, {1.059f}},
+      {256, 128, 1, 0.63f, 3.91f, 1.14f, {0.799f}},
+      {128, 128, 1, 2.26f, 1.51f, 0.80f, {0.580f}}}},
+    {{{128, 128, 2, 2.58f, 1.08f, 0.55f, {0.548f, 0.897f}},
+      {128, 96, 2, 2.49f, 0.72f, 0.50f, {0.489f, 0.759f}},
+      {64, 128, 2, 2.70f, 0.51f, 0.39f, {0.411f, 0.621f}},
+      {64, 64, 2, 2.67f, 0.42f, 0.24f, {0.307f, 0.421f}}}},
 };
-// bf16; the first is gemm_bf16_ring_kernel (gemm.hip).
-constexpr int BF16_TILES = 6;
-static const TileCost kBf16Tiles[BF16_TILES] = {
-    {256, 256, 1, 0.0f, 4.98f, 2.84f, {1.268f}},
-    {256, 192, 1, 0.0f, 4.94f, 1.50f, {1.050f}},
-    {128, 128, 2, 2.51f, 0.40f, 0.60f, {0.604f, 0.972f}},
-    {128, 96, 2, 2.46f, 0.40f, 0.55f, {0.563f, 0.829f}},
-    {64, 128, 2, 2.94f, 0.20f, 0.44f, {0.396f, 0.600f}},
-    {64, 64, 2, 2.81f, 0.25f, 0.19f, {0.284f, 0.399f}},
-};
-
-static double tile_us(const TileCost& t, double M, int N, int nk, bool gelu, int S) {
-    const int cus = device_cu_count();
-    const int64_t rows = std::max<int64_t>(1, (int64_t)std::ceil(M / t.bm));
-    const int64_t items = rows * ((N + t.bn - 1) / t.bn) * S, per = (items + cus - 1) / cus;
-    const int64_t full = per / t.wpc, rem = per % t.wpc;
-    const double k = (double)nk / S, e = t.epi + (gelu ? t.epi_gelu : 0.0f);
-    double us = t.launch + full * (k * t.kt[t.wpc - 1] + e * t.wpc) + (S - 1) * (M * N * 4e-6 / 4.0);
-    if (rem) us += k * t.kt[rem - 1] + e * rem;
-    return us;
-}
+// gemm_bf16_ring_kernel (gemm.hip)
+static const TileFamily kBf16Ring = {{{256, 256, 1, 0.0f, 5.04f, 3.33f, {1.265f}}, {}, {}, {}}};
 
 // The estimate at M rows, or summed over the fills of M that a device-buffer
 // call may meet.
 template <class F>
 static double over_fills(int M, bool exact, F&& us_at) {
-    if (exact) return us_at((double)M);
+    if (exact) return us_at(M);
     double us = 0.0;
-    for (double fill : {0.5, 0.6, 0.7, 0.8, 0.9, 1.0, 1.0}) us += us_at(fill * M);
+    for (double fill : {0.5, 0.6, 0.7, 0.8, 0.9, 1.0, 1.0}) us += us_at(std::max(1, (int)(fill * M)));
     return us;
 }
 
-static double tile_us_of(const TileCost& t, int M, bool exact, int N, int nk, bool gelu, int S) {
-    return over_fills(M, exact, [&](double m) { return tile_us(t, m, N, nk, gelu, S); });
+static TileChoice choice_for(const TileFamily& f, int N, int nk, bool gelu, int S) {
+    TileChoice c{};
+    for (int i = 0; i < FAM_TILES; ++i) {
+        const TileCost& t = f.t[i];
+        if (t.bm == 0) continue;                 // a family of fewer tiles
+        const float k = (float)nk / (float)S, e = t.epi + (gelu ? t.epi_gelu : 0.0f);
+        c.t[i] = {t.bm == 256 ? 8 : (t.bm == 128 ? 7 : 6), (N + t.bn - 1) / t.bn * S, t.wpc == 2, t.launch,
+                  k * t.kt[t.wpc - 1] + e * (float)t.wpc, k * t.kt[0] + e};
+    }
+    c.inv_cus = 1.0f / (float)device_cu_count();
+    return c;
+}
+
+static double family_us(const TileChoice& c, int M) {
+    double best = 1e30;
+    for (int i = 0; i < FAM_TILES; ++i) best = std::min(best, (double)choice_us(c, i, M));
+    return best;
 }
 
 Gemm16Plan gemm16_pair_plan(int M, bool exact, int N, int K, bool gelu, int min_splits, int max_splits, double* us_out) {
     Gemm16Plan best{0, 1};
     double best_us = 1e30;
-    for (int i = 0; i < GEMM16_TILES; ++i)
+    for (int i = 0; i < FAMILIES; ++i)
         for (int S : {1, 2, 3, 4, 6, 8}) {
             if (S < min_splits || S > std::max(max_splits, 1) || K % (64 * S)) continue;
-            const double us = tile_us_of(kPairTiles[i], M, exact, N, K / 32, gelu, S);
+            const TileChoice c = choice_for(kPairFamilies[i], N, K / 32, gelu, S);
+            const double us = over_fills(M, exact, [&](int m) {
+                return family_us(c, m) + (S - 1) * ((double)m * N * 4e-6 / 4.0);
+            });
             if (us < best_us) {
                 best_us = us;
                 best = Gemm16Plan{i, S};
@@ -143,19 +148,18 @@ Gemm16Plan gemm16_pair_plan(int M, bool exact, int N, int K, bool gelu, int min_
 
 // ffn_pair_kernel: rounds of one workgroup per CU; a chunk of 128 intermediate
 // columns takes 12.6 us with up to half of the CUs at work and 16.6 us with all
-// (measured at 256 .. 40,000 rows, 1 .. 12 splits; a product kernel per step takes
-// as long or longer where these rounds are filled, e.g. 14,355 rows: 105 us in 2
-// splits against 108).  The estimate is weighed at 0.9: the two products' own
-// takes the best tile for granted, which a call that knows only the padded
-// rows often misses (the same rows of 24,750 padded ones, in a forward: 138 us).
-static double ffn_us(double M, int I, int S) {
+// (measured at 256 .. 40,000 rows, 1 .. 12 splits; 14,355 rows: 105 us in 2
+// splits, the two products 108 on their best tiles).  The estimate is weighed
+// at 0.95: in a forward the products lose more against these back-to-back
+// timings than this kernel does (32,768 rows: 203 -> 233 us against 201 -> 224).
+static double ffn_us(int M, int I, int S) {
     const int cus = device_cu_count();
-    const int64_t items = std::max<int64_t>(1, (int64_t)std::ceil(M / 128)) * S;
+    const int64_t items = (int64_t)((M + 127) / 128) * S;
     const double chunks = (double)(I / 128) / S;
     auto round = [&](int64_t n) {
         return 3.0 + chunks * 12.6 * (1.0 + 0.64 * std::max(0.0, (double)n / cus - 0.5));
     };
-    double us = (double)(items / cus) * round(cus) + (S - 1) * (M * 384 * 4e-6 / 4.0);
+    double us = (double)(items / cus) * round(cus) + (S - 1) * ((double)M * 384 * 4e-6 / 4.0);
     if (items % cus) us += round(items % cus);
     return us;
 }
@@ -171,7 +175,7 @@ FfnPairPlan ffn_pair_plan(int M, bool exact, int H, int I, int min_splits, int m
     if (!ffn_pair_shape_ok(H, I)) return best;
     for (int S : {1, 2, 3, 4, 6}) {
         if (S < min_splits || S > std::max(max_splits, 1) || (I / 128) % S) continue;
-        const double us = 0.9 * over_fills(M, exact, [&](double m) { return ffn_us(m, I, S); });
+        const double us = 0.95 * over_fills(M, exact, [&](int m) { return ffn_us(m, I, S); });
         if (us < best_us) {
             best_us = us;
             best.fused = true;
@@ -181,74 +185,56 @@ FfnPairPlan ffn_pair_plan(int M, bool exact, int H, int I, int min_splits, int m
     return best;
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int NST>
-static hipError_t launch_pair_tile(const Gemm16Args& a, int epi, bool out_pair, int wpc, hipStream_t s) {
-    const int64_t items = (int64_t)((a.M_max + BM - 1) / BM) * ((a.N + BN - 1) / BN) * (a.splits > 1 ? a.splits : 1);
+// One family's kernel: enough workgroups for the smallest of its tiles, or all
+// that are resident at a time.
+template <bool PAIR, int EPI, int OUT>
+static hipError_t launch_family(Gemm16Args a, int family, hipStream_t s) {
+    const TileFamily& f = (PAIR ? kPairFamilies : kBf16Families)[family];
+    const int S = a.splits > 1 ? a.splits : 1;
+    int64_t items = 0;
+    for (const TileCost& t : f.t)
+        items = std::max(items, (int64_t)((a.M_max + t.bm - 1) / t.bm) * ((a.N + t.bn - 1) / t.bn) * S);
     if (items == 0) return hipSuccess;
-    const dim3 grid((unsigned)std::min<int64_t>(items, (int64_t)device_cu_count() * wpc)), block(64 * WAVES_M * WAVES_N);
-    if (epi == EPI_BIAS && out_pair)
-        hipLaunchKernelGGL((gemm16_kernel<true, BM, BN, WAVES_M, WAVES_N, NST, EPI_BIAS, OUT_PAIR>), grid, block, 0, s, a);
-    else if (epi == EPI_NONE && !out_pair)
-        hipLaunchKernelGGL((gemm16_kernel<true, BM, BN, WAVES_M, WAVES_N, NST, EPI_NONE, OUT_F32>), grid, block, 0, s, a);
-    else if (epi == EPI_BIAS_GELU && out_pair)
-        hipLaunchKernelGGL((gemm16_kernel<true, BM, BN, WAVES_M, WAVES_N, NST, EPI_BIAS_GELU, OUT_PAIR>), grid, block, 0, s, a);
-    else
-        return hipErrorInvalidValue;
+    const TileChoice c = choice_for(f, a.N, a.K / (PAIR ? 32 : 64), EPI == EPI_BIAS_GELU, S);
+    const dim3 grid((unsigned)std::min<int64_t>(items, (int64_t)device_cu_count() * (family == 0 ? 1 : 2)));
+    if (family == 0) hipLaunchKernelGGL((gemm16_kernel<PAIR, 0, EPI, OUT>), grid, dim3(512), 0, s, a, c);
+    else hipLaunchKernelGGL((gemm16_kernel<PAIR, 1, EPI, OUT>), grid, dim3(256), 0, s, a, c);
     return hipGetLastError();
 }
 
-hipError_t launch_gemm16_pair(const Gemm16Args& a, int epi, bool out_pair, int tile, hipStream_t s) {
+hipError_t launch_gemm16_pair(const Gemm16Args& a, int epi, bool out_pair, int family, hipStream_t s) {
     auto al16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
     const int S = a.splits > 1 ? a.splits : 1;
     const bool ok = a.M_max >= 0 && a.N > 0 && a.K > 0 && a.N % 8 == 0 && a.K % (64 * S) == 0 && a.lda % 8 == 0 &&
                     a.ldw % 8 == 0 && a.ldc % 8 == 0 && a.lda >= a.K && a.ldw >= a.K && a.ldc >= a.N &&
                     al16(a.A) && al16(a.W) && al16(a.C) && (S == 1 || (epi == EPI_NONE && a.split_stride % 8 == 0)) &&
                     (epi == EPI_NONE || (a.bias && al16(a.bias))) && gemm_offsets_fit32(a.lda, a.ldw, 4) &&
-                    a.ldc <= gemm_stride_max(4);
+                    a.ldc <= gemm_stride_max(4) && family >= 0 && family < FAMILIES && a.tile < FAM_TILES;
     if (!ok) return hipErrorInvalidValue;
-    switch (tile) {
-        case 0: return launch_pair_tile<256, 256, 2, 4, 2>(a, epi, out_pair, 1, s);
-        case 1: return launch_pair_tile<256, 192, 4, 2, 2>(a, epi, out_pair, 1, s);
-        case 2: return launch_pair_tile<128, 128, 2, 2, 2>(a, epi, out_pair, 2, s);
-        case 3: return launch_pair_tile<128, 96, 4, 1, 2>(a, epi, out_pair, 2, s);
-        case 4: return launch_pair_tile<64, 128, 2, 2, 3>(a, epi, out_pair, 2, s);
-        case 5: return launch_pair_tile<128, 64, 2, 2, 2>(a, epi, out_pair, 3, s);
-        case 6: return launch_pair_tile<64, 64, 2, 2, 2>(a, epi, out_pair, 4, s);
-        default: return hipErrorInvalidValue;
-    }
-}
-
-template <int BM, int BN, int WAVES_M, int WAVES_N, int NST>
-static hipError_t launch_bf16_tile(const Gemm16Args& a, int epi, int wpc, hipStream_t s) {
-    const int64_t items = (int64_t)((a.M_max + BM - 1) / BM) * ((a.N + BN - 1) / BN);
-    const dim3 grid((unsigned)std::min<int64_t>(items, (int64_t)device_cu_count() * wpc)), block(64 * WAVES_M * WAVES_N);
-    switch (epi) {
-        case EPI_BIAS:
-            hipLaunchKernelGGL((gemm16_kernel<false, BM, BN, WAVES_M, WAVES_N, NST, EPI_BIAS, OUT_BF16>), grid, block, 0, s, a);
-            break;
-        case EPI_BIAS_GELU:
-            hipLaunchKernelGGL((gemm16_kernel<false, BM, BN, WAVES_M, WAVES_N, NST, EPI_BIAS_GELU, OUT_BF16>), grid, block, 0, s, a);
-            break;
-        case EPI_NONE:
-            hipLaunchKernelGGL((gemm16_kernel<false, BM, BN, WAVES_M, WAVES_N, NST, EPI_NONE, OUT_BF16>), grid, block, 0, s, a);
-            break;
-        default:
-            return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    if (epi == EPI_BIAS && out_pair) return launch_family<true, EPI_BIAS, OUT_PAIR>(a, family, s);
+    if (epi == EPI_BIAS_GELU && out_pair) return launch_family<true, EPI_BIAS_GELU, OUT_PAIR>(a, family, s);
+    if (epi == EPI_NONE && !out_pair) return launch_family<true, EPI_NONE, OUT_F32>(a, family, s);
+    return hipErrorInvalidValue;
 }
 
 bool launch_gemm16_bf16(const GemmArgs& g, int epi, hipStream_t s, hipError_t* err) {
     if (g.M_max <= 0 || g.K % 128 || g.lda < g.K || g.ldw < g.K || g.ldc < g.N || g.ldc > gemm_stride_max(4)) return false;
-    int best = 0;
-    double best_us = 1e30;
-    for (int i = 0; i < BF16_TILES; ++i) {
-        const double us = tile_us_of(kBf16Tiles[i], g.M_max, g.M_dev == nullptr, g.N, g.K / 64, epi == EPI_BIAS_GELU, 1);
+    const bool exact = g.M_dev == nullptr, gelu = epi == EPI_BIAS_GELU;
+    int best = -1;
+    // The ring kernel's estimate is weighed at 0.92: its three A stages hide what
+    // a forward's cold operands cost the others (131,072 rows, FFN down: 481 us
+    // against 523, where back to back they are within 2%).
+    const TileChoice ring = choice_for(kBf16Ring, g.N, g.K / 64, gelu, 1);
+    double best_us = 0.92 * over_fills(g.M_max, exact, [&](int m) { return (double)choice_us(ring, 0, m); });
+    for (int i = 0; i < FAMILIES; ++i) {
+        const TileChoice c = choice_for(kBf16Families[i], g.N, g.K / 64, gelu, 1);
+        const double us = over_fills(g.M_max, exact, [&](int m) { return family_us(c, m); });
         if (us < best_us) {
             best_us = us;
             best = i;
         }
     }
+    if (best < 0) return false;
     Gemm16Args a{};
     a.A = g.A;
     a.W = g.W;
@@ -262,14 +248,14 @@ bool launch_gemm16_bf16(const GemmArgs& g, int epi, hipStream_t s, hipError_t* e
     a.N = g.N;
     a.K = g.K;
     a.splits = 1;
-    switch (best) {
-        case 1: *err = launch_bf16_tile<256, 192, 4, 2, 2>(a, epi, 1, s); return true;
-        case 2: *err = launch_bf16_tile<128, 128, 2, 2, 2>(a, epi, 2, s); return true;
-        case 3: *err = launch_bf16_tile<128, 96, 4, 1, 2>(a, epi, 2, s); return true;
-        case 4: *err = launch_bf16_tile<64, 128, 2, 2, 3>(a, epi, 2, s); return true;
-        case 5: *err = launch_bf16_tile<64, 64, 2, 2, 4>(a, epi, 2, s); return true;
-        default: return false;   // the ring kernel
+    a.tile = -1;
+    switch (epi) {
+        case EPI_BIAS: *err = launch_family<false, EPI_BIAS, OUT_BF16>(a, best, s); break;
+        case EPI_BIAS_GELU: *err = launch_family<false, EPI_BIAS_GELU, OUT_BF16>(a, best, s); break;
+        case EPI_NONE: *err = launch_family<false, EPI_NONE, OUT_BF16>(a, best, s); break;
+        default: return false;
     }
+    return true;
 }
 
 }  // namespace ebh

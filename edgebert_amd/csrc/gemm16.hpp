@@ -58,8 +58,12 @@ enum Out16 : int { OUT_F32 = 0, OUT_PAIR = 1, OUT_BF16 = 2 };
 // barrier, so that the pipes work while the barrier releases and the first
 // fragments arrive; two sets of W fragments make that possible, and k-tiles
 // come in pairs so that the sets have fixed registers.
-template <bool PAIR, int BM, int BN, int WAVES_M, int WAVES_N, int NST, int EPI, int OUT>
-__global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm16_kernel(Gemm16Args p) {
+constexpr int gemm16_lds(int bm, int bn, int waves, int nsa, int nsw, bool bias) {
+    return (nsa * bm + nsw * bn) * 128 + (bias ? 2 * waves * 1024 : 0);
+}
+
+template <bool PAIR, int BM, int BN, int WAVES_M, int WAVES_N, int NSA, int NSW, int EPI, int OUT>
+__device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, char* const smem) {
     constexpr int NT = 64 * WAVES_M * WAVES_N, NW = WAVES_M * WAVES_N;
     constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
     constexpr int FM = WM / 16, FN = WN / 16;
@@ -68,17 +72,21 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm16_kernel(Gemm1
     static_assert(NS % 2 == 0, "steps alternate between two A sets");
     constexpr int ES = PAIR ? 4 : 2, KT = 128 / ES;
     constexpr int RPT = NT / 8;                   // tile rows a pass of loads covers
-    constexpr int LA = BM / RPT, LW = BN / RPT, NL = LA + LW;
+    constexpr int LA = BM / RPT, LW = BN / RPT;
     static_assert(LA * RPT == BM && LW * RPT == BN && RPT % 32 == 0, "every wave issues the same loads");
-    constexpr int STAGE = (BM + BN) * 128;        // bytes
-    constexpr int D = NST - 1;                    // k-tiles in flight ahead
+    constexpr int ST_A = BM * 128, ST_W = BN * 128;   // bytes of a stage
+    constexpr int W_OFF = NSA * ST_A, B_OFF = W_OFF + NSW * ST_W;
+    // k-tiles in flight ahead.  A streams from HBM (a forward's operands have left
+    // the last-level cache by the time they are read), W comes from the caches:
+    // where the LDS is short A has the deeper ring.
+    constexpr int DA = NSA - 1, DW = NSW - 1;
+    static_assert(DA == DW || DA == DW + 1, "load order");
     constexpr bool HAS_BIAS = EPI != EPI_NONE;
     constexpr int CES = OUT == OUT_BF16 ? 2 : 4;
     constexpr int NSTO = FM * (FN / 2) * (OUT == OUT_BF16 ? 1 : 2);   // stores per lane and tile
     constexpr int BIAS_BYTES = 1024;              // one wave's 64 x 16-byte bias chunks
-    __shared__ __attribute__((aligned(16))) char smem[NST * STAGE + (HAS_BIAS ? 2 * NW * BIAS_BYTES : 0)];
+    static_assert(gemm16_lds(BM, BN, WAVES_M * WAVES_N, NSA, NSW, HAS_BIAS) <= 160 * 1024, "LDS");
 
-    const int M = p.M_dev ? *p.M_dev : p.M_max;
     const int N = p.N;
     const int ntn = (N + BN - 1) / BN, ntiles = ((M + BM - 1) / BM) * ntn;
     const int S = p.splits > 1 ? p.splits : 1;
@@ -112,51 +120,65 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm16_kernel(Gemm1
     const uint32_t lda_b = (uint32_t)p.lda * ES, ldw_b = (uint32_t)p.ldw * ES;
     const uint32_t avoff = r0 * lda_b + chunk, wvoff = rw * ldw_b + chunk;
 
-    // Load cursor: the next k-tile to load, its panels' descriptors and k offset.
+    // Load cursors: the next k-tile of A and of W to load, their panels'
+    // descriptors and k offsets.
     g16_v4i arsrc, wrsrc;
-    uint32_t koff = 0;
+    uint32_t ako = 0, wko = 0;
     const float* bias_src = nullptr;
-    int nit = 0, nkt = 0, nt_ = 0;                 // k-tile count, k-tile within the tile, tile
-    auto point_at = [&](int t) __attribute__((always_inline)) {
-        const int u = u0 + t * ustep, split = u / ntiles, tile = u - split * ntiles;
-        const int mt = tile / ntn, m0 = mt * BM, n0 = (tile - mt * ntn) * BN;
+    int ia = 0, akt = 0, at_ = 0, iw = 0, wkt = 0, wt_ = 0;   // k-tile count, k-tile within the tile, tile
+    auto a_at = [&](int t) __attribute__((always_inline)) {
+        const int u = u0 + t * ustep, split = u / ntiles, tile = u - split * ntiles, m0 = (tile / ntn) * BM;
         arsrc = make_rsrc(static_cast<const char*>(p.A) + (int64_t)m0 * p.lda * ES, (uint32_t)min(M - m0, BM) * lda_b);
+        ako = (uint32_t)(split * nk) * 128;
+    };
+    auto w_at_tile = [&](int t) __attribute__((always_inline)) {
+        const int u = u0 + t * ustep, split = u / ntiles, tile = u - split * ntiles, n0 = (tile - (tile / ntn) * ntn) * BN;
         wrsrc = make_rsrc(static_cast<const char*>(p.W) + (int64_t)n0 * p.ldw * ES, (uint32_t)min(N - n0, BN) * ldw_b);
-        koff = (uint32_t)(split * nk) * 128;
+        wko = (uint32_t)(split * nk) * 128;
         if (HAS_BIAS) bias_src = p.bias + min(n0 + wn * WN + 4 * lane, N - 4);
     };
     int vm = 0;                                    // vector memory instructions issued by this wave
-    int mark[D];                                   // vm after the loads of the next D k-tiles to enter
+    // vm after the last load that the next k-tiles to enter need: their W where A
+    // runs further ahead, else their A.
+    int mark[DW];
 #pragma unroll
-    for (int d = 0; d < D; ++d) mark[d] = 0;
-    constexpr int NPART = NS < 2 ? 1 : 2, PER = (NL + NPART - 1) / NPART;
-    auto issue_part = [&](int part) __attribute__((always_inline)) {
-        const uint32_t st = lds0 + (uint32_t)(nit % NST) * STAGE + (uint32_t)wave * 1024;
+    for (int d = 0; d < DW; ++d) mark[d] = 0;
+    auto issue_w = [&]() __attribute__((always_inline)) {
+        if (iw >= total) return;
+        const uint32_t st = lds0 + W_OFF + (uint32_t)(iw % NSW) * ST_W + (uint32_t)wave * 1024;
 #pragma unroll
-        for (int i = 0; i < NL; ++i)
-            if (i / PER == part) {
-                if (i < LA) load_lds16_buf(arsrc, avoff + i * RPT * lda_b, koff, st + i * RPT * 128);
-                else load_lds16_buf(wrsrc, wvoff + (i - LA) * RPT * ldw_b, koff, st + BM * 128 + (i - LA) * RPT * 128);
-                ++vm;
-            }
-        if (part == NPART - 1) {
-            if (HAS_BIAS && nkt == 0) {
-                load_lds16_async(bias_src, reinterpret_cast<const float*>(smem + NST * STAGE + ((nt_ & 1) * NW + wave) * BIAS_BYTES));
-                ++vm;
-            }
-            mark[D - 1] = vm;
-            ++nit;
-            koff += 128;
-            if (++nkt == nk) {
-                nkt = 0;
-                if (++nt_ < my_tiles) point_at(nt_);
-            }
+        for (int i = 0; i < LW; ++i) load_lds16_buf(wrsrc, wvoff + i * RPT * ldw_b, wko, st + i * RPT * 128);
+        vm += LW;
+        if (HAS_BIAS && wkt == 0) {
+            load_lds16_async(bias_src, reinterpret_cast<const float*>(smem + B_OFF + ((wt_ & 1) * NW + wave) * BIAS_BYTES));
+            ++vm;
+        }
+        if constexpr (DA > DW) mark[DW - 1] = vm;
+        ++iw;
+        wko += 128;
+        if (++wkt == nk) {
+            wkt = 0;
+            if (++wt_ < my_tiles) w_at_tile(wt_);
+        }
+    };
+    auto issue_a = [&]() __attribute__((always_inline)) {
+        if (ia >= total) return;
+        const uint32_t st = lds0 + (uint32_t)(ia % NSA) * ST_A + (uint32_t)wave * 1024;
+#pragma unroll
+        for (int i = 0; i < LA; ++i) load_lds16_buf(arsrc, avoff + i * RPT * lda_b, ako, st + i * RPT * 128);
+        vm += LA;
+        if constexpr (DA == DW) mark[DW - 1] = vm;
+        ++ia;
+        ako += 128;
+        if (++akt == nk) {
+            akt = 0;
+            if (++at_ < my_tiles) a_at(at_);
         }
     };
 
     const int r16 = lane & 15, q16 = lane >> 4;
     const uint32_t frag = r16 * 128 + 16 * ((2 * q16) ^ chunk_swizzle16<8>(r16));
-    const uint32_t a_at = wm * WM * 128 + frag, w_at = BM * 128 + wn * WN * 128 + frag;
+    const uint32_t a_off = wm * WM * 128 + frag, w_off = wn * WN * 128 + frag;
     g16_v4f acc[FM][FN];
     g16_v4f af[2][SB][2], wf[2][FN][2];
 
@@ -164,10 +186,14 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm16_kernel(Gemm1
     auto enter = [&]() __attribute__((always_inline)) {
         const int n = vm - mark[0];
         constexpr auto c = [](int v) { return v > 63 ? 63 : v; };
-        if constexpr (D == 1) wait_vmcnt_of<c(NSTO)>(n);
-        else wait_vmcnt_of<c(NSTO + (D - 1) * NL + 1), c(NSTO + (D - 1) * NL), (D - 1) * NL + 1, (D - 1) * NL>(n);
+        // issued after the loads waited for: later k-tiles' A and W (and a bias),
+        // and a tile's stores
+        constexpr int AH = DA > DW ? LA : (DW - 1) * (LA + LW);
+        if constexpr (AH == 0) wait_vmcnt_of<c(NSTO)>(n);
+        else if constexpr (DA > DW) wait_vmcnt_of<c(NSTO + AH), AH>(n);
+        else wait_vmcnt_of<c(NSTO + AH + 1), c(NSTO + AH), AH + 1, AH>(n);
 #pragma unroll
-        for (int d = 0; d + 1 < D; ++d) mark[d] = mark[d + 1];
+        for (int d = 0; d + 1 < DW; ++d) mark[d] = mark[d + 1];
         lds_barrier();
     };
     auto mfma_step = [&](int s, int as, int ws) __attribute__((always_inline)) {
@@ -191,26 +217,25 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm16_kernel(Gemm1
     };
     auto run_ktile = [&](auto pset, bool first) __attribute__((always_inline)) {
         constexpr int P = decltype(pset)::value;
-        const bool refill = nit < total;
-        const char* st = smem + (it % NST) * STAGE;
+        const char *sa = smem + (it % NSA) * ST_A, *sw = smem + W_OFF + (it % NSW) * ST_W;
         auto rd_a = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < SB; ++i) {
-                const char* at = st + a_at + (s * SB + i) * 16 * 128;
-                af[s & 1][i][0] = *reinterpret_cast<const g16_v4f*>(at);
-                af[s & 1][i][1] = *reinterpret_cast<const g16_v4f*>(st + ((a_at ^ 16) + (s * SB + i) * 16 * 128));
+                af[s & 1][i][0] = *reinterpret_cast<const g16_v4f*>(sa + a_off + (s * SB + i) * 16 * 128);
+                af[s & 1][i][1] = *reinterpret_cast<const g16_v4f*>(sa + (a_off ^ 16) + (s * SB + i) * 16 * 128);
             }
         };
         rd_a(0);
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-            wf[P][j][0] = *reinterpret_cast<const g16_v4f*>(st + w_at + j * 16 * 128);
-            wf[P][j][1] = *reinterpret_cast<const g16_v4f*>(st + (w_at ^ 16) + j * 16 * 128);
+            wf[P][j][0] = *reinterpret_cast<const g16_v4f*>(sw + w_off + j * 16 * 128);
+            wf[P][j][1] = *reinterpret_cast<const g16_v4f*>(sw + (w_off ^ 16) + j * 16 * 128);
         }
         if (!first) mfma_step(NS - 1, 1, P ^ 1);   // the previous k-tile's last step
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            if (refill && s < NPART) issue_part(s);
+            if (s == 0) issue_w();
+            if (s == 1) issue_a();
             if (s + 1 < NS) rd_a(s + 1);
             if (s + 1 < NS) mfma_step(s, s & 1, P);
         }
@@ -226,7 +251,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm16_kernel(Gemm1
         int el = lane;
         asm volatile("" : "+v"(el));
         const int er = el & 15, eq = el >> 4;
-        const char* bs = smem + NST * STAGE + ((t & 1) * NW + wave) * BIAS_BYTES + 32 * eq;
+        const char* bs = smem + B_OFF + ((t & 1) * NW + wave) * BIAS_BYTES + 32 * eq;
         const float sc = p.acc_scale, so = p.out_scale;
         g16_v4f bb0[FN / 2], bb1[FN / 2]; uint32_t vo[FN / 2];
 #pragma unroll
@@ -290,16 +315,18 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm16_kernel(Gemm1
         vm += NSTO;
     };
 
-    point_at(0);
+    // Prologue, in the order of the loop: k-tile d's A before its W where A runs
+    // ahead (whose mark is its W), else W first.
+    a_at(0);
+    w_at_tile(0);
+    if constexpr (DA > DW) issue_a();
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-        if (nit < total) {
-#pragma unroll
-            for (int part = 0; part < NPART; ++part) issue_part(part);
-        }
-        // mark[D - 1] was just set; the d-th k-tile's mark belongs at mark[d]
-        if constexpr (D > 1) mark[d] = vm;
+    for (int d = 0; d < DW; ++d) {
+        issue_w();
+        issue_a();
+        if constexpr (DA == DW) mark[d] = vm;
     }
+    if constexpr (DA > DW) static_assert(DW == 1, "one mark");
     typedef std::integral_constant<int, 0> set0;
     typedef std::integral_constant<int, 1> set1;
     for (int t = 0; t < my_tiles; ++t) {
@@ -319,6 +346,73 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm16_kernel(Gemm1
         }
         mfma_step(NS - 1, 1, 1);
         epilogue(t);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The tiles, in two families that each are one kernel: a device-buffer call
+// knows only the padded row count, so the host picks the family and the kernel,
+// which reads the real count, the tile.  Cost model (us; host and device): with
+// n items on the busiest CU, wpc of them resident at a time,
+//   launch + sum over rounds of (k-tiles * kt[resident] + resident * epi).
+// ---------------------------------------------------------------------------
+struct TileCost {
+    int bm, bn, wpc;
+    float launch, epi, epi_gelu, kt[2];
+};
+constexpr int FAM_TILES = 4;                     // tiles per family
+struct TileFamily {
+    TileCost t[FAM_TILES];
+};
+
+// The model for one shape as the kernel evaluates it: few operations, no
+// divisions, since every launch waits for the choice.
+struct TileChoice {
+    struct {
+        int bm_shift, cols;                      // log2 of the tile's rows; column tiles times splits
+        int two;                                 // two workgroups per CU
+        float launch, full, rem;                 // us: fixed, a full round, a last round of one per CU
+    } t[FAM_TILES];
+    float inv_cus;
+};
+
+__host__ __device__ inline float choice_us(const TileChoice& c, int i, int M) {
+    const int items = ((M + (1 << c.t[i].bm_shift) - 1) >> c.t[i].bm_shift) * c.t[i].cols;
+    const int per = (int)((float)items * c.inv_cus + 0.9999f);
+    const int full = c.t[i].two ? per >> 1 : per, rem = c.t[i].two ? per & 1 : 0;
+    return c.t[i].launch + (float)full * c.t[i].full + (float)rem * c.t[i].rem;
+}
+
+template <bool PAIR, int FAM, int EPI, int OUT>
+__global__ __launch_bounds__(FAM == 0 ? 512 : 256, 2) void gemm16_kernel(Gemm16Args p, TileChoice f) {
+    constexpr bool HB = EPI != EPI_NONE;
+    // With no bias row to keep, 256 x 256 and 128 x 128 have room for a third A stage.
+    constexpr int NA0 = HB ? 2 : 3;
+    __shared__ __attribute__((aligned(16))) char smem[FAM == 0 ? 160 * 1024 : 80 * 1024];
+    const int M = p.M_dev ? *p.M_dev : p.M_max;
+    int tile = p.tile;
+    if (tile < 0) {
+        float best = 1e30f;
+#pragma unroll
+        for (int i = 0; i < FAM_TILES; ++i) {
+            const float us = choice_us(f, i, M);
+            if (us < best) {
+                best = us;
+                tile = i;
+            }
+        }
+    }
+    tile = __builtin_amdgcn_readfirstlane(tile);
+    if constexpr (FAM == 0) {
+        if (tile == 0) gemm16_body<PAIR, 256, 256, 2, 4, NA0, 2, EPI, OUT>(p, M, smem);
+        else if (tile == 1) gemm16_body<PAIR, 256, 192, 4, 2, 3, 2, EPI, OUT>(p, M, smem);
+        else if (tile == 2) gemm16_body<PAIR, 256, 128, 4, 2, 3, 3, EPI, OUT>(p, M, smem);
+        else gemm16_body<PAIR, 128, 128, 2, 4, 4, 4, EPI, OUT>(p, M, smem);
+    } else {
+        if (tile == 0) gemm16_body<PAIR, 128, 128, 2, 2, NA0, 2, EPI, OUT>(p, M, smem);
+        else if (tile == 1) gemm16_body<PAIR, 128, 96, 4, 1, 3, 2, EPI, OUT>(p, M, smem);
+        else if (tile == 2) gemm16_body<PAIR, 64, 128, 2, 2, 3, 3, EPI, OUT>(p, M, smem);
+        else gemm16_body<PAIR, 64, 64, 2, 2, 4, 4, EPI, OUT>(p, M, smem);
     }
 }
 

@@ -60,23 +60,24 @@ struct Gemm16Args {
     int64_t split_stride;
     float acc_scale;     // pairs: 1 / (scale of A * scale of W)
     float out_scale;     // scale of a pair output
+    int tile;            // within the kernel's family; -1: the kernel picks by the row count
 };
 
-// Tile and split count the 16-bit products take for a shape: gelu is the FFN
-// up epilogue's cost; split counts from min_splits to max_splits are weighed
+// Tile family and split count the 16-bit products take for a shape: gelu is the
+// FFN up epilogue's cost; split counts from min_splits to max_splits are weighed
 // (above 1 for EPI_NONE only).  exact: M is the row count; else it is the
 // padded one, of which a ragged batch fills a part.
 struct Gemm16Plan {
-    int tile, splits;
+    int family, splits;
 };
 Gemm16Plan gemm16_pair_plan(int M, bool exact, int N, int K, bool gelu, int min_splits, int max_splits,
                             double* us = nullptr);
-constexpr int GEMM16_TILES = 7;
+constexpr int GEMM16_TILES = 8;   // tile t is number t % 4 of family t / 4
 // N % 8 == 0, K % (64 * splits) == 0, strides multiples of 8 elements and at
 // most gemm_stride_max(4), 16-byte aligned operands (hipErrorInvalidValue
 // otherwise).  out_pair: C as pairs of scale out_scale, with EPI_BIAS and
 // EPI_BIAS_GELU; fp32 with EPI_NONE.
-hipError_t launch_gemm16_pair(const Gemm16Args& a, int epi, bool out_pair, int tile, hipStream_t s);
+hipError_t launch_gemm16_pair(const Gemm16Args& a, int epi, bool out_pair, int family, hipStream_t s);
 // FFN up + GELU + FFN down on fp16 pairs in one launch (ffn.hip), H = 384, I a
 // multiple of 128: partial sums of gelu(X . W1^T + b1) . W2^T, split s over the
 // s-th of `splits` ranges of I (which divides I / 128), at Y + s * split_stride.

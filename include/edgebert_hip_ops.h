@@ -58,9 +58,9 @@ EBH_API int ebh_op_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, 
  * = 1 / (sA * sW).  c_scale > 0: C [M, N] as pairs of that scale, epilogue
  * EBH_EPI_BIAS or EBH_EPI_BIAS_GELU; c_scale 0: C fp32, EBH_EPI_NONE.
  * splits > 1 (EBH_EPI_NONE): split s sums k in [s K / splits, (s + 1) K /
- * splits) into C + s * split_stride.  tile: -1, or one of 0 .. 6 (256x256,
- * 256x192, 128x128, 128x96, 64x128, 128x64, 64x64); the result does not depend
- * on it.  N % 8 == 0, K % (64 splits) == 0, strides (elements) multiples of 8
+ * splits) into C + s * split_stride.  tile: -1 (chosen by the shape), or one of 0 .. 7
+ * (256x256, 256x192, 256x128 and 128x128 on 8 waves; 128x128, 128x96, 64x128
+ * and 64x64 on 4); the result does not depend on it.  N % 8 == 0, K % (64 splits) == 0, strides (elements) multiples of 8
  * and at most 2,796,202, 16-byte aligned operands (EBH_ERR_INVALID_ARG
  * otherwise). */
 EBH_API int ebh_op_gemm_pair(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t ldw, float acc_scale,

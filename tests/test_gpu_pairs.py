@@ -56,7 +56,7 @@ SHAPES = [(1, 64, 64, 1), (63, 96, 128, 2), (65, 200, 192, 3), (129, 392, 384, 1
           (300, 1536, 384, 1), (513, 384, 1536, 4), (1000, 264, 448, 1)]
 
 
-@pytest.mark.parametrize("tile", range(-1, 7))
+@pytest.mark.parametrize("tile", range(-1, 8))
 @pytest.mark.parametrize("M,Nn,K,S", SHAPES)
 def test_gemm_pair(env, M, Nn, K, S, tile):
     torch, eb, N, L = env
@@ -154,7 +154,7 @@ def test_gemm_pair_refuses(env):
                                   tile, s)
 
     bad = N.EBH_ERR_INVALID_ARG
-    assert call(K=96) == bad and call(Nn=60) == bad and call(ldc=60) == bad and call(tile=7) == bad
+    assert call(K=96) == bad and call(Nn=60) == bad and call(ldc=60) == bad and call(tile=8) == bad
     assert call(epi=EPI_GELU) == bad and call(c_scale=2.0) == bad and call(splits=2) == bad
     assert call(epi=EPI_BIAS, c_scale=2.0) == bad          # no bias
     assert call(A=ctypes.c_void_p(t.data_ptr() + 4)) == bad

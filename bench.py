@@ -47,13 +47,36 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-# MI355X published dense peaks: fp32 matrix 157.3 TFLOP/s, bf16 2.5 PFLOP/s; HBM3E 8 TB/s.
-# Dense matrix peaks of MI355X per algorithmic flop: fp32 MFMA, bf16 MFMA, and
-# fp32 products formed from six bf16 MFMA products (the bf16 peak / 6).
-PEAK_TFLOPS = {"fp32": 157.3, "bf16": 2500.0, "fp32-bf16x6": 2500.0 / 6}
+# MI355X published dense peaks: fp32 matrix 157.3 TFLOP/s, bf16 / fp16 2.5 PFLOP/s; HBM3E 8 TB/s.
+# Dense matrix peaks of MI355X per algorithmic flop: fp32 products formed from
+# three fp16 MFMA products (the fp16 peak / 3), bf16 MFMA, and fp32 products
+# formed from six bf16 MFMA products (the bf16 peak / 6).  At most FEW_TOKENS
+# positions the fp32 dtypes run fp32 MFMA.
+PEAK_TFLOPS = {"fp32": 2500.0 / 3, "bf16": 2500.0, "fp32-bf16x6": 2500.0 / 6}
+FP32_MFMA_TFLOPS = 157.3
+FEW_TOKENS = 64
 HBM_PEAK_GBS = 8000.0
 KERNELS = ("gemm_qkv", "attention", "gemm_out", "gemm_ffn_up", "gemm_ffn_down", "layernorm",
            "embed", "pool")
+
+
+def matrix_peak(dtype: str, positions: int) -> float:
+    """The matrix rate (TFLOP/s per algorithmic flop) that bounds a forward of
+    this many padded positions."""
+    return FP32_MFMA_TFLOPS if dtype != "bf16" and positions <= FEW_TOKENS else round(PEAK_TFLOPS[dtype], 1)
+
+
+def gemm_arithmetic(dtype: str, positions: int) -> str:
+    """How the dtype's matrix products are formed at this many padded positions."""
+    if dtype == "bf16":
+        return "bf16 MFMA products, fp32 accumulate"
+    if positions <= FEW_TOKENS:
+        return f"fp32 MFMA products (the few-token kernels, at most {FEW_TOKENS} positions)"
+    if dtype == "fp32":
+        return ("fp32 operands held as fp16 pairs (23 bits), three fp16 MFMA products per fp32 product, "
+                "fp32 accumulate; models whose weights lie outside the pairs' range run fp32 MFMA")
+    return ("fp32 operands split into three bf16 parts, six bf16 MFMA products per fp32 product, "
+            "fp32 accumulate (EBH_DTYPE_F32_BF16X6)")
 
 
 def few_fused(cfg, B: int, S: int, dtype: str) -> bool:
@@ -236,7 +259,7 @@ def split_product_run(eb, torch, spec, weights, d_ids, d_mask, d_ref, lengths, s
     """The same workload on an EBH_DTYPE_F32_BF16X6 model: fp32 weights and
     activations, every large GEMM product formed from six bf16 MFMA products
     of three-way bf16 splits (fp32 accumulate).  Reported beside the headline,
-    which stays on the fp32 MFMA path: sentences/s, its FFN-up roofline
+    whose products are of fp16 pairs: sentences/s, its FFN-up roofline
     against the bf16 peak / 6, and the largest difference of its vectors from
     the fp32 path's on this batch."""
     cfg = spec.model
@@ -272,29 +295,24 @@ def split_product_run(eb, torch, spec, weights, d_ids, d_mask, d_ref, lengths, s
     launches, prof_ms = m.profile_read()
     m.profile_enable("none")
     m.close()
-    # At most 64 positions the few-token kernels run plain fp32 MFMA products
-    # for this dtype too (their products are memory round trips, not MFMA work).
-    few = B * S <= 64
     work, bound, wunit = kernel_work(cfg, lengths, B, profile_kernel, few_fused(cfg, B, S, "fp32-bf16x6"))
     avg = prof_ms / max(launches, 1)
-    peak = PEAK_TFLOPS["fp32" if few else "fp32-bf16x6"] if bound == "mfma" else HBM_PEAK_GBS
+    peak = matrix_peak("fp32-bf16x6", B * S) if bound == "mfma" else HBM_PEAK_GBS
     achieved = work / (avg * 1e-3) / (1e12 if bound == "mfma" else 1e9)
     return {"value": round(B * steps / wall, 2), "unit": "sentences/s",
             "ms_per_step": round(1e3 * wall / steps, 4),
             "p50_batch_latency_ms": round(float(np.median(times)) * 1e3, 4),
             "max_abs_vs_fp32_path": max_abs,
-            "gemm_arithmetic": "fp32 MFMA products: at most 64 positions the few-token kernels do not "
-                               "split (EBH_DTYPE_F32_BF16X6)" if few else
-                               "fp32 operands split into three bf16 parts, six bf16 MFMA products "
-                               "per fp32 product, fp32 accumulate (EBH_DTYPE_F32_BF16X6)",
+            "gemm_arithmetic": gemm_arithmetic("fp32-bf16x6", B * S),
             "roofline": {"kernel": profile_kernel, "bound": bound, "achieved": round(achieved, 3),
-                         "peak": round(peak, 1), "unit": "TFLOP/s" if bound == "mfma" else "GB/s",
+                         "peak": peak, "unit": "TFLOP/s" if bound == "mfma" else "GB/s",
                          "frac": round(achieved / peak, 4), "avg_launch_ms": round(avg, 5),
                          "launches": launches}}
 
 
 LEG_DTYPE_NOTE = {
-    "fp32": "f32 (GEMM operands, accumulation, residual stream, LayerNorm, softmax)",
+    "fp32": "f32 (GEMM operands, held as fp16 pairs above 64 positions; accumulation, residual stream, "
+            "LayerNorm, softmax)",
     "bf16": "bf16 GEMM and attention operands with fp32 accumulation; bf16 residual stream "
             "(the skip connection carries bf16-rounded values); LayerNorm statistics, softmax "
             "and pooling in fp32",
@@ -356,20 +374,25 @@ def config_leg(eb, torch, name: str, steps: int, warmup: int, graph_replay: bool
             continue
         avg = prof_ms / launches
         work, bound, wunit = kernel_work(cfg, lengths, B, fam, fused, dtype)
+        if fam == "gemm_ffn_down" and "gemm_ffn_up" not in families:   # one launch for both
+            work += kernel_work(cfg, lengths, B, "gemm_ffn_up", fused, dtype)[0]
         if bound == "mfma":
-            achieved, peak, punit = work / (avg * 1e-3) / 1e12, PEAK_TFLOPS[dtype], "TFLOP/s"
+            achieved, peak, punit = work / (avg * 1e-3) / 1e12, matrix_peak(dtype, B * S), "TFLOP/s"
         else:
             achieved, peak, punit = work / (avg * 1e-3) / 1e9, HBM_PEAK_GBS, "GB/s"
         families[fam] = {"bound": bound, "achieved": round(achieved, 3), "peak": peak, "unit": punit,
                          "frac": round(achieved / peak, 4), "avg_launch_ms": round(avg, 5),
                          "launches": launches, "per_forward": launches // steps,
                          "traffic": measured_traffic(name, fam, dtype)}
+    if "gemm_ffn_up" not in families:
+        families["gemm_ffn_down"]["covers"] = "gemm_ffn_up, GELU and gemm_ffn_down in one launch"
     model.close()
     ms = 1e3 * wall / steps
     top = max(families, key=lambda f: families[f]["avg_launch_ms"] * families[f]["per_forward"])
     return {"value": round(B * steps / wall, 2), "unit": "sentences/s", "steps": steps, "warmup": warmup,
             "ms_per_step": round(ms, 4), "p50_batch_latency_ms": round(float(np.median(times)) * 1e3, 4),
             "dtype": LEG_DTYPE_NOTE[dtype],
+            "gemm_arithmetic": gemm_arithmetic(dtype, B * S),
             "workload": f"{name}: {cfg.num_hidden_layers}L H{cfg.hidden_size} I{cfg.intermediate_size} "
                         f"heads{cfg.num_attention_heads} batch {B} x seq {S}, lengths "
                         f"{spec.len_lo}-{spec.len_hi}",
@@ -462,11 +485,16 @@ def main():
     # for the roofline.
     wall, times = timed(args.steps)
     model.synchronize()
-    model.profile_enable(args.profile_kernel)
-    timed(args.steps)
-    model.synchronize()
-    launches, prof_ms = model.profile_read()
-    model.profile_enable("none")
+    launches, prof_ms, covers = 0, 0.0, ""
+    for fam in dict.fromkeys((args.profile_kernel, "gemm_ffn_down")):
+        model.profile_enable(fam)
+        timed(args.steps)
+        model.synchronize()
+        launches, prof_ms = model.profile_read()
+        model.profile_enable("none")
+        if launches or fam != "gemm_ffn_up":
+            break
+        covers = " (FFN up, GELU and FFN down in one launch)"
 
     times = np.array(times)
     ms_per_step = 1e3 * wall / args.steps
@@ -475,8 +503,10 @@ def main():
     avg_kernel_ms = prof_ms / max(launches, 1)
     fused = few_fused(cfg, B, S, dtype)
     work, bound, wunit = kernel_work(cfg, lengths, B, args.profile_kernel, fused, dtype)
+    if covers:
+        work += kernel_work(cfg, lengths, B, "gemm_ffn_down", fused, dtype)[0]
     if bound == "mfma":
-        achieved, peak, punit = work / (avg_kernel_ms * 1e-3) / 1e12, PEAK_TFLOPS[dtype], "TFLOP/s"
+        achieved, peak, punit = work / (avg_kernel_ms * 1e-3) / 1e12, matrix_peak(dtype, B * S), "TFLOP/s"
     else:
         achieved, peak, punit = work / (avg_kernel_ms * 1e-3) / 1e9, HBM_PEAK_GBS, "GB/s"
     fwd_flops = forward_flops(cfg, lengths)
@@ -495,6 +525,7 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": {"fp32": "f32", "bf16": "bf16", "fp32-bf16x6": "f32 (bf16x6 GEMM products)"}[dtype],
+        "gemm_arithmetic": gemm_arithmetic(dtype, B * S),
         "data": "synthetic (seeded ids, random-init N(0,0.02) weights; no checkpoint offline)",
         "config": {"workload": f"{args.config}: {cfg.num_hidden_layers}L H{cfg.hidden_size} "
                                f"I{cfg.intermediate_size} heads{cfg.num_attention_heads} "
@@ -504,7 +535,7 @@ def main():
         "forward_tflops": round(fwd_flops / (ms_per_step * 1e-3) / 1e12, 2),
         "graph_replay": not args.no_graph_replay,
         "roofline": {"kernel": args.profile_kernel + (" (with the output projection)"
-                                                      if fused and args.profile_kernel == "attention" else ""),
+                                                      if fused and args.profile_kernel == "attention" else covers),
                      "bound": bound, "achieved": round(achieved, 3),
                      "peak": peak, "unit": punit, "frac": round(achieved / peak, 4),
                      "traffic": measured_traffic(args.config, args.profile_kernel, dtype),
@@ -547,9 +578,11 @@ def main():
         model.profile_enable("none")
         if n:
             fwork, fbound, _ = kernel_work(cfg, lengths, B, fam, fused, dtype)
+            if fam == "gemm_ffn_down" and "gemm_ffn_up" not in fams:
+                fwork += kernel_work(cfg, lengths, B, "gemm_ffn_up", fused, dtype)[0]
             favg = fms / n
             if fbound == "mfma":
-                fa, fp, fu = fwork / (favg * 1e-3) / 1e12, PEAK_TFLOPS[dtype], "TFLOP/s"
+                fa, fp, fu = fwork / (favg * 1e-3) / 1e12, matrix_peak(dtype, B * S), "TFLOP/s"
             else:
                 fa, fp, fu = fwork / (favg * 1e-3) / 1e9, HBM_PEAK_GBS, "GB/s"
             fams[fam] = {"bound": fbound, "achieved": round(fa, 3), "peak": fp, "unit": fu,

@@ -269,19 +269,31 @@ void drop_graphs(ebh_model* m) {
     m->graphs.clear();
 }
 
+// Partial products that Y holds for a forward of T positions.  Few-token fp32
+// forwards split the bias-free projections over K, one partial per split;
+// few-token attention with the output projection writes one per head.
+int y_parts_for(const ebh_model* m, int64_t T) {
+    const ebh_config& c = m->cfg;
+    if (m->dtype == EBH_DTYPE_BF16) return 1;
+    const int H = c.hidden_size, I = c.intermediate_size;
+    const int parts = std::max(ebh::gemm_f32_splits((int)T, H, H), ebh::gemm_f32_splits((int)T, H, I));
+    return ebh::few_attn_fits((int)T, H, c.num_attention_heads) ? std::max(parts, c.num_attention_heads) : parts;
+}
+
 // Place a workspace for tcap tokens and bcap sequences at `base` (nullptr:
-// only count); returns the bytes it spans.  Few-token fp32 forwards split the
-// bias-free projections over K; Y then holds one partial product per split.
-size_t layout_workspace(const ebh_model* m, int64_t tcap, int bcap, char* base, Workspace& w) {
+// only count); returns the bytes it spans.  any_fewer: the workspace also
+// serves forwards of fewer positions, which may split further than one of
+// tcap; Y is then large enough that each of them splits as it would in a
+// workspace of its own size, and gives the same bits whatever ran before it.
+size_t layout_workspace(const ebh_model* m, int64_t tcap, int bcap, char* base, Workspace& w, bool any_fewer) {
     const ebh_config& c = m->cfg;
     const size_t H = c.hidden_size, I = c.intermediate_size;
     const bool b16 = m->dtype == EBH_DTYPE_BF16;
-    int yparts = b16 ? 1
-                     : std::max(ebh::gemm_f32_splits((int)tcap, (int)H, (int)H),
-                                ebh::gemm_f32_splits((int)tcap, (int)H, (int)I));
-    // Few-token attention + output projection: one partial per head.
-    if (!b16 && ebh::few_attn_fits((int)tcap, (int)H, c.num_attention_heads))
-        yparts = std::max(yparts, c.num_attention_heads);
+    int64_t yparts = y_parts_for(m, tcap);
+    // Split counts fall at whole 64-row tiles; partials may run on into QKV's
+    // three rows a position (enqueue_pair_layers).
+    for (int64_t T = 64; any_fewer && T < tcap; T += 64)
+        yparts = std::max(yparts, ((int64_t)(y_parts_for(m, T) + 3) * T + tcap - 1) / tcap - 3);
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off += align_up(std::max<size_t>(bytes, 1)); return o; };
     const size_t oErr = take(4), oX = take(b16 ? 0 : tcap * H * 4), oX16 = take(b16 ? tcap * H * 2 : 0),
@@ -294,7 +306,7 @@ size_t layout_workspace(const ebh_model* m, int64_t tcap, int bcap, char* base, 
     w.base = base;
     w.tok_cap = tcap;
     w.b_cap = bcap;
-    w.y_parts = yparts;
+    w.y_parts = (int)yparts;
     w.err = (int*)(base + oErr);
     w.X = b16 ? nullptr : (float*)(base + oX);
     w.X16 = b16 ? (uint16_t*)(base + oX16) : nullptr;
@@ -322,7 +334,7 @@ int ensure_workspace(ebh_model* m, int B, int S) {
     const int64_t tcap = std::max<int64_t>(T, w.tok_cap);
     const int bcap = std::max(B, w.b_cap);
     Workspace nw;
-    const size_t bytes = layout_workspace(m, tcap, bcap, nullptr, nw);
+    const size_t bytes = layout_workspace(m, tcap, bcap, nullptr, nw, true);
     // Work from the previous call may still use the old block, and recorded
     // forwards hold its addresses.  A raised id-range flag is carried over to
     // the new block (it stays raised until ebh_synchronize reads it).
@@ -334,7 +346,7 @@ int ensure_workspace(ebh_model* m, int B, int S) {
     w = Workspace{};
     void* base = nullptr;
     HIP_TRY(hipMalloc(&base, bytes));
-    layout_workspace(m, tcap, bcap, static_cast<char*>(base), w);
+    layout_workspace(m, tcap, bcap, static_cast<char*>(base), w, true);
     HIP_TRY(hipMemcpy(w.err, &old_err, 4, hipMemcpyHostToDevice));
     // The model's stream does not wait for the null stream: the flag must be
     // written before the first forward on this workspace can set it.
@@ -402,8 +414,10 @@ int enqueue_pair_layers(ebh_model* m, Workspace& w, int B, int S, int normalize,
     const int T = tokens >= 0 && tokens < (int64_t)B * S ? (int)std::max<int64_t>(tokens, 1) : B * S;
     uint32_t* const xp = reinterpret_cast<uint32_t*>(w.CTX);
     // Split partials lie T * H floats apart from Y on, into QKV's buffer behind
-    // it (3 rows' worth a token), which nobody reads by then.
-    const int max_splits = (int)std::min<int64_t>(8, ((int64_t)w.y_parts + 3) * w.tok_cap / T_pad);
+    // it (3 rows' worth a token), which nobody reads by then.  The limit goes
+    // by T_pad, not by the workspace (whose layout has the room).
+    const int max_splits = (int)std::min<int64_t>({8, y_parts_for(m, T_pad) + 3,
+                                                   ((int64_t)w.y_parts + 3) * w.tok_cap / T_pad});
     auto gemm = [&](int kind, const void* A, const uint32_t* W, const float* bias, void* C, int N, int K, int epi,
                     bool out_pair, float acc_scale, float out_scale, const ebh::Gemm16Plan& plan) -> int {
         ebh::Gemm16Args a{};
@@ -1386,7 +1400,7 @@ int ebh_encode_device_noalloc(ebh_model* m, const int32_t* ids, const int32_t* m
     if (!ids || !mask || !out) return fail(EBH_ERR_INVALID_ARG, "null buffer");
     Workspace w;
     const int64_t T = (int64_t)B * S;
-    const size_t need = layout_workspace(m, T, B, nullptr, w);
+    const size_t need = layout_workspace(m, T, B, nullptr, w, false);
     if (need > (size_t)EBH_NOALLOC_SCRATCH_BYTES)
         return fail(EBH_ERR_RANGE,
                     "batch %d x %d needs %zu bytes of workspace, more than the %zu bytes of the static scratch "
@@ -1401,7 +1415,7 @@ int ebh_encode_device_noalloc(ebh_model* m, const int32_t* ids, const int32_t* m
     if (S == 0) {
         HIP_TRY(ebh::launch_zero_words(out, (int64_t)B * m->cfg.hidden_size, s));
     } else {
-        layout_workspace(m, T, B, base, w);
+        layout_workspace(m, T, B, base, w, false);
         w.err = m->noalloc_err;   // this model's flag, not the shared array's
         if ((rc = enqueue_kernels(m, w, ids, mask, B, S, normalize ? 1 : 0, out, s, nullptr, -1, false)))
             return rc;

@@ -488,17 +488,18 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 __device__ __forceinline__ void split_f16x2(float a, float b, uint32_t& h, uint32_t& l) {
     typedef _Float16 v2h __attribute__((ext_vector_type(2)));
     typedef float v2f __attribute__((ext_vector_type(2)));
-    h = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{a, b}), v2h));
-    // a - (float)h, exact, as one instruction that takes its half of h as it is
-    // (the compiler makes a conversion and a subtraction of it: six VALU
-    // instructions a pair of values instead of four, on kernels whose epilogues
-    // and softmax are VALU work; forwards 1-2% faster).  The conversion above
-    // reads a and b first, so whatever wrote them (an exp2, a multiply) is at
-    // least one instruction back.
-    float ra, rb;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(ra) : "v"(h), "v"(a));
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(rb) : "v"(h), "v"(b));
-    const v2h ll = __builtin_convertvector((v2f{ra, rb}), v2h);
+    const v2h hh = __builtin_convertvector((v2f{a, b}), v2h);
+    // a - (float)h, exact, as one v_fma_mix_f32 that takes its half of h as it
+    // is: four VALU instructions a pair of values instead of six, on kernels
+    // whose epilogues and softmax are VALU work (forwards 1-2% faster).  The
+    // factor is kept from the compiler, which makes a conversion and a
+    // subtraction of a known -1; the instruction itself is the compiler's, so
+    // that it places the waits around it.
+    float minus1 = -1.f;
+    asm("" : "+s"(minus1));
+    const v2h ll = __builtin_convertvector((v2f{__builtin_fmaf((float)hh[0], minus1, a),
+                                                __builtin_fmaf((float)hh[1], minus1, b)}), v2h);
+    h = __builtin_bit_cast(uint32_t, hh);
     l = __builtin_bit_cast(uint32_t, ll);
 }
 

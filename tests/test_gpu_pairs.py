@@ -260,3 +260,27 @@ def test_models_at_the_ends_of_the_range(env, weights_for, how):
     want = oracle.OracleModel(cfg, w).encode_unpadded(ids * mask, mask, normalize=True)
     assert np.isfinite(got).all()
     assert np.abs(got - want).max() <= 1e-5
+
+
+@pytest.mark.parametrize("B,S,after", [(3, 22, (6, 60)), (5, 128, (20, 67)), (40, 50, (43, 64)), (63, 128, (65, 128))])
+def test_vectors_do_not_depend_on_earlier_batches(env, weights_for, B, S, after):
+    """A batch gives the same bits in a fresh model and in one whose workspace a
+    larger batch has grown (a product's split count goes by the batch alone)."""
+    torch, eb, N, L = env
+    cfg = eb.MINILM_L6
+    w = weights_for(cfg)
+    rng = np.random.default_rng(7)
+
+    def batch(b, s):
+        return rng.integers(10, cfg.vocab_size, (b, s)).astype(np.uint32), np.ones((b, s), np.uint32)
+
+    ids, mask = batch(B, S)
+    fresh, grown = eb.Model.from_weights(w, cfg, "fp32"), eb.Model.from_weights(w, cfg, "fp32")
+    try:
+        want = fresh.encode_ids(ids, mask)
+        grown.encode_ids(*batch(*after))
+        got = grown.encode_ids(ids, mask)
+    finally:
+        fresh.close()
+        grown.close()
+    assert np.array_equal(got, want)

@@ -51,6 +51,10 @@ enum Out16 : int { OUT_F32 = 0, OUT_PAIR = 1, OUT_BF16 = 2 };
 // of a pair chunk, stored straight from the accumulators, four lanes to a
 // 128-byte line.  The epilogue needs no LDS pass and no barrier, and the next
 // k-tile's loads are in flight ahead of its stores.
+// fp32 and pair outputs are stored through the caches, whose last level hands
+// them to the next kernel (non-temporal: 256 x 128 tokens of MiniLM 2.71 ->
+// 3.25 ms, 99 x 250 ragged 1.52 -> 1.65 ms); bf16 outputs non-temporal (through
+// the caches 64 x 128 289 -> 296 us, 1024 x 128 of BERT-base 24.45 -> 25.0 ms).
 //
 // What bounds it: the matrix cores (a 256 x 256 k-tile is 64 KB of loads for
 // 3,072 cycles of MFMAs per SIMD).  A k-tile's fragments are read a step (SB

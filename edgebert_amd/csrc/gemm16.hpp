@@ -42,8 +42,12 @@ enum Out16 : int { OUT_F32 = 0, OUT_PAIR = 1, OUT_BF16 = 2 };
 // chunks XOR-swizzled, by direct-to-LDS buffer loads whose descriptors end at
 // the last real row (rows past it read as zeros).
 //
-// Chunks 2q and 2q + 1 of a row are lane group q's operands: h and l of
-// k = 8q .. 8q + 7 (pairs), or two 8-deep runs of k (bf16).  The MFMAs take W
+// Lane group q's operands are chunks 2q and 2q + 1 of a row (pairs: h and l of
+// k = 8q .. 8q + 7), or q and q + 4 (bf16: two 32-deep slices of k, in order).
+// bf16 sums start at the bias and run over the slices, as the ring kernel's
+// (gemm.hip) do, so every tile there is gives a row the same bits and a bf16
+// vector does not depend on the batch it is in.  Pairs add the bias last: their
+// sums hold a scale of their own.  The MFMAs take W
 // as their first operand, so lane (r, q) of a 16 x 16 block holds C row r and
 // the block's W rows 4q .. 4q + 3.  W rows are permuted on their way into LDS
 // (within each 32, LDS row 16 jj + 4q + e holds column 8q + 4 jj + e), so a lane
@@ -181,7 +185,8 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
     };
 
     const int r16 = lane & 15, q16 = lane >> 4;
-    const uint32_t frag = r16 * 128 + 16 * ((2 * q16) ^ chunk_swizzle16<8>(r16));
+    constexpr uint32_t FX = PAIR ? 16 : 64;       // from a lane's first chunk to its second
+    const uint32_t frag = r16 * 128 + 16 * ((PAIR ? 2 * q16 : q16) ^ chunk_swizzle16<8>(r16));
     const uint32_t a_off = wm * WM * 128 + frag, w_off = wn * WN * 128 + frag;
     g16_v4f acc[FM][FN];
     g16_v4f af[2][SB][2], wf[2][FN][2];
@@ -226,14 +231,14 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
 #pragma unroll
             for (int i = 0; i < SB; ++i) {
                 af[s & 1][i][0] = *reinterpret_cast<const g16_v4f*>(sa + a_off + (s * SB + i) * 16 * 128);
-                af[s & 1][i][1] = *reinterpret_cast<const g16_v4f*>(sa + (a_off ^ 16) + (s * SB + i) * 16 * 128);
+                af[s & 1][i][1] = *reinterpret_cast<const g16_v4f*>(sa + (a_off ^ FX) + (s * SB + i) * 16 * 128);
             }
         };
         rd_a(0);
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
             wf[P][j][0] = *reinterpret_cast<const g16_v4f*>(sw + w_off + j * 16 * 128);
-            wf[P][j][1] = *reinterpret_cast<const g16_v4f*>(sw + (w_off ^ 16) + j * 16 * 128);
+            wf[P][j][1] = *reinterpret_cast<const g16_v4f*>(sw + (w_off ^ FX) + j * 16 * 128);
         }
         if (!first) mfma_step(NS - 1, 1, P ^ 1);   // the previous k-tile's last step
 #pragma unroll
@@ -246,6 +251,8 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
         ++it;
     };
 
+    // This wave's bias row segment of local tile t.
+    auto bias_of = [&](int t) __attribute__((always_inline)) { return smem + B_OFF + ((t & 1) * NW + wave) * BIAS_BYTES; };
     auto epilogue = [&](int t) __attribute__((always_inline)) {
         const int u = u0 + t * ustep, split = u / ntiles, tile = u - split * ntiles;
         const int mt = tile / ntn, wrow = mt * BM + wm * WM, n0 = (tile - mt * ntn) * BN;
@@ -255,13 +262,13 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
         int el = lane;
         asm volatile("" : "+v"(el));
         const int er = el & 15, eq = el >> 4;
-        const char* bs = smem + B_OFF + ((t & 1) * NW + wave) * BIAS_BYTES + 32 * eq;
+        const char* bs = bias_of(t) + 32 * eq;
         const float sc = p.acc_scale, so = p.out_scale;
         g16_v4f bb0[FN / 2], bb1[FN / 2]; uint32_t vo[FN / 2];
 #pragma unroll
         for (int jp = 0; jp < FN / 2; ++jp) {
             bb0[jp] = bb1[jp] = g16_v4f{0, 0, 0, 0};
-            if (HAS_BIAS) {
+            if (PAIR && HAS_BIAS) {
                 bb0[jp] = *reinterpret_cast<const g16_v4f*>(bs + jp * 128);
                 bb1[jp] = *reinterpret_cast<const g16_v4f*>(bs + jp * 128 + 16);
             }
@@ -281,8 +288,8 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
                         v[e] = HAS_BIAS ? fmaf(acc[i][2 * jp][e], sc, b0[e]) : acc[i][2 * jp][e] * sc;
                         v[4 + e] = HAS_BIAS ? fmaf(acc[i][2 * jp + 1][e], sc, b1[e]) : acc[i][2 * jp + 1][e] * sc;
                     } else {
-                        v[e] = acc[i][2 * jp][e] + b0[e];
-                        v[4 + e] = acc[i][2 * jp + 1][e] + b1[e];
+                        v[e] = acc[i][2 * jp][e];
+                        v[4 + e] = acc[i][2 * jp + 1][e];
                     }
                     if constexpr (EPI == EPI_BIAS_GELU) {
                         v[e] = gelu_tanh_fast(v[e]);
@@ -339,6 +346,14 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
 #pragma unroll
             for (int j = 0; j < FN; ++j) acc[i][j] = g16_v4f{0.0f, 0.0f, 0.0f, 0.0f};
         enter();
+        if constexpr (!PAIR && HAS_BIAS) {         // it came with the tile's first W
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                const g16_v4f b = *reinterpret_cast<const g16_v4f*>(bias_of(t) + 32 * q16 + (j >> 1) * 128 + (j & 1) * 16);
+#pragma unroll
+                for (int i = 0; i < FM; ++i) acc[i][j] = b;
+            }
+        }
         run_ktile(set0{}, true);
         enter();
         run_ktile(set1{}, false);

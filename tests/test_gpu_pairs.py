@@ -186,6 +186,30 @@ def test_gemm_bf16_tiles(env, M, Nn, K, epi):
     assert (C[M:] == 7).all()
 
 
+# M: rows of the one call that the ring kernel takes; fewer rows take the smaller
+# tiles in turn (64x64, 64x128, 128x96, 128x128, 256x128, 256x192)
+@pytest.mark.parametrize("M,Nn,K", [(20481, 2304, 768), (20481, 768, 3072), (20481, 3072, 768), (33000, 192, 128),
+                                    (20481, 1544, 384)])
+@pytest.mark.parametrize("epi", [EPI_BIAS, EPI_GELU, EPI_NONE])
+def test_bf16_rows_do_not_depend_on_the_batch(env, M, Nn, K, epi):
+    torch, eb, N, L = env
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator(device="cuda").manual_seed(Nn + K)
+    A = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    W = (0.04 * torch.randn(Nn, K, device="cuda", generator=g)).bfloat16()
+    b = torch.randn(Nn, device="cuda", generator=g)
+
+    def product(m):
+        C = torch.empty(m, Nn, device="cuda", dtype=torch.bfloat16)
+        N.check(L.ebh_op_gemm_bf16(vp(A), K, vp(W), K, vp(b) if epi != EPI_NONE else None, vp(C), Nn, N.EBH_DTYPE_BF16, m,
+                                   Nn, K, epi, s))
+        return C.view(torch.int16)
+
+    want = product(M)
+    for m in (1, 65, 1300, 2050, 4353, 8191, 12000):
+        assert torch.equal(product(m), want[:m]), m
+
+
 @pytest.mark.parametrize("H,nh", [(384, 12), (768, 12), (64, 1)])
 @pytest.mark.parametrize("lens", [[1], [31, 32, 33, 0, 64, 65], [127, 128, 129, 7], [192, 193, 512, 300]])
 def test_attention_pair(env, H, nh, lens):

@@ -420,13 +420,201 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 }
 
 // ---------------------------------------------------------------------------
-// Attention that streams K and V through LDS, for any length.
-//  * PAIR: the fp32 forward above 64 tokens.  Q, K, V and the context in the
-//    pair format (gemm16.hpp; a head's row is 4 HD bytes, as in fp32), every
-//    product from three v_mfma_f32_32x32x16_f16 with fp32 sums.
-//  * otherwise bf16 models' sequences of more than 128 tokens (the kernel above
-//    takes the shorter ones): Q, K, V, the context and the probabilities bf16,
-//    scores, softmax and sums fp32.
+// bf16 attention of sequences of more than 128 tokens (the kernel above takes
+// the shorter ones): Q, K, V, the context and the probabilities bf16, scores,
+// softmax and sums fp32.
+//
+// Work split: workgroup = (head, 128-query block, sequence), 4 waves of 32
+// queries.  Softmax is online over 128-key chunks.  K and V go straight into
+// LDS (buffer loads; rows past the sequence read as zeros), K in two stages, so
+// that chunk c + 1's is on its way while chunk c is computed, V in one: it lands
+// while the scores and the softmax run, behind a barrier of its own.  That is
+// 48 KB with heads of 64, three workgroups per CU.  A lane's query goes straight
+// to registers; layouts, swizzles and the transposing V read are those of the
+// kernel above.
+//
+// What bounds it: the softmax's VALU work, of which the scale, the subtraction
+// of the maximum and the factor log2 e are an operation each: folded into one
+// FMA, on 64-key chunks, they would be 3 us less (39.9) but other bits.  40
+// sequences of 200-512, heads of 64: 66.2 -> 43.2 us (heads of 32: 40.4 -> 31.7)
+// against the same sums with both chunks staged through registers and V
+// transposed on its way into LDS.
+// ---------------------------------------------------------------------------
+template <int HD>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void attention_bf16_long_kernel(
+    const uint16_t* __restrict__ qkv, const int* __restrict__ cu_seqlens, uint16_t* __restrict__ ctx, int H,
+    float scale, const int* __restrict__ order) {
+    constexpr int KC = 128, NB = KC / 32;   // keys per chunk, 32-key blocks
+    constexpr int RB = 2 * HD;              // bytes per K / V row
+    constexpr int CPR = RB / 16;            // 16-byte chunks per K / V row
+    constexpr int NLD = KC * CPR / 256;     // 16-byte loads per thread for K (and for V)
+    constexpr int NJ = HD / 32, NS = HD / 16;
+    __shared__ __attribute__((aligned(16))) char Ks[2][KC * RB];
+    __shared__ __attribute__((aligned(16))) char Vs[KC * RB];
+
+    const int head = blockIdx.x, qb = blockIdx.y, b = order ? order[blockIdx.z] : (int)blockIdx.z;
+    const int start = cu_seqlens[b];
+    const int len = cu_seqlens[b + 1] - start;
+    if (qb * 128 >= len) return;  // uniform over the workgroup
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, half = lane >> 5;
+    const int64_t ld = 3 * (int64_t)H;
+    const uint32_t ldb = 3 * (uint32_t)H * 2;
+
+    uint32_t kvo[NLD], vvo[NLD];
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+        const int P = i * 256 + tid, r = P / CPR, pc = P % CPR;
+        kvo[i] = r * ldb + (H + head * HD) * 2 + 16 * (pc ^ chunk_swizzle16<CPR>(r));
+        vvo[i] = r * ldb + (2 * H + head * HD) * 2 + 16 * (pc ^ v_swizzle<HD>(r));
+    }
+    auto rows_of = [&](int c) __attribute__((always_inline)) {
+        return make_rsrc(qkv + (start + c * KC) * ld, (uint32_t)min(len - c * KC, KC) * ldb);
+    };
+    auto issue_k = [&](int c) __attribute__((always_inline)) {
+        const g16_v4i rsrc = rows_of(c);
+        const uint32_t ks = (uint32_t)(uintptr_t)&Ks[c & 1][0] + wave * 1024;
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) load_lds16_buf(rsrc, kvo[i], 0, ks + i * 4096);
+    };
+    auto issue_v = [&](int c) __attribute__((always_inline)) {
+        const g16_v4i rsrc = rows_of(c);
+        const uint32_t vs = (uint32_t)(uintptr_t)&Vs[0] + wave * 1024;
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) load_lds16_buf(rsrc, vvo[i], 0, vs + i * 4096);
+    };
+
+    // This lane's query as the B operand: dims 16 s + 8 half .. +7.
+    const int q0 = qb * 128 + wave * 32;
+    v8s_t qf[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+        qf[s] = *reinterpret_cast<const v8s_t*>(qkv + (start + min(q0 + l32, len - 1)) * ld + head * HD + 16 * s + 8 * half);
+    issue_k(0);
+    issue_v(0);
+
+    v16f o[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[j][r] = 0.0f;
+    float m_run = -INFINITY, l_run = 0.0f;
+    const bool active = q0 < len;   // a wave past the sequence's queries only helps load
+    const int g16 = lane >> 4, i16 = lane & 15;
+    const int vrow = i16 >> 2, vdim = 16 * (g16 & 1) + 4 * (i16 & 3);
+    const int nchunks = (len + KC - 1) / KC;
+    for (int c = 0; c < nchunks; ++c) {
+        if (c == 0) wait_vmcnt(NLD);   // K is here, V(0) may be in flight
+        else wait_vmcnt(0);
+        lds_barrier();                 // everyone's K, and everyone is done with chunk c - 1
+        if (c > 0) issue_v(c);
+        if (c + 1 < nchunks) issue_k(c + 1);
+        const int lim = len - c * KC, nkb = active ? min(NB, (lim + 31) / 32) : 0;
+        const char* K = Ks[c & 1];
+        v16f sc[NB];
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sc[kb][r] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int kb = 0; kb < NB; ++kb)
+                if (kb < nkb) {
+                    const int kr = kb * 32 + l32;
+                    const v8s_t kf = *reinterpret_cast<const v8s_t*>(K + kr * RB + 16 * ((2 * s + half) ^ chunk_swizzle16<CPR>(kr)));
+                    sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf_t, kf),
+                                                                      __builtin_bit_cast(v8bf_t, qf[s]), sc[kb], 0, 0, 0);
+                }
+        // The scale after q.k^T (src/lib.rs:714), rounded by itself, and the
+        // key-padding mask (src/lib.rs:887-891).
+        float cmax = -INFINITY;
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb)
+            if (kb < nkb) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sc[kb][r] *= scale;
+                if ((kb + 1) * 32 > lim) {             // the block that straddles the sequence end
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        if (kb * 32 + 8 * (r >> 2) + (r & 3) >= lim - 4 * half) sc[kb][r] = -INFINITY;
+                }
+#pragma unroll
+                for (int r = 0; r < 16; ++r) cmax = fmaxf(cmax, sc[kb][r]);
+            }
+        cmax = fmaxf(cmax, __shfl_xor(cmax, 32));
+        const float m_new = fmaxf(m_run, cmax);
+        const float alpha = fast_exp(m_run - m_new);   // 0 on the first chunk
+        float psum = 0.0f;
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb)
+            if (kb < nkb) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float pr = fast_exp(sc[kb][r] - m_new);
+                    sc[kb][r] = pr;
+                    psum += pr;
+                }
+            }
+        l_run = l_run * alpha + psum;
+        m_run = m_new;
+        if (c > 0) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[j][r] *= alpha;
+        }
+        if (c + 1 < nchunks) wait_vmcnt(NLD);          // V is here, K(c + 1) may be in flight
+        else wait_vmcnt(0);
+        lds_barrier();                                 // and everyone else's
+        // context^T += V^T . P^T, 16 keys a step, as in the kernel above.
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb)
+            if (kb < nkb) {
+#pragma unroll
+                for (int mm = 0; mm < 2; ++mm) {
+                    const float* pf = reinterpret_cast<const float*>(&sc[kb]) + 8 * mm;
+                    const v8s_t pa = __builtin_bit_cast(
+                        v8s_t, make_uint4(pack_bf16x2(pf[0], pf[1]), pack_bf16x2(pf[2], pf[3]),
+                                          pack_bf16x2(pf[4], pf[5]), pack_bf16x2(pf[6], pf[7])));
+                    const int ra = kb * 32 + 16 * mm + 4 * (g16 >> 1) + vrow, rb = ra + 8;
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) {
+                        const int d = j * 32 + vdim;
+                        auto rd = [&](int r) __attribute__((always_inline)) {
+                            return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                (__attribute__((address_space(3))) v4s_t*)(Vs + r * RB + 16 * ((d >> 3) ^ v_swizzle<HD>(r)) + 2 * (d & 7)));
+                        };
+                        const v4s_t va = rd(ra), vb = rd(rb);
+                        const v8s_t vf = {va[0], va[1], va[2], va[3], vb[0], vb[1], vb[2], vb[3]};
+                        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf_t, vf),
+                                                                        __builtin_bit_cast(v8bf_t, pa), o[j], 0, 0, 0);
+                    }
+                }
+            }
+    }
+
+    // Lane holds dims j*32 + 8*g + 4*half + 0..3 (g = r / 4) of query l32.
+    const float l_tot = l_run + __shfl_xor(l_run, 32);
+    const int q = q0 + l32;
+    if (q < len) {
+        const float inv = 1.0f / l_tot;
+        uint16_t* dst = ctx + (int64_t)(start + q) * H + head * HD + 4 * half;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *reinterpret_cast<uint2*>(dst + j * 32 + 8 * g) =
+                    make_uint2(pack_bf16x2(o[j][4 * g] * inv, o[j][4 * g + 1] * inv),
+                               pack_bf16x2(o[j][4 * g + 2] * inv, o[j][4 * g + 3] * inv));
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Attention on fp16 pairs, for any length: the fp32 forward above 64 tokens.
+// Q, K, V and the context are in the pair format (gemm16.hpp; a head's row is
+// 4 HD bytes, as in fp32), every product from three v_mfma_f32_32x32x16_f16
+// with fp32 sums.
 //
 // Work split: workgroup = (head, 128-query block, sequence), 4 waves of 32
 // queries; 64-key chunks of K and V in two LDS stages, chunk c + 1 on its way
@@ -434,40 +622,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // chunk c is computed.  A lane's query goes straight to registers.
 //
 // The layouts are those of the kernels above: S^T = K . Q^T, so a lane owns one
-// query's scores; the probabilities (pairs: scaled by 2^12 in the exponent, so
-// that l of small ones stays out of fp16's subnormals, and split in registers)
+// query's scores; the probabilities (scaled by 2^12 in the exponent, so that l
+// of small ones stays out of fp16's subnormals, and split in registers)
 // are the B operand of O^T = V^T . P^T, whose A operand comes from row-major V
 // through ds_read_b64_tr_b16.  K chunks are swizzled as GEMM rows are.  A
 // half-wave's transposing read takes the h (or l) chunks, every other 16 bytes,
-// of four rows (bf16: all chunks of 32 dims); V's swizzle moves rows that share
-// banks (r and r + 2 of 128-byte rows, all four of 256-byte ones) apart.
+// of four rows; V's swizzle moves rows that share banks (r and r + 2 of 128-byte
+// rows, all four of 256-byte ones) apart.
 //
 // What bounds it: HBM at c3 (201 MB a layer), the softmax's VALU work (the
 // split of P included, it outweighs the twelve MFMAs per 32 x 32 block) on long
 // sequences.  Unlike fp32 MFMAs, fp16 ones leave the VALU free meanwhile.
 // Against the fp32 kernel above, in the forward, per layer: 256 sequences of
 // 128 tokens 76 -> 47 us (4.3 TB/s), 16 of 256-512 53 -> 26 us, 32 of 8-128
-// 12.4 -> 8.3 us; heads of 64, 48 of 16-128 24.9 -> 15.2 us.  bf16 (heads of
-// 64, 40 sequences of 200-512): 72 -> 43 us against 128-key chunks staged
-// through registers with V transposed on its way.
+// 12.4 -> 8.3 us; heads of 64, 48 of 16-128 24.9 -> 15.2 us.
 // ---------------------------------------------------------------------------
 template <int HD>
 __device__ __forceinline__ int v_pair_swizzle(int r) {
     return HD == 32 ? ((r >> 1) & 1) : (r & 1) | ((r >> 1) & 1) << 3;
 }
 
-template <int HD, bool PAIR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 || !PAIR ? 4 : 2))) void attention_stream_kernel(
-    const void* __restrict__ qkv_, const int* __restrict__ cu_seqlens, void* __restrict__ ctx_, int H, float c2,
+template <int HD>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ? 4 : 2))) void attention_stream_kernel(
+    const uint32_t* __restrict__ qkv_, const int* __restrict__ cu_seqlens, uint32_t* __restrict__ ctx_, int H, float c2,
     float out_mul, const int* __restrict__ order) {
     constexpr int KC = 64, NB = KC / 32;    // keys per chunk, 32-key blocks
-    constexpr int ES = PAIR ? 4 : 2;        // bytes per element
+    constexpr int ES = 4;                   // bytes per element
     constexpr int RB = ES * HD;             // bytes per K / V row
     constexpr int CPR = RB / 16;            // 16-byte chunks per K / V row
-    const char* qkv = static_cast<const char*>(qkv_);
+    const char* qkv = reinterpret_cast<const char*>(qkv_);
     constexpr int NLD = KC * CPR / 256;     // 16-byte loads per thread for K (and for V)
     constexpr int NJ = HD / 32, NS = HD / 16;
-    constexpr float P_LOG2 = PAIR ? 12.0f : 0.0f;   // pairs: probabilities are held times 2^12
+    constexpr float P_LOG2 = 12.0f;         // probabilities are held times 2^12
     __shared__ __attribute__((aligned(16))) char Ks[2][KC * RB];
     __shared__ __attribute__((aligned(16))) char Vs[2][KC * RB];
 
@@ -478,14 +664,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ||
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
     const uint32_t ldb = 3 * (uint32_t)H * ES;
-    auto v_swz = [](int r) { return PAIR ? v_pair_swizzle<HD>(r) : v_swizzle<HD>(r); };
 
     uint32_t kvo[NLD], vvo[NLD];
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         const int P = i * 256 + tid, r = P / CPR, pc = P % CPR;
         kvo[i] = r * ldb + (H + head * HD) * ES + 16 * (pc ^ chunk_swizzle16<CPR>(r));
-        vvo[i] = r * ldb + (2 * H + head * HD) * ES + 16 * (pc ^ v_swz(r));
+        vvo[i] = r * ldb + (2 * H + head * HD) * ES + 16 * (pc ^ v_pair_swizzle<HD>(r));
     }
     auto issue = [&](int c) __attribute__((always_inline)) {
         const g16_v4i rsrc = make_rsrc(qkv + (int64_t)(start + c * KC) * ldb, (uint32_t)min(len - c * KC, KC) * ldb);
@@ -496,15 +681,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ||
         for (int i = 0; i < NLD; ++i) load_lds16_buf(rsrc, vvo[i], 0, vs + i * 4096);
     };
 
-    // One 32 x 32 x 16 product step: PAIR, of (h, l) operands; else of h alone.
+    // One 32 x 32 x 16 product step of (h, l) operands.
     auto mul = [](const v8h& ah, const v8h& al, const v8h& bh, const v8h& bl, v16f d) __attribute__((always_inline)) {
-        if constexpr (PAIR) {
-            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, d, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, d, 0, 0, 0);
-            return __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, d, 0, 0, 0);
-        } else {
-            return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf_t, ah), __builtin_bit_cast(v8bf_t, bh), d, 0, 0, 0);
-        }
+        d = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, d, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, d, 0, 0, 0);
     };
     // This lane's query: dims 16 s + 8 half .. +7 (h and l).
     const int q0 = qb * 128 + wave * 32;
@@ -514,7 +695,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ||
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             qh[s] = *reinterpret_cast<const v8h*>(qr + 16 * ES * s);
-            ql[s] = PAIR ? *reinterpret_cast<const v8h*>(qr + 16 * ES * s + 16) : qh[s];
+            ql[s] = *reinterpret_cast<const v8h*>(qr + 16 * ES * s + 16);
         }
     }
     issue(0);
@@ -546,9 +727,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ||
 #pragma unroll
             for (int kb = 0; kb < NB; ++kb)
                 if (kb < nkb) {
-                    const int kr = kb * 32 + l32, ch = ((PAIR ? 2 : 1) * (2 * s + half)) ^ chunk_swizzle16<CPR>(kr);
+                    const int kr = kb * 32 + l32, ch = (2 * (2 * s + half)) ^ chunk_swizzle16<CPR>(kr);
                     const v8h kh = *reinterpret_cast<const v8h*>(K + kr * RB + 16 * ch);
-                    const v8h kl = PAIR ? *reinterpret_cast<const v8h*>(K + kr * RB + 16 * (ch ^ 1)) : kh;
+                    const v8h kl = *reinterpret_cast<const v8h*>(K + kr * RB + 16 * (ch ^ 1));
                     sc[kb] = mul(kh, kl, qh[s], ql[s], sc[kb]);
                 }
         // Key-padding mask (src/lib.rs:887-891), only in the block that
@@ -566,8 +747,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ||
                 for (int r = 0; r < 16; ++r) cmax = fmaxf(cmax, sc[kb][r]);
             }
         cmax = fmaxf(cmax, __shfl_xor(cmax, 32));
-        // exp(scale (s - m)) as 2^(s c2 - m c2) (pairs: times 2^12); c2 holds
-        // the scale, log2 e and the operands' scales.
+        // exp(scale (s - m)) as 2^(s c2 - m c2), times 2^12; c2 holds the scale,
+        // log2 e and the operands' scales.
         const float m_new = fmaxf(m_run, cmax), mc = m_new * c2, off = P_LOG2 - mc;
         const float alpha = __builtin_amdgcn_exp2f(m_run * c2 - mc);   // 0 on the first chunk
         float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -600,26 +781,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ||
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const float p0 = sc[kb][8 * mm + 2 * e], p1 = sc[kb][8 * mm + 2 * e + 1];
-                        if constexpr (PAIR) split_f16x2(p0, p1, hw[e], lw[e]);
-                        else hw[e] = lw[e] = pack_bf16x2(p0, p1);
+                        split_f16x2(p0, p1, hw[e], lw[e]);
                     }
                     const v8h ph = __builtin_bit_cast(v8h, make_uint4(hw[0], hw[1], hw[2], hw[3]));
                     const v8h pl = __builtin_bit_cast(v8h, make_uint4(lw[0], lw[1], lw[2], lw[3]));
                     const int ra = kb * 32 + 16 * mm + 4 * (g16 >> 1) + vrow, rb = ra + 8;
 #pragma unroll
                     for (int j = 0; j < NJ; ++j) {
-                        const int d = j * 32 + vdim, ch = (PAIR ? 2 : 1) * (d >> 3), in = 2 * (d & 7);
+                        const int d = j * 32 + vdim, ch = 2 * (d >> 3), in = 2 * (d & 7);
                         auto rd = [&](int r, int part) __attribute__((always_inline)) {
                             return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                (__attribute__((address_space(3))) v4s_t*)(V + r * RB + 16 * ((ch + part) ^ v_swz(r)) + in));
+                                (__attribute__((address_space(3))) v4s_t*)(V + r * RB + 16 * ((ch + part) ^ v_pair_swizzle<HD>(r)) + in));
                         };
                         const v4s_t ha = rd(ra, 0), hb = rd(rb, 0);
                         const v8h vh = __builtin_bit_cast(v8h, (v8s_t){ha[0], ha[1], ha[2], ha[3], hb[0], hb[1], hb[2], hb[3]});
-                        v8h vl = vh;
-                        if constexpr (PAIR) {
-                            const v4s_t la = rd(ra, 1), lb = rd(rb, 1);
-                            vl = __builtin_bit_cast(v8h, (v8s_t){la[0], la[1], la[2], la[3], lb[0], lb[1], lb[2], lb[3]});
-                        }
+                        const v4s_t la = rd(ra, 1), lb = rd(rb, 1);
+                        const v8h vl = __builtin_bit_cast(v8h, (v8s_t){la[0], la[1], la[2], la[3], lb[0], lb[1], lb[2], lb[3]});
                         o[j] = mul(vh, vl, ph, pl, o[j]);
                     }
                 }
@@ -630,18 +807,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 32 ||
     const float l_tot = l_run + __shfl_xor(l_run, 32);
     const int q = q0 + l32;
     if (q < len) {
-        const float inv = out_mul / l_tot;   // pairs: ctx scale / qkv scale; the 2^12 cancels
-        char* dst = static_cast<char*>(ctx_) + ((int64_t)(start + q) * H + head * HD) * ES + 8 * half;
+        const float inv = out_mul / l_tot;   // ctx scale / qkv scale; the 2^12 cancels
+        char* dst = reinterpret_cast<char*>(ctx_) + ((int64_t)(start + q) * H + head * HD) * ES + 8 * half;
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                if constexpr (!PAIR) {
-                    *reinterpret_cast<uint2*>(dst + 64 * j + 16 * g) =
-                        make_uint2(pack_bf16x2(o[j][4 * g] * inv, o[j][4 * g + 1] * inv),
-                                   pack_bf16x2(o[j][4 * g + 2] * inv, o[j][4 * g + 3] * inv));
-                    continue;
-                }
                 uint2 h, l;
                 split_f16x2(o[j][4 * g] * inv, o[j][4 * g + 1] * inv, h.x, l.x);
                 split_f16x2(o[j][4 * g + 2] * inv, o[j][4 * g + 3] * inv, h.y, l.y);
@@ -658,9 +829,9 @@ hipError_t launch_attention_pair(const uint32_t* qkv, const int* cu_seqlens, int
     const dim3 grid(nh, (max_len + 127) / 128, B), block(256);
     const float c2 = scale * 1.4426950408889634f / (qkv_scale * qkv_scale), mul = ctx_scale / qkv_scale;
     if (head_dim == 32)
-        hipLaunchKernelGGL((attention_stream_kernel<32, true>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, mul, order);
+        hipLaunchKernelGGL((attention_stream_kernel<32>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, mul, order);
     else if (head_dim == 64)
-        hipLaunchKernelGGL((attention_stream_kernel<64, true>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, mul, order);
+        hipLaunchKernelGGL((attention_stream_kernel<64>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, mul, order);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();
@@ -683,11 +854,10 @@ hipError_t launch_attention_bf16(const uint16_t* qkv, const int* cu_seqlens, int
         return hipGetLastError();
     }
     const dim3 grid(nh, (max_len + 127) / 128, B), block(256);
-    const float c2 = scale * 1.4426950408889634f;
     if (head_dim == 32)
-        hipLaunchKernelGGL((attention_stream_kernel<32, false>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, 1.0f, order);
+        hipLaunchKernelGGL(attention_bf16_long_kernel<32>, grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order);
     else if (head_dim == 64)
-        hipLaunchKernelGGL((attention_stream_kernel<64, false>), grid, block, 0, s, qkv, cu_seqlens, ctx, H, c2, 1.0f, order);
+        hipLaunchKernelGGL(attention_bf16_long_kernel<64>, grid, block, 0, s, qkv, cu_seqlens, ctx, H, scale, order);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();

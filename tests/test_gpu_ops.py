@@ -5,6 +5,7 @@ masks with holes, ids out of range, concurrent callers, workspace growth,
 safetensors loading).  Device memory comes from torch; every call is
 enqueued on torch's current stream."""
 import ctypes
+import hashlib
 import json
 import os
 import threading
@@ -478,6 +479,27 @@ def test_attention_bf16(env, H, nh, lengths):
     # |ctx| <= max|v| ~ 4; probabilities carry 2^-9 relative error, the output one
     # more bf16 rounding.
     np.testing.assert_allclose(dctx.float().cpu().numpy(), want, rtol=2 ** -8, atol=1e-2)
+
+
+# sha256 (first 16 digits) of the context bits as staged 128-key chunks with the
+# scale, the maximum and each exponential rounded one by one give them: a
+# bf16 model's long-sequence vectors stay the bits they have been.  Chunk and
+# block edges, an empty sequence, both head sizes.
+@pytest.mark.parametrize("H,nh,lengths,digest", [
+    (768, 12, [129, 1, 512, 0, 300], "145ae66f4bbbc7a0"),
+    (64, 1, [160, 255, 256, 257, 384], "9db6902df4b2a47b"),
+    (384, 12, [200, 128, 131, 449], "3e840dd7f1a8ad92"),
+    (64, 2, [97, 140, 500], "e131512c8c6932fb"),
+])
+def test_attention_bf16_long_bits(env, H, nh, lengths, digest):
+    torch, eb, Nn, L = env
+    r = np.random.RandomState(H + nh + len(lengths))
+    qkv = dev(torch, (r.standard_normal((sum(lengths), 3 * H)) * 1.5).astype(np.float32)).bfloat16()
+    cu = dev(torch, np.array([0] + list(np.cumsum(lengths)), np.int32))
+    ctx = torch.zeros(sum(lengths), H, device="cuda", dtype=torch.bfloat16)
+    Nn.check(L.ebh_op_attention_bf16(vp(qkv), vp(cu), len(lengths), max(lengths), H, nh, vp(ctx), stream(torch)))
+    torch.cuda.synchronize()
+    assert hashlib.sha256(ctx.view(torch.int16).cpu().numpy().tobytes()).hexdigest()[:16] == digest
 
 
 def test_attention_empty_sequence_writes_nothing(env):

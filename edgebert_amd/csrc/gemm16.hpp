@@ -66,8 +66,14 @@ enum Out16 : int { OUT_F32 = 0, OUT_PAIR = 1, OUT_BF16 = 2 };
 // barrier, so that the pipes work while the barrier releases and the first
 // fragments arrive; two sets of W fragments make that possible, and k-tiles
 // come in pairs so that the sets have fixed registers.
+//
+// Bias row segments ride in with their tile's first W k-tile, up to nsw - 1
+// k-tiles before it is computed.  A tile has at least two k-tiles, so at a tile's
+// last k-tile that reaches (nsw - 2) / 2 tiles past the next one: a slot for
+// each of those, for the next tile and for the one whose epilogue comes.
+constexpr int gemm16_bias_slots(int nsw) { return 2 + (nsw - 2) / 2; }
 constexpr int gemm16_lds(int bm, int bn, int waves, int nsa, int nsw, bool bias) {
-    return (nsa * bm + nsw * bn) * 128 + (bias ? 2 * waves * 1024 : 0);
+    return (nsa * bm + nsw * bn) * 128 + (bias ? gemm16_bias_slots(nsw) * waves * 1024 : 0);
 }
 
 template <bool PAIR, int BM, int BN, int WAVES_M, int WAVES_N, int NSA, int NSW, int EPI, int OUT>
@@ -93,12 +99,13 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
     constexpr int CES = OUT == OUT_BF16 ? 2 : 4;
     constexpr int NSTO = FM * (FN / 2) * (OUT == OUT_BF16 ? 1 : 2);   // stores per lane and tile
     constexpr int BIAS_BYTES = 1024;              // one wave's 64 x 16-byte bias chunks
-    static_assert(gemm16_lds(BM, BN, WAVES_M * WAVES_N, NSA, NSW, HAS_BIAS) <= 160 * 1024, "LDS");
+    constexpr int NBIAS = gemm16_bias_slots(NSW);
+    static_assert(gemm16_lds(BM, BN, NW, NSA, NSW, HAS_BIAS) <= (NW == 8 ? 160 : 80) * 1024, "LDS");
 
     const int N = p.N;
     const int ntn = (N + BN - 1) / BN, ntiles = ((M + BM - 1) / BM) * ntn;
     const int S = p.splits > 1 ? p.splits : 1;
-    const int nwork = ntiles * S, nk = p.K / KT / S;   // nk is even
+    const int nwork = ntiles * S, nk = p.K / KT / S;   // nk is even and at least 2
     // Workgroup b runs on XCD b % 8; each XCD's workgroups take consecutive
     // tiles, which share A row panels in that XCD's L2.  Whole rounds: 32
     // consecutive tiles per XCD and round; otherwise an eighth of the items
@@ -158,7 +165,7 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
         for (int i = 0; i < LW; ++i) load_lds16_buf(wrsrc, wvoff + i * RPT * ldw_b, wko, st + i * RPT * 128);
         vm += LW;
         if (HAS_BIAS && wkt == 0) {
-            load_lds16_async(bias_src, reinterpret_cast<const float*>(smem + B_OFF + ((wt_ & 1) * NW + wave) * BIAS_BYTES));
+            load_lds16_async(bias_src, reinterpret_cast<const float*>(smem + B_OFF + ((wt_ % NBIAS) * NW + wave) * BIAS_BYTES));
             ++vm;
         }
         if constexpr (DA > DW) mark[DW - 1] = vm;
@@ -252,7 +259,7 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
     };
 
     // This wave's bias row segment of local tile t.
-    auto bias_of = [&](int t) __attribute__((always_inline)) { return smem + B_OFF + ((t & 1) * NW + wave) * BIAS_BYTES; };
+    auto bias_of = [&](int t) __attribute__((always_inline)) { return smem + B_OFF + ((t % NBIAS) * NW + wave) * BIAS_BYTES; };
     auto epilogue = [&](int t) __attribute__((always_inline)) {
         const int u = u0 + t * ustep, split = u / ntiles, tile = u - split * ntiles;
         const int mt = tile / ntn, wrow = mt * BM + wm * WM, n0 = (tile - mt * ntn) * BN;

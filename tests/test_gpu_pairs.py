@@ -111,6 +111,41 @@ def test_gemm_pair(env, M, Nn, K, S, tile):
     assert padding_kept(D)
 
 
+# at least three items for every workgroup on every tile, in whole rounds of
+# 256 x 256 tiles and not, rows and columns ending inside a tile; tiles of two
+# k-tiles, of four and of more.  The columns of a workgroup's items differ, and so
+# do their biases.
+@pytest.mark.parametrize("M,Nn", [(8187, 6136), (8450, 6392)])
+@pytest.mark.parametrize("K,S", [(64, 1), (128, 2), (384, 3)])
+def test_gemm_pair_many_tiles(env, M, Nn, K, S):
+    torch, eb, N, L = env
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    A, W = torch.randn(M, K, device="cuda", generator=g), 0.04 * torch.randn(Nn, K, device="cuda", generator=g)
+    b = 3 * torch.randn(Nn, device="cuda", generator=g)
+    sa, sw, sc = 2.0 ** 8, 2.0 ** 14, 2.0 ** 4
+    Ap, Wp = to_pair(torch, N, L, A, sa, s), to_pair(torch, N, L, W, sw, s)
+
+    def run(tile, epi, splits=1):
+        C = torch.empty(splits, M, Nn, device="cuda")
+        N.check(L.ebh_op_gemm_pair(vp(Ap), K, vp(Wp), K, 1 / (sa * sw), vp(b) if epi != EPI_NONE else None, vp(C), Nn,
+                                   sc if epi != EPI_NONE else 0.0, M, Nn, K, epi, splits, M * Nn, tile, s))
+        return C
+
+    ref = A.double() @ W.double().t()
+    tol = (2.0 ** -21 + 3 * K / 32 * 2.0 ** -22) * (A.abs().double() @ W.abs().double().t())   # as in test_gemm_pair
+    for epi, splits in ((EPI_BIAS, 1), (EPI_GELU, 1), (EPI_NONE, S)):
+        first = run(0, epi, splits)
+        if epi == EPI_BIAS:
+            u = ref + b.double()
+            assert ((unpair(torch, first[0], sc) - u).abs() <= tol + 2.0 ** -22 * (ref.abs() + b.abs().double()) + 2.0 ** -25 / sc).all()
+        elif epi == EPI_NONE:
+            assert ((first.double().sum(0) - ref).abs() <= tol + 2.0 ** -23 * ref.abs() * S).all()
+        for tile in range(1, 8):
+            for _ in range(2):
+                assert torch.equal(run(tile, epi, splits).view(torch.int32), first.view(torch.int32)), (tile, epi)
+
+
 @pytest.mark.parametrize("M,I,S", [(1, 128, 1), (127, 256, 2), (129, 384, 1), (300, 1536, 3), (1000, 1536, 12), (2600, 1536, 1)])
 def test_ffn_pair(env, M, I, S):
     """Against float64, and bit for bit against the two products that it stands

@@ -48,33 +48,50 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 # MI355X published dense peaks: fp32 matrix 157.3 TFLOP/s, bf16 / fp16 2.5 PFLOP/s; HBM3E 8 TB/s.
-# Dense matrix peaks of MI355X per algorithmic flop: fp32 products formed from
-# three fp16 MFMA products (the fp16 peak / 3), bf16 MFMA, and fp32 products
-# formed from six bf16 MFMA products (the bf16 peak / 6).  At most FEW_TOKENS
-# positions the fp32 dtypes run fp32 MFMA.
-PEAK_TFLOPS = {"fp32": 2500.0 / 3, "bf16": 2500.0, "fp32-bf16x6": 2500.0 / 6}
+# Dense matrix peaks of MI355X per algorithmic flop: bf16 MFMA, and fp32
+# products formed from six bf16 MFMA products (the bf16 peak / 6), or from three
+# or four fp16 ones (/ 3, / 4: fp16 pairs, without and with the weights' rest).
+# At most FEW_TOKENS positions the fp32 dtypes run fp32 MFMA.
+PEAK_TFLOPS = {"bf16": 2500.0, "fp32-bf16x6": 2500.0 / 6}
 FP32_MFMA_TFLOPS = 157.3
+PAIR_PEAK_TFLOPS = 2500.0 / 3
+PAIR_REST_PEAK_TFLOPS = 2500.0 / 4
 FEW_TOKENS = 64
 HBM_PEAK_GBS = 8000.0
 KERNELS = ("gemm_qkv", "attention", "gemm_out", "gemm_ffn_up", "gemm_ffn_down", "layernorm",
            "embed", "pool")
 
 
-def matrix_peak(dtype: str, positions: int) -> float:
-    """The matrix rate (TFLOP/s per algorithmic flop) that bounds a forward of
-    this many padded positions."""
+def fp32_products(model, B: int, S: int) -> str:
+    """How an fp32 model forms its products over [B, S] positions (its own rule,
+    by the padded length, the layers and the weights' range)."""
+    from edgebert_amd import _native
+    return {1: "pair", 2: "pair_rest"}.get(_native.lib().ebh_op_products(model._h, B, S), "mfma")
+
+
+def matrix_peak(dtype: str, positions: int, products: str = "mfma", family: str = "gemm") -> float:
+    """The matrix rate (TFLOP/s per algorithmic flop) that bounds a kernel family
+    of a forward of this many padded positions; products: fp32_products."""
+    if dtype == "fp32":
+        if products == "mfma":
+            return FP32_MFMA_TFLOPS
+        rest = products == "pair_rest" and family.startswith("gemm")
+        return round(PAIR_REST_PEAK_TFLOPS if rest else PAIR_PEAK_TFLOPS, 1)
     return FP32_MFMA_TFLOPS if dtype != "bf16" and positions <= FEW_TOKENS else round(PEAK_TFLOPS[dtype], 1)
 
 
-def gemm_arithmetic(dtype: str, positions: int) -> str:
+def gemm_arithmetic(dtype: str, positions: int, products: str = "mfma") -> str:
     """How the dtype's matrix products are formed at this many padded positions."""
     if dtype == "bf16":
         return "bf16 MFMA products, fp32 accumulate"
     if positions <= FEW_TOKENS:
         return f"fp32 MFMA products (the few-token kernels, at most {FEW_TOKENS} positions)"
     if dtype == "fp32":
-        return ("fp32 operands held as fp16 pairs (23 bits), three fp16 MFMA products per fp32 product, "
-                "fp32 accumulate; models whose weights lie outside the pairs' range run fp32 MFMA")
+        return {"mfma": "fp32 MFMA products",
+                "pair": "fp32 operands held as fp16 pairs (23 bits), three fp16 MFMA products per fp32 product, "
+                        "fp32 accumulate",
+                "pair_rest": "fp32 operands held as fp16 pairs (23 bits) and the weights' 24th bit beside them, four "
+                             "fp16 MFMA products per fp32 product, fp32 accumulate"}[products]
     return ("fp32 operands split into three bf16 parts, six bf16 MFMA products per fp32 product, "
             "fp32 accumulate (EBH_DTYPE_F32_BF16X6)")
 
@@ -359,6 +376,7 @@ def config_leg(eb, torch, name: str, steps: int, warmup: int, graph_replay: bool
     wall = time.perf_counter() - t_all
     model.synchronize()
     fused = few_fused(cfg, B, S, dtype)
+    products = fp32_products(model, B, S)
     families = {}
     for fam in KERNELS:
         if fused and fam == "gemm_out":
@@ -377,7 +395,7 @@ def config_leg(eb, torch, name: str, steps: int, warmup: int, graph_replay: bool
         if fam == "gemm_ffn_down" and "gemm_ffn_up" not in families:   # one launch for both
             work += kernel_work(cfg, lengths, B, "gemm_ffn_up", fused, dtype)[0]
         if bound == "mfma":
-            achieved, peak, punit = work / (avg * 1e-3) / 1e12, matrix_peak(dtype, B * S), "TFLOP/s"
+            achieved, peak, punit = work / (avg * 1e-3) / 1e12, matrix_peak(dtype, B * S, products, fam), "TFLOP/s"
         else:
             achieved, peak, punit = work / (avg * 1e-3) / 1e9, HBM_PEAK_GBS, "GB/s"
         families[fam] = {"bound": bound, "achieved": round(achieved, 3), "peak": peak, "unit": punit,
@@ -392,7 +410,7 @@ def config_leg(eb, torch, name: str, steps: int, warmup: int, graph_replay: bool
     return {"value": round(B * steps / wall, 2), "unit": "sentences/s", "steps": steps, "warmup": warmup,
             "ms_per_step": round(ms, 4), "p50_batch_latency_ms": round(float(np.median(times)) * 1e3, 4),
             "dtype": LEG_DTYPE_NOTE[dtype],
-            "gemm_arithmetic": gemm_arithmetic(dtype, B * S),
+            "gemm_arithmetic": gemm_arithmetic(dtype, B * S, products),
             "workload": f"{name}: {cfg.num_hidden_layers}L H{cfg.hidden_size} I{cfg.intermediate_size} "
                         f"heads{cfg.num_attention_heads} batch {B} x seq {S}, lengths "
                         f"{spec.len_lo}-{spec.len_hi}",
@@ -502,11 +520,12 @@ def main():
     tokens = int(mask.sum())
     avg_kernel_ms = prof_ms / max(launches, 1)
     fused = few_fused(cfg, B, S, dtype)
+    products = fp32_products(model, B, S)
     work, bound, wunit = kernel_work(cfg, lengths, B, args.profile_kernel, fused, dtype)
     if covers:
         work += kernel_work(cfg, lengths, B, "gemm_ffn_down", fused, dtype)[0]
     if bound == "mfma":
-        achieved, peak, punit = work / (avg_kernel_ms * 1e-3) / 1e12, matrix_peak(dtype, B * S), "TFLOP/s"
+        achieved, peak, punit = work / (avg_kernel_ms * 1e-3) / 1e12, matrix_peak(dtype, B * S, products, args.profile_kernel), "TFLOP/s"
     else:
         achieved, peak, punit = work / (avg_kernel_ms * 1e-3) / 1e9, HBM_PEAK_GBS, "GB/s"
     fwd_flops = forward_flops(cfg, lengths)
@@ -525,7 +544,7 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": {"fp32": "f32", "bf16": "bf16", "fp32-bf16x6": "f32 (bf16x6 GEMM products)"}[dtype],
-        "gemm_arithmetic": gemm_arithmetic(dtype, B * S),
+        "gemm_arithmetic": gemm_arithmetic(dtype, B * S, products),
         "data": "synthetic (seeded ids, random-init N(0,0.02) weights; no checkpoint offline)",
         "config": {"workload": f"{args.config}: {cfg.num_hidden_layers}L H{cfg.hidden_size} "
                                f"I{cfg.intermediate_size} heads{cfg.num_attention_heads} "
@@ -582,7 +601,7 @@ def main():
                 fwork += kernel_work(cfg, lengths, B, "gemm_ffn_up", fused, dtype)[0]
             favg = fms / n
             if fbound == "mfma":
-                fa, fp, fu = fwork / (favg * 1e-3) / 1e12, matrix_peak(dtype, B * S), "TFLOP/s"
+                fa, fp, fu = fwork / (favg * 1e-3) / 1e12, matrix_peak(dtype, B * S, products, fam), "TFLOP/s"
             else:
                 fa, fp, fu = fwork / (favg * 1e-3) / 1e9, HBM_PEAK_GBS, "GB/s"
             fams[fam] = {"bound": fbound, "achieved": round(fa, 3), "peak": fp, "unit": fu,

@@ -81,6 +81,10 @@ _SIGS = {
                                 _vp]),
     "ebh_op_gemm_pair": (_i32, [_vp, _i64, _vp, _i64, _f32, _vp, _vp, _i64, _f32, _i32, _i32, _i32, _i32, _i32,
                                 _i64, _i32, _vp]),
+    "ebh_op_products": (_i32, [_vp, _i32, _i32]),
+    "ebh_op_gemm_pair_rest": (_i32, [_vp, _i64, _vp, _i64, _f32, _vp, _vp, _i64, _f32, _i32, _i32, _i32, _i32, _i32,
+                                     _i64, _i32, _vp]),
+    "ebh_op_to_pair_rest": (_i32, [_vp, _vp, _i32, _i32, _f32, _vp]),
     "ebh_op_ffn_pair": (_i32, [_vp, _vp, _vp, _vp, _f32, _f32, _f32, _vp, _i32, _i32, _i32, _i64, _vp]),
     "ebh_op_attention_pair": (_i32, [_vp, _f32, _vp, _i32, _i32, _i32, _i32, _vp, _f32, _vp]),
     "ebh_op_to_pair": (_i32, [_vp, _vp, _i64, _f32, _vp]),

@@ -79,7 +79,7 @@ struct DevLayer {
     float *wqkv, *bqkv, *wo, *bo, *ln1_g, *ln1_b, *w1, *b1, *w2, *b2, *ln2_g, *ln2_b;
     uint16_t *wqkv16, *wo16, *w116, *w216;
     // fp32 models whose products run on fp16 pairs (PairScales): the weights
-    // in the pair format
+    // in the pair format, each row's rest behind it (launch_to_pair_rest)
     uint32_t *wqkvp, *wop, *w1p, *w2p;
 };
 
@@ -397,12 +397,42 @@ int enqueue_pool(ebh_model* m, Workspace& w, int B, int S, int normalize, float*
     return EBH_OK;
 }
 
+// The products of an fp32 model's forward (wpair): on fp32 MFMA, on fp16 pairs,
+// or on pairs with the weights' rest (gemm16.hpp).  The rule goes by the padded
+// length S and the layers, which every entry point knows.
+//  * At most 64 positions in all a product is a chain of memory round trips, and
+//    the few-token kernels stay.
+//  * A weight's pair rounding is the same for every token, so it adds up over
+//    layers and is not averaged out by the mean over a sequence, as the other
+//    roundings are.  Error of the vectors against float64 over that of fp32
+//    MFMA products, full batches of S tokens, mean over seeds, pairs / pairs with
+//    the rest:
+//      S                 48         96         128        192        256        384        512
+//      H 384, 1 layer    0.85/0.79  0.95/0.83  0.95/0.86  1.07/0.94  1.01/0.90  1.12/0.98  1.20/0.99
+//      H 384, 6 layers   0.89/0.78  0.97/0.79  1.03/0.79  1.17/0.84  1.22/0.84  1.27/0.96  1.39/0.97
+//      H 768, 2 layers   0.75/0.69  0.80/0.72  0.81/0.72  0.92/0.78  0.95/0.78  1.05/0.86  1.05/0.86
+//      H 768, 12 layers  0.94/0.81  1.09/0.87  1.19/0.94  1.31/1.00  1.37/1.03  1.79/1.32  1.69/1.34
+//    (256 x 128 of MiniLM-L6: 0.88.)  So pairs alone are for S <= 128 and at most
+//    64 times 12 layers squared, pairs with the rest for at most 192 times 12
+//    layers squared.  Beyond that (deep models on long sequences, whose tokens
+//    have become so alike that even the sums round alike) the fp32 MFMA products
+//    stay.
+enum class Products { mfma, pair, pair_rest };
+Products products_for(const ebh_model* m, int B, int S) {
+    const ebh_config& c = m->cfg;
+    const int64_t depth = (int64_t)S * c.num_hidden_layers * c.num_hidden_layers;
+    if (!m->wpair || (int64_t)B * S <= ebh::SKINNY_MAX_ROWS || depth > 192 * 144) return Products::mfma;
+    if (S <= 128 && depth <= 64 * 144) return Products::pair;
+    // the rest's k-tiles come in pairs of 64
+    return c.hidden_size % 128 == 0 && c.intermediate_size % 128 == 0 ? Products::pair_rest : Products::mfma;
+}
+
 // The encoder layers and the pool of an fp32 forward whose products run on
 // fp16 pairs (after the embeddings, which wrote X and its pairs).  Every
 // operand of a product is written as pairs by the kernel that makes it (4
 // bytes an element, as in fp32); X itself stays fp32 for the residual sums.
 int enqueue_pair_layers(ebh_model* m, Workspace& w, int B, int S, int normalize, float* d_out, hipStream_t s,
-                        float* d_scores, int64_t tokens, int prof_kind, const int* seq_order) {
+                        float* d_scores, int64_t tokens, int prof_kind, const int* seq_order, bool rest) {
     const ebh_config& c = m->cfg;
     const int H = c.hidden_size, I = c.intermediate_size, nh = c.num_attention_heads, hd = H / nh;
     const float eps = c.layer_norm_eps, scale = 1.0f / sqrtf((float)hd);
@@ -425,7 +455,8 @@ int enqueue_pair_layers(ebh_model* m, Workspace& w, int B, int S, int normalize,
         a.W = W;
         a.bias = bias;
         a.C = C;
-        a.lda = a.ldw = K;
+        a.lda = K;
+        a.ldw = K + K / 2;
         a.ldc = N;
         a.M_max = T;
         a.M_dev = w.ntok;
@@ -436,6 +467,7 @@ int enqueue_pair_layers(ebh_model* m, Workspace& w, int B, int S, int normalize,
         a.acc_scale = acc_scale;
         a.out_scale = out_scale;
         a.tile = -1;
+        a.rest = rest;
         ProfPair p2{};
         bool on2 = false;
         prof_begin(m, prof_kind, kind, s, p2, on2);
@@ -454,11 +486,11 @@ int enqueue_pair_layers(ebh_model* m, Workspace& w, int B, int S, int normalize,
         return EBH_OK;
     };
     const bool exact = tokens >= 0;
-    const int sp_out = ebh::gemm16_pair_plan(T_pad, false, H, H, false, 1, max_splits).splits,
-              sp_down = ebh::ffn_pair_plan(T_pad, false, H, I, 1, max_splits).splits;
-    const ebh::Gemm16Plan p_qkv = ebh::gemm16_pair_plan(T, exact, 3 * H, H, false, 1, 1),
-                          p_out = ebh::gemm16_pair_plan(T, exact, H, H, false, sp_out, sp_out);
-    const ebh::FfnPairPlan p_ffn = ebh::ffn_pair_plan(T, exact, H, I, sp_down, sp_down);
+    const int sp_out = ebh::gemm16_pair_plan(T_pad, false, H, H, false, 1, max_splits, rest).splits,
+              sp_down = ebh::ffn_pair_plan(T_pad, false, H, I, 1, max_splits, rest).splits;
+    const ebh::Gemm16Plan p_qkv = ebh::gemm16_pair_plan(T, exact, 3 * H, H, false, 1, 1, rest),
+                          p_out = ebh::gemm16_pair_plan(T, exact, H, H, false, sp_out, sp_out, rest);
+    const ebh::FfnPairPlan p_ffn = ebh::ffn_pair_plan(T, exact, H, I, sp_down, sp_down, rest);
     for (size_t l = 0; l < m->layers.size(); ++l) {
         const DevLayer& L = m->layers[l];
         const PairScales& q = m->pair_scales[l];
@@ -486,6 +518,8 @@ int enqueue_pair_layers(ebh_model* m, Workspace& w, int B, int S, int normalize,
             a.M_max = T;
             a.M_dev = w.ntok;
             a.I = I;
+            a.ldw1 = H + H / 2;
+            a.ldw2 = I + I / 2;
             a.splits = p_ffn.splits;
             a.split_stride = (int64_t)T * H;
             a.scale1 = 1.0f / (q.mid * q.w1);
@@ -530,9 +564,8 @@ int enqueue_kernels(ebh_model* m, Workspace& w, const int* d_ids, const int* d_m
     bool on = false;
     const bool bf16 = m->dtype == EBH_DTYPE_BF16;
     const bool few_pack = ebh::pack_embed_few_fits(B, S, H);
-    // fp32 products on fp16 pairs (gemm16.hpp).  Up to 64 rows a product is a
-    // chain of memory round trips, and the few-token kernels stay.
-    const bool pair = m->wpair && T > ebh::SKINNY_MAX_ROWS;
+    const Products products = products_for(m, B, S);
+    const bool pair = products != Products::mfma;
     // The pair copy of X shares CTX's memory: X is read by the QKV product
     // before attention writes the context there, and the context by the
     // output product before the LayerNorm writes the next X.
@@ -552,7 +585,9 @@ int enqueue_kernels(ebh_model* m, Workspace& w, const int* d_ids, const int* d_m
                                      w.X16, s, xp, pair ? m->pair_scales[0].x : 0.0f));
         prof_end(m, s, pp, on);
     }
-    if (pair) return enqueue_pair_layers(m, w, B, S, normalize, d_out, s, d_scores, tokens, prof_kind, seq_order);
+    if (pair)
+        return enqueue_pair_layers(m, w, B, S, normalize, d_out, s, d_scores, tokens, prof_kind, seq_order,
+                                   products == Products::pair_rest);
 
     // bf16 models keep the residual stream in bf16 (X16, written by each
     // LayerNorm; every sum and statistic stays fp32) and hand the GEMMs bf16
@@ -1102,7 +1137,7 @@ static int prepare_pairs(ebh_model* m) {
             if (!(f > 0.0f)) return EBH_OK;
         in = norm_of(p + 2 * H, p + 3 * H);
     }
-    const size_t words = 4 * H * H + 2 * H * I;          // pair weights of a layer
+    const size_t words = (4 * H * H + 2 * H * I) * 3 / 2;   // pair weights of a layer, with their rests
     if (hipMalloc(&m->wpair, L * words * 4) != hipSuccess) {   // no room: the fp32 kernels need none
         (void)hipGetLastError();
         m->wpair = nullptr;
@@ -1111,14 +1146,14 @@ static int prepare_pairs(ebh_model* m) {
     for (size_t l = 0; l < L; ++l) {
         DevLayer& d = m->layers[l];
         uint32_t* w = static_cast<uint32_t*>(m->wpair) + l * words;
-        d.wqkvp = w;
-        d.wop = w + 3 * H * H;
-        d.w1p = w + 4 * H * H;
-        d.w2p = w + 4 * H * H + H * I;
-        HIP_TRY(ebh::launch_to_pair(d.wqkv, d.wqkvp, 3 * H * H, sc[l].wqkv, st));
-        HIP_TRY(ebh::launch_to_pair(d.wo, d.wop, H * H, sc[l].wo, st));
-        HIP_TRY(ebh::launch_to_pair(d.w1, d.w1p, H * I, sc[l].w1, st));
-        HIP_TRY(ebh::launch_to_pair(d.w2, d.w2p, H * I, sc[l].w2, st));
+        const struct { const float* x; uint32_t** p; size_t n, k; float scale; } mats[] = {
+            {d.wqkv, &d.wqkvp, 3 * H, H, sc[l].wqkv}, {d.wo, &d.wop, H, H, sc[l].wo},
+            {d.w1, &d.w1p, I, H, sc[l].w1}, {d.w2, &d.w2p, H, I, sc[l].w2}};
+        for (const auto& x : mats) {
+            *x.p = w;
+            HIP_TRY(ebh::launch_to_pair_rest(x.x, w, (int64_t)x.n, (int)x.k, x.scale, st));
+            w += x.n * x.k * 3 / 2;
+        }
     }
     HIP_TRY(hipStreamSynchronize(st));
     m->pair_scales = std::move(sc);
@@ -1661,9 +1696,9 @@ int ebh_op_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, int64_t 
     return EBH_OK;
 }
 
-int ebh_op_gemm_pair(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t ldw, float acc_scale,
-                     const float* bias, void* C, int64_t ldc, float c_scale, int32_t M, int32_t N, int32_t K,
-                     int32_t epilogue, int32_t splits, int64_t split_stride, int32_t tile, void* stream) {
+static int op_gemm_pair(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t ldw, float acc_scale,
+                        const float* bias, void* C, int64_t ldc, float c_scale, int32_t M, int32_t N, int32_t K,
+                        int32_t epilogue, int32_t splits, int64_t split_stride, int32_t tile, void* stream, bool rest) {
     if (!A || !W || !C || M < 0 || N <= 0 || K <= 0 || splits < 1 || tile < -1 || tile >= ebh::GEMM16_TILES ||
         !(acc_scale > 0.0f) || !(c_scale >= 0.0f) || epilogue < EBH_EPI_BIAS || epilogue > EBH_EPI_NONE ||
         epilogue == EBH_EPI_BIAS_RESID || (epilogue != EBH_EPI_NONE) != (c_scale > 0.0f) ||
@@ -1685,11 +1720,34 @@ int ebh_op_gemm_pair(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t 
     a.acc_scale = acc_scale;
     a.out_scale = c_scale;
     a.tile = tile < 0 ? -1 : tile % 4;
-    const int family = tile < 0 ? ebh::gemm16_pair_plan(M, true, N, K, epilogue == EBH_EPI_BIAS_GELU, splits, splits).family
+    a.rest = rest;
+    const int family = tile < 0 ? ebh::gemm16_pair_plan(M, true, N, K, epilogue == EBH_EPI_BIAS_GELU, splits, splits, rest).family
                                 : tile / 4;
     const hipError_t e = ebh::launch_gemm16_pair(a, epilogue, c_scale > 0.0f, family, (hipStream_t)stream);
     if (e == hipErrorInvalidValue) return fail(EBH_ERR_INVALID_ARG, "pair gemm shape, stride or alignment");
     if (e != hipSuccess) return fail(EBH_ERR_HIP, "gemm launch failed: %s", hipGetErrorString(e));
+    return EBH_OK;
+}
+
+int ebh_op_gemm_pair(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t ldw, float acc_scale,
+                     const float* bias, void* C, int64_t ldc, float c_scale, int32_t M, int32_t N, int32_t K,
+                     int32_t epilogue, int32_t splits, int64_t split_stride, int32_t tile, void* stream) {
+    return op_gemm_pair(A, lda, W, ldw, acc_scale, bias, C, ldc, c_scale, M, N, K, epilogue, splits, split_stride, tile,
+                        stream, false);
+}
+
+int ebh_op_gemm_pair_rest(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t ldw, float acc_scale,
+                          const float* bias, void* C, int64_t ldc, float c_scale, int32_t M, int32_t N, int32_t K,
+                          int32_t epilogue, int32_t splits, int64_t split_stride, int32_t tile, void* stream) {
+    return op_gemm_pair(A, lda, W, ldw, acc_scale, bias, C, ldc, c_scale, M, N, K, epilogue, splits, split_stride, tile,
+                        stream, true);
+}
+
+int ebh_op_to_pair_rest(const float* w, uint32_t* y, int32_t N, int32_t K, float scale, void* stream) {
+    if (!w || !y || N < 0 || K <= 0 || !(scale > 0.0f)) return fail(EBH_ERR_INVALID_ARG, "bad pair arguments");
+    const hipError_t e = ebh::launch_to_pair_rest(w, y, N, K, scale, (hipStream_t)stream);
+    if (e == hipErrorInvalidValue) return fail(EBH_ERR_INVALID_ARG, "K must be a multiple of 8, w and y 16-byte aligned");
+    if (e != hipSuccess) return fail(EBH_ERR_HIP, "launch failed: %s", hipGetErrorString(e));
     return EBH_OK;
 }
 
@@ -1706,6 +1764,8 @@ int ebh_op_ffn_pair(const uint32_t* X, const uint32_t* W1, const float* b1, cons
     a.Y = Y;
     a.M_max = M;
     a.I = I;
+    a.ldw1 = 384;
+    a.ldw2 = I;
     a.splits = splits;
     a.split_stride = split_stride;
     a.scale1 = scale1;
@@ -1723,6 +1783,17 @@ int ebh_op_to_pair(const float* x, uint32_t* y, int64_t n, float scale, void* st
     if (e == hipErrorInvalidValue) return fail(EBH_ERR_INVALID_ARG, "n must be a multiple of 8, x and y 16-byte aligned");
     if (e != hipSuccess) return fail(EBH_ERR_HIP, "launch failed: %s", hipGetErrorString(e));
     return EBH_OK;
+}
+
+int ebh_op_products(const ebh_model* m, int32_t B, int32_t S) {
+    int rc = check_model_ready(m);
+    if (rc || (rc = check_dims(m, B, S))) return rc;
+    if (m->dtype != EBH_DTYPE_F32) return EBH_PRODUCTS_DTYPE;
+    switch (products_for(m, B, S)) {
+        case Products::pair: return EBH_PRODUCTS_PAIR;
+        case Products::pair_rest: return EBH_PRODUCTS_PAIR_REST;
+        default: return EBH_PRODUCTS_MFMA;
+    }
 }
 
 int ebh_op_attention(const float* qkv, const int32_t* cu_seqlens, int32_t B, int32_t max_len,

@@ -14,7 +14,8 @@
 // A row block's ranges (splits) are workgroups of their own, writing partial
 // sums that the LayerNorm adds in order, as split-K products do.
 //
-// LDS is all 160 KB: G, and 96 KB that step 1 uses as three stages of 32 KB (X
+// LDS is all 160 KB (so there is no room for the weights' rest, and products
+// that need it run as two): G, and 96 KB that step 1 uses as three stages of 32 KB (X
 // and W1, two k-tiles in flight ahead) and step 3 as two of 48 KB (W2).  The
 // steps hand it over without a gap: W2's first k-tile is loaded during step 1's
 // last k-tile (into the two stages that are done), its second during the GELU,
@@ -63,17 +64,17 @@ __global__ __launch_bounds__(512, 2) void ffn_pair_kernel(FfnPairArgs p) {
     const uint32_t chunk = 16 * ((tid & 7) ^ chunk_swizzle16<8>(r0));
     const int rw = (r0 & ~31) + 8 * ((r0 >> 2) & 3) + 4 * ((r0 >> 4) & 1) + (r0 & 3);
     constexpr uint32_t XB = FH * 4;
-    const uint32_t w2b = (uint32_t)p.I * 4;
-    const uint32_t xvo = r0 * XB + chunk, w1vo = rw * XB + chunk, w2vo = rw * w2b + chunk;
+    const uint32_t w1b = (uint32_t)p.ldw1 * 4, w2b = (uint32_t)p.ldw2 * 4;
+    const uint32_t xvo = r0 * XB + chunk, w1vo = rw * w1b + chunk, w2vo = rw * w2b + chunk;
     const g16_v4i xr = make_rsrc(p.X + (int64_t)m0 * FH, (uint32_t)min(M - m0, FBM) * XB);
     const g16_v4i w2r = make_rsrc(p.W2, (uint32_t)FH * w2b);
     auto issue_k = [&](int c, int j) __attribute__((always_inline)) {   // step 1's k-tile j of chunk c: 4 loads
-        const g16_v4i w1r = make_rsrc(p.W1 + (int64_t)c * FBC * FH, FBC * XB);
+        const g16_v4i w1r = make_rsrc(p.W1 + (int64_t)c * FBC * p.ldw1, FBC * w1b);
         const uint32_t st = ldsR + (uint32_t)(j % 3) * ST1 + wave * 1024, ko = j * 128;
 #pragma unroll
         for (int i = 0; i < 2; ++i) load_lds16_buf(xr, xvo + i * 64 * XB, ko, st + i * 8192);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) load_lds16_buf(w1r, w1vo + i * 64 * XB, ko, st + FBM * 128 + i * 8192);
+        for (int i = 0; i < 2; ++i) load_lds16_buf(w1r, w1vo + i * 64 * w1b, ko, st + FBM * 128 + i * 8192);
     };
     auto issue_w = [&](int c, int kt) __attribute__((always_inline)) {  // step 3's k-tile kt: 6 loads
         const uint32_t st = ldsR + (uint32_t)(kt & 1) * ST2 + wave * 1024, ko = (uint32_t)(c * FBC + kt * 32) * 4;
@@ -272,6 +273,7 @@ bool ffn_pair_shape_ok(int H, int I) { return H == FH && I > 0 && I % FBC == 0; 
 hipError_t launch_ffn_pair(const FfnPairArgs& a, hipStream_t s) {
     auto al16 = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
     if (a.M_max < 0 || a.I <= 0 || a.I % FBC || a.splits < 1 || (a.I / FBC) % a.splits || a.I > (1 << 20) / 4 ||
+        a.ldw1 < FH || a.ldw2 < a.I || a.ldw1 % 4 || a.ldw2 % 4 || a.ldw1 > (1 << 20) || a.ldw2 > (1 << 20) ||
         !al16(a.X) || !al16(a.W1) || !al16(a.W2) || !al16(a.b1) || !al16(a.Y) || a.split_stride % 4)
         return hipErrorInvalidValue;
     const int64_t items = (int64_t)((a.M_max + FBM - 1) / FBM) * a.splits;

@@ -14,9 +14,21 @@
 // of the fp32 MFMA's (K = 384: 2.2e-7 against 3.5e-7; K = 3072: 6.2e-7 against
 // 9.9e-7; the same on GELU outputs and on rows with outlier features), because
 // the fp32 form rounds its sum every k and this one every 32: the pairs'
-// own rounding (2^-24 per operand) is a small part of either.  The error is
-// flat for scales from 2^4 to 2^10, so one scale per matrix, taken from a
-// bound of its values, is enough.
+// own rounding is a small part of either.  (h and l hold 23 of a value's 24
+// bits: three values in four exactly, the fourth off by one unit of the 24th,
+// at most 2^-23 of it.)  The error is flat for scales from 2^4 to 2^10, so one
+// scale per matrix, taken from a bound of its values, is enough.
+//
+// The rest.  Rounding errors differ from token to token, and a mean over a
+// sequence takes them out; a weight's is the same for every token and stays.
+// Over long sequences it is what is left (MiniLM-L6, 512 tokens: 0.9e-7 of the
+// vector's 1.5e-7, where fp32 MFMA products give 1.2e-7).  So weight rows carry
+// their rest, r = fp16(s w - h - l), which makes them exact, behind their pairs
+// (launch_to_pair_rest), and products that are told to add ah.br, one more
+// v_mfma_f32_16x16x32_f16 per 32 k: k-tiles of 64 rests against the h of 64 k,
+// before the pairs', while the sums are small.  They take 1.2-1.25 times as long
+// (forwards: 256 x 128 2.75 -> 3.42 ms, 16 x 512 907 -> 1,094 us, fp32 MFMA 5.7 ms
+// and 1,642 us).
 //
 // The fp16 MFMA rounds its aligned terms down (towards minus infinity), so its
 // sums sit 1e-8 (K = 384) to 4e-8 (K = 1536) of their size low on average, a
@@ -76,7 +88,7 @@ constexpr int gemm16_lds(int bm, int bn, int waves, int nsa, int nsw, bool bias)
     return (nsa * bm + nsw * bn) * 128 + (bias ? gemm16_bias_slots(nsw) * waves * 1024 : 0);
 }
 
-template <bool PAIR, int BM, int BN, int WAVES_M, int WAVES_N, int NSA, int NSW, int EPI, int OUT>
+template <bool PAIR, bool REST, int BM, int BN, int WAVES_M, int WAVES_N, int NSA, int NSW, int EPI, int OUT>
 __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, char* const smem) {
     constexpr int NT = 64 * WAVES_M * WAVES_N, NW = WAVES_M * WAVES_N;
     constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
@@ -104,13 +116,15 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
 
     const int N = p.N;
     const int ntn = (N + BN - 1) / BN, ntiles = ((M + BM - 1) / BM) * ntn;
-    const int S = p.splits > 1 ? p.splits : 1;
+    const int S = EPI == EPI_NONE && p.splits > 1 ? p.splits : 1;
     const int nwork = ntiles * S, nk = p.K / KT / S;   // nk is even and at least 2
+    const int nr = REST ? nk / 2 : 0, nkt = nr + nk;   // k-tiles of the rest, even, and of the tile
     // Workgroup b runs on XCD b % 8; each XCD's workgroups take consecutive
     // tiles, which share A row panels in that XCD's L2.  Whole rounds: 32
     // consecutive tiles per XCD and round; otherwise an eighth of the items
     // per XCD, so that the last, partial round spreads over all of them.
-    const int G = gridDim.x;
+    int G = gridDim.x;
+    asm("" : "+s"(G));   // opaque: the tiles' bodies share nothing derived from it, which would be held (and spilled) across them
     int u0 = blockIdx.x, ustep = G, uend = nwork;
     if ((G & 7) == 0 && nwork % G == 0) {
         u0 = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
@@ -121,8 +135,7 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
         uend = (int)((int64_t)(x + 1) * nwork / 8);
     }
     const int my_tiles = u0 < uend ? (uend - u0 + ustep - 1) / ustep : 0;
-    const int total = my_tiles * nk;
-    if (total == 0) return;  // uniform over the workgroup
+    if (my_tiles == 0) return;  // uniform over the workgroup
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WAVES_N, wn = wave % WAVES_N;
@@ -134,13 +147,14 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
     const int rw = (r0 & ~31) + 8 * ((r0 >> 2) & 3) + 4 * ((r0 >> 4) & 1) + (r0 & 3);
     const uint32_t lda_b = (uint32_t)p.lda * ES, ldw_b = (uint32_t)p.ldw * ES;
     const uint32_t avoff = r0 * lda_b + chunk, wvoff = rw * ldw_b + chunk;
+    uint32_t avo = REST ? avoff + chunk : avoff;  // k-tiles of the rest: A's h chunks, every other one of 64 k
 
     // Load cursors: the next k-tile of A and of W to load, their panels'
     // descriptors and k offsets.
     g16_v4i arsrc, wrsrc;
     uint32_t ako = 0, wko = 0;
     const float* bias_src = nullptr;
-    int ia = 0, akt = 0, at_ = 0, iw = 0, wkt = 0, wt_ = 0;   // k-tile count, k-tile within the tile, tile
+    int akt = 0, at_ = 0, wkt = 0, wt_ = 0;       // k-tile within the tile, tile
     auto a_at = [&](int t) __attribute__((always_inline)) {
         const int u = u0 + t * ustep, split = u / ntiles, tile = u - split * ntiles, m0 = (tile / ntn) * BM;
         arsrc = make_rsrc(static_cast<const char*>(p.A) + (int64_t)m0 * p.lda * ES, (uint32_t)min(M - m0, BM) * lda_b);
@@ -149,7 +163,7 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
     auto w_at_tile = [&](int t) __attribute__((always_inline)) {
         const int u = u0 + t * ustep, split = u / ntiles, tile = u - split * ntiles, n0 = (tile - (tile / ntn) * ntn) * BN;
         wrsrc = make_rsrc(static_cast<const char*>(p.W) + (int64_t)n0 * p.ldw * ES, (uint32_t)min(N - n0, BN) * ldw_b);
-        wko = (uint32_t)(split * nk) * 128;
+        wko = REST ? (uint32_t)p.K * 4 + (uint32_t)(split * nk) * 64 : (uint32_t)(split * nk) * 128;
         if (HAS_BIAS) bias_src = p.bias + min(n0 + wn * WN + 4 * lane, N - 4);
     };
     int vm = 0;                                    // vector memory instructions issued by this wave
@@ -158,8 +172,8 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
     int mark[DW];
 #pragma unroll
     for (int d = 0; d < DW; ++d) mark[d] = 0;
-    auto issue_w = [&]() __attribute__((always_inline)) {
-        if (iw >= total) return;
+    auto issue_w = [&](int iw) __attribute__((always_inline)) {   // the workgroup's iw-th k-tile
+        if (wt_ >= my_tiles) return;
         const uint32_t st = lds0 + W_OFF + (uint32_t)(iw % NSW) * ST_W + (uint32_t)wave * 1024;
 #pragma unroll
         for (int i = 0; i < LW; ++i) load_lds16_buf(wrsrc, wvoff + i * RPT * ldw_b, wko, st + i * RPT * 128);
@@ -169,24 +183,30 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
             ++vm;
         }
         if constexpr (DA > DW) mark[DW - 1] = vm;
-        ++iw;
         wko += 128;
-        if (++wkt == nk) {
+        ++wkt;
+        if (REST && wkt == nr) wko = 2 * (wko - (uint32_t)p.K * 4) - nk * 128;   // from the rest's end to the pairs' start
+        if (wkt == nkt) {
             wkt = 0;
             if (++wt_ < my_tiles) w_at_tile(wt_);
         }
     };
-    auto issue_a = [&]() __attribute__((always_inline)) {
-        if (ia >= total) return;
+    auto issue_a = [&](int ia) __attribute__((always_inline)) {
+        if (at_ >= my_tiles) return;
         const uint32_t st = lds0 + (uint32_t)(ia % NSA) * ST_A + (uint32_t)wave * 1024;
 #pragma unroll
-        for (int i = 0; i < LA; ++i) load_lds16_buf(arsrc, avoff + i * RPT * lda_b, ako, st + i * RPT * 128);
+        for (int i = 0; i < LA; ++i) load_lds16_buf(arsrc, avo + i * RPT * lda_b, ako, st + i * RPT * 128);
         vm += LA;
         if constexpr (DA == DW) mark[DW - 1] = vm;
-        ++ia;
-        ako += 128;
-        if (++akt == nk) {
+        ako += REST && akt < nr ? 256 : 128;
+        ++akt;
+        if (REST && akt == nr) {
+            ako -= nk * 128;
+            avo = avoff;
+        }
+        if (akt == nkt) {
             akt = 0;
+            if (REST) avo = avoff + chunk;
             if (++at_ < my_tiles) a_at(at_);
         }
     };
@@ -212,18 +232,20 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
         for (int d = 0; d + 1 < DW; ++d) mark[d] = mark[d + 1];
         lds_barrier();
     };
-    auto mfma_step = [&](int s, int as, int ws) __attribute__((always_inline)) {
-        // smallest products first; consecutive MFMAs on different accumulators
+    auto mfma_step = [&](int s, int as, int ws, auto two) __attribute__((always_inline)) {
+        // smallest products first; consecutive MFMAs on different accumulators;
+        // two: a lane's two chunks are two runs of k (bf16, the rest), not h and l
+        constexpr bool TWO = decltype(two)::value;
 #pragma unroll
-        for (int pr = PAIR ? 0 : 1; pr < 3; ++pr)
+        for (int pr = TWO ? 1 : 0; pr < 3; ++pr)
 #pragma unroll
             for (int i = 0; i < SB; ++i)
 #pragma unroll
                 for (int j = 0; j < FN; ++j) {
                     g16_v4f& d = acc[s * SB + i][j];
                     if constexpr (PAIR) {
-                        const g16_v4f& w = wf[ws][j][pr == 1 ? 1 : 0];
-                        const g16_v4f& a = af[as][i][pr == 0 ? 1 : 0];
+                        const g16_v4f& w = wf[ws][j][TWO ? pr - 1 : (pr == 1 ? 1 : 0)];
+                        const g16_v4f& a = af[as][i][TWO ? pr - 1 : (pr == 0 ? 1 : 0)];
                         d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, w), __builtin_bit_cast(v8h, a), d, 0, 0, 0);
                     } else {
                         d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(g16_v8bf, wf[ws][j][pr - 1]),
@@ -231,7 +253,7 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
                     }
                 }
     };
-    auto run_ktile = [&](auto pset, bool first) __attribute__((always_inline)) {
+    auto run_ktile = [&](auto pset, bool first, auto two) __attribute__((always_inline)) {
         constexpr int P = decltype(pset)::value;
         const char *sa = smem + (it % NSA) * ST_A, *sw = smem + W_OFF + (it % NSW) * ST_W;
         auto rd_a = [&](int s) __attribute__((always_inline)) {
@@ -247,13 +269,13 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
             wf[P][j][0] = *reinterpret_cast<const g16_v4f*>(sw + w_off + j * 16 * 128);
             wf[P][j][1] = *reinterpret_cast<const g16_v4f*>(sw + (w_off ^ FX) + j * 16 * 128);
         }
-        if (!first) mfma_step(NS - 1, 1, P ^ 1);   // the previous k-tile's last step
+        if (!first) mfma_step(NS - 1, 1, P ^ 1, two);   // the previous k-tile's last step
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            if (s == 0) issue_w();
-            if (s == 1) issue_a();
+            if (s == 0) issue_w(it + DW);
+            if (s == 1) issue_a(it + DA);
             if (s + 1 < NS) rd_a(s + 1);
-            if (s + 1 < NS) mfma_step(s, s & 1, P);
+            if (s + 1 < NS) mfma_step(s, s & 1, P, two);
         }
         ++it;
     };
@@ -263,7 +285,7 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
     auto epilogue = [&](int t) __attribute__((always_inline)) {
         const int u = u0 + t * ustep, split = u / ntiles, tile = u - split * ntiles;
         const int mt = tile / ntn, wrow = mt * BM + wm * WM, n0 = (tile - mt * ntn) * BN;
-        char* const cb = static_cast<char*>(p.C) + (int64_t)split * p.split_stride * CES;
+        char* const cb = static_cast<char*>(p.C) + (EPI == EPI_NONE ? (int64_t)split * p.split_stride * CES : 0);
         const int64_t rowb = p.ldc * CES;
         // lane-derived values opaque here: formed at the epilogue, not held across the k-loop
         int el = lane;
@@ -337,11 +359,11 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
     // ahead (whose mark is its W), else W first.
     a_at(0);
     w_at_tile(0);
-    if constexpr (DA > DW) issue_a();
+    if constexpr (DA > DW) issue_a(0);
 #pragma unroll
     for (int d = 0; d < DW; ++d) {
-        issue_w();
-        issue_a();
+        issue_w(d);
+        issue_a(d + DA - DW);
         if constexpr (DA == DW) mark[d] = vm;
     }
     if constexpr (DA > DW) static_assert(DW == 1, "one mark");
@@ -361,16 +383,30 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
                 for (int i = 0; i < FM; ++i) acc[i][j] = b;
             }
         }
-        run_ktile(set0{}, true);
+        if constexpr (REST) {                      // the smallest products, while the sums are small
+            run_ktile(set0{}, true, std::true_type{});
+            enter();
+            run_ktile(set1{}, false, std::true_type{});
+            for (int kt = 2; kt < nr; kt += 2) {
+                enter();
+                run_ktile(set0{}, false, std::true_type{});
+                enter();
+                run_ktile(set1{}, false, std::true_type{});
+            }
+            mfma_step(NS - 1, 1, 1, std::true_type{});
+            enter();
+        }
+        typedef std::integral_constant<bool, !PAIR> two;
+        run_ktile(set0{}, true, two{});
         enter();
-        run_ktile(set1{}, false);
+        run_ktile(set1{}, false, two{});
         for (int kt = 2; kt < nk; kt += 2) {
             enter();
-            run_ktile(set0{}, false);
+            run_ktile(set0{}, false, two{});
             enter();
-            run_ktile(set1{}, false);
+            run_ktile(set1{}, false, two{});
         }
-        mfma_step(NS - 1, 1, 1);
+        mfma_step(NS - 1, 1, 1, two{});
         epilogue(t);
     }
 }
@@ -385,6 +421,7 @@ __device__ __forceinline__ void gemm16_body(const Gemm16Args& p, const int M, ch
 struct TileCost {
     int bm, bn, wpc;
     float launch, epi, epi_gelu, kt[2];
+    float rest;                                  // a k-tile of the rest, in pair k-tiles
 };
 constexpr int FAM_TILES = 4;                     // tiles per family
 struct TileFamily {
@@ -409,7 +446,7 @@ __host__ __device__ inline float choice_us(const TileChoice& c, int i, int M) {
     return c.t[i].launch + (float)full * c.t[i].full + (float)rem * c.t[i].rem;
 }
 
-template <bool PAIR, int FAM, int EPI, int OUT>
+template <bool PAIR, bool REST, int FAM, int EPI, int OUT>
 __global__ __launch_bounds__(FAM == 0 ? 512 : 256, 2) void gemm16_kernel(Gemm16Args p, TileChoice f) {
     constexpr bool HB = EPI != EPI_NONE;
     // With no bias row to keep, 256 x 256 and 128 x 128 have room for a third A stage.
@@ -430,15 +467,15 @@ __global__ __launch_bounds__(FAM == 0 ? 512 : 256, 2) void gemm16_kernel(Gemm16A
     }
     tile = __builtin_amdgcn_readfirstlane(tile);
     if constexpr (FAM == 0) {
-        if (tile == 0) gemm16_body<PAIR, 256, 256, 2, 4, NA0, 2, EPI, OUT>(p, M, smem);
-        else if (tile == 1) gemm16_body<PAIR, 256, 192, 4, 2, 3, 2, EPI, OUT>(p, M, smem);
-        else if (tile == 2) gemm16_body<PAIR, 256, 128, 4, 2, 3, 3, EPI, OUT>(p, M, smem);
-        else gemm16_body<PAIR, 128, 128, 2, 4, 4, 4, EPI, OUT>(p, M, smem);
+        if (tile == 0) gemm16_body<PAIR, REST, 256, 256, 2, 4, NA0, 2, EPI, OUT>(p, M, smem);
+        else if (tile == 1) gemm16_body<PAIR, REST, 256, 192, 4, 2, 3, 2, EPI, OUT>(p, M, smem);
+        else if (tile == 2) gemm16_body<PAIR, REST, 256, 128, 4, 2, 3, 3, EPI, OUT>(p, M, smem);
+        else gemm16_body<PAIR, REST, 128, 128, 2, 4, 4, 4, EPI, OUT>(p, M, smem);
     } else {
-        if (tile == 0) gemm16_body<PAIR, 128, 128, 2, 2, NA0, 2, EPI, OUT>(p, M, smem);
-        else if (tile == 1) gemm16_body<PAIR, 128, 96, 4, 1, 3, 2, EPI, OUT>(p, M, smem);
-        else if (tile == 2) gemm16_body<PAIR, 64, 128, 2, 2, 3, 3, EPI, OUT>(p, M, smem);
-        else gemm16_body<PAIR, 64, 64, 2, 2, 4, 4, EPI, OUT>(p, M, smem);
+        if (tile == 0) gemm16_body<PAIR, REST, 128, 128, 2, 2, NA0, 2, EPI, OUT>(p, M, smem);
+        else if (tile == 1) gemm16_body<PAIR, REST, 128, 96, 4, 1, 3, 2, EPI, OUT>(p, M, smem);
+        else if (tile == 2) gemm16_body<PAIR, REST, 64, 128, 2, 2, 3, 3, EPI, OUT>(p, M, smem);
+        else gemm16_body<PAIR, REST, 64, 64, 2, 2, 4, 4, EPI, OUT>(p, M, smem);
     }
 }
 

@@ -61,19 +61,20 @@ struct Gemm16Args {
     float acc_scale;     // pairs: 1 / (scale of A * scale of W)
     float out_scale;     // scale of a pair output
     int tile;            // within the kernel's family; -1: the kernel picks by the row count
+    bool rest;           // pairs: W rows of launch_to_pair_rest (ldw >= 3 K / 2), and their rest takes part
 };
 
 // Tile family and split count the 16-bit products take for a shape: gelu is the
 // FFN up epilogue's cost; split counts from min_splits to max_splits are weighed
 // (above 1 for EPI_NONE only).  exact: M is the row count; else it is the
-// padded one, of which a ragged batch fills a part.
+// padded one, of which a ragged batch fills a part.  rest: Gemm16Args::rest.
 struct Gemm16Plan {
     int family, splits;
 };
-Gemm16Plan gemm16_pair_plan(int M, bool exact, int N, int K, bool gelu, int min_splits, int max_splits,
+Gemm16Plan gemm16_pair_plan(int M, bool exact, int N, int K, bool gelu, int min_splits, int max_splits, bool rest,
                             double* us = nullptr);
 constexpr int GEMM16_TILES = 8;   // tile t is number t % 4 of family t / 4
-// N % 8 == 0, K % (64 * splits) == 0, strides multiples of 8 elements and at
+// N % 8 == 0, K % (64 * splits) == 0 (with the rest: 128 * splits), strides multiples of 8 elements and at
 // most gemm_stride_max(4), 16-byte aligned operands (hipErrorInvalidValue
 // otherwise).  out_pair: C as pairs of scale out_scale, with EPI_BIAS and
 // EPI_BIAS_GELU; fp32 with EPI_NONE.
@@ -90,6 +91,7 @@ struct FfnPairArgs {
     int M_max;
     const int* M_dev;
     int I, splits;
+    int64_t ldw1, ldw2;   // row strides (words) of W1 and W2
     int64_t split_stride;
     float scale1, scale_g, scale2;   // 1 / (sX sW1), the GELU output's scale, 1 / (scale_g sW2)
 };
@@ -101,7 +103,7 @@ struct FfnPairPlan {
     int splits;
     Gemm16Plan up, down;   // not fused
 };
-FfnPairPlan ffn_pair_plan(int M, bool exact, int H, int I, int min_splits, int max_splits);
+FfnPairPlan ffn_pair_plan(int M, bool exact, int H, int I, int min_splits, int max_splits, bool rest);
 hipError_t launch_ffn_pair(const FfnPairArgs& a, hipStream_t s);
 // The bf16 products of launch_gemm_bf16_act (bf16 C, N and ldc multiples of 8,
 // aligned operands) on the tiles of gemm16.hpp: false, and nothing launched,
@@ -109,6 +111,10 @@ hipError_t launch_ffn_pair(const FfnPairArgs& a, hipStream_t s);
 bool launch_gemm16_bf16(const GemmArgs& a, int epi, hipStream_t s, hipError_t* err);
 // y = the pairs of scale * x, n a multiple of 8.
 hipError_t launch_to_pair(const float* x, uint32_t* y, int64_t n, float scale, hipStream_t s);
+// Weights [N, K] as rows of 3 K / 2 words: the row's pairs, then its rest,
+// fp16(scale * x - h - l) in order of k, which is exact down to fp16's smallest
+// step.  K a multiple of 8, x and y 16-byte aligned.
+hipError_t launch_to_pair_rest(const float* x, uint32_t* y, int64_t N, int K, float scale, hipStream_t s);
 // norm2[n], amax[n]: each row's sum of squares and largest magnitude (NaN if
 // the row has one), W [N, K].
 hipError_t launch_row_stats(const float* W, int N, int K, float* norm2, float* amax, hipStream_t s);

@@ -40,7 +40,14 @@ extern "C" {
 #define EBH_ERR_HIP (-5)         /* HIP runtime failure                         */
 #define EBH_ERR_RANGE (-6)       /* token id >= vocab, S > max positions, ...   */
 
-#define EBH_DTYPE_F32 0  /* fp32 GEMMs (parity path)                          */
+/* fp32 weights, activations and sums (parity path).  Products run on fp32 MFMA
+ * or, above 64 positions, on operands held as pairs of fp16 numbers (23 of 24
+ * bits; the weights' 24th beside them on longer sequences and in deeper models),
+ * by a rule on the padded length, the layers and the weights' range under which
+ * the vectors' error against fp64 is on average no larger than fp32 MFMA's
+ * (ebh_op_products in edgebert_hip_ops.h says which a model takes).
+ * EBH_DTYPE_F32_BF16X6 holds all 24 bits of every operand. */
+#define EBH_DTYPE_F32 0
 #define EBH_DTYPE_BF16 1 /* bf16 GEMM inputs, fp32 accumulate; LN/softmax fp32 */
 /* fp32 model (fp32 weights and activations, everything else as EBH_DTYPE_F32)
  * whose GEMMs form each fp32 product from bf16 MFMA products: both operands

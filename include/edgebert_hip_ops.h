@@ -52,7 +52,16 @@ EBH_API int ebh_op_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, 
                      const float* bias, void* C, int64_t ldc, int32_t c_dtype, int32_t M, int32_t N,
                      int32_t K, int32_t epilogue, void* stream);
 
-/* fp32 products from fp16 pairs, as the fp32 forward runs them above 64 tokens
+/* How a finalized model forms its products over [B, S] positions: fp32 models on
+ * fp32 MFMA, on fp16 pairs or on pairs with the weights' rest; other models as
+ * their dtype says.  Negative: an error code. */
+#define EBH_PRODUCTS_MFMA 0
+#define EBH_PRODUCTS_PAIR 1
+#define EBH_PRODUCTS_PAIR_REST 2
+#define EBH_PRODUCTS_DTYPE 3
+EBH_API int ebh_op_products(const ebh_model* m, int32_t B, int32_t S);
+
+/* fp32 products from fp16 pairs, as the fp32 forward may run them
  * (src/lib.rs:691-698, 732-733, 741-747, 795-849, 958-978): A [M, K] and W
  * [N, K] in the pair format of ebh_op_to_pair with scales sA and sW, acc_scale
  * = 1 / (sA * sW).  c_scale > 0: C [M, N] as pairs of that scale, epilogue
@@ -60,10 +69,18 @@ EBH_API int ebh_op_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, 
  * splits > 1 (EBH_EPI_NONE): split s sums k in [s K / splits, (s + 1) K /
  * splits) into C + s * split_stride.  tile: -1 (chosen by the shape), or one of 0 .. 7
  * (256x256, 256x192, 256x128 and 128x128 on 8 waves; 128x128, 128x96, 64x128
- * and 64x64 on 4); the result does not depend on it.  N % 8 == 0, K % (64 splits) == 0, strides (elements) multiples of 8
- * and at most 2,796,202, 16-byte aligned operands (EBH_ERR_INVALID_ARG
+ * and 64x64 on 4); the result does not depend on it.  N % 8 == 0,
+ * K % (64 splits) == 0, strides (elements) multiples of 8 and at most
+ * 2,796,202, 16-byte aligned operands (EBH_ERR_INVALID_ARG
  * otherwise). */
 EBH_API int ebh_op_gemm_pair(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t ldw, float acc_scale,
+                     const float* bias, void* C, int64_t ldc, float c_scale, int32_t M, int32_t N, int32_t K,
+                     int32_t epilogue, int32_t splits, int64_t split_stride, int32_t tile, void* stream);
+
+/* The same product with the weights' rest: W rows are ebh_op_to_pair_rest's (ldw at
+ * least 3 K / 2), and each product adds ah.br, which makes the weights exact;
+ * K % (128 splits) == 0. */
+EBH_API int ebh_op_gemm_pair_rest(const uint32_t* A, int64_t lda, const uint32_t* W, int64_t ldw, float acc_scale,
                      const float* bias, void* C, int64_t ldc, float c_scale, int32_t M, int32_t N, int32_t K,
                      int32_t epilogue, int32_t splits, int64_t split_stride, int32_t tile, void* stream);
 
@@ -82,6 +99,12 @@ EBH_API int ebh_op_ffn_pair(const uint32_t* X, const uint32_t* W1, const float* 
  * fp16 h = fp16(v) and eight fp16 l = fp16(v - h), round to nearest even (32
  * bytes); scale a power of two, n a multiple of 8, x and y 16-byte aligned. */
 EBH_API int ebh_op_to_pair(const float* x, uint32_t* y, int64_t n, float scale, void* stream);
+
+/* Weights [N, K] as rows of 3 K / 2 words: the K values in the pair format, then
+ * their rests r = fp16(scale * w - h - l) in order (two to a word).  h + l + r
+ * is scale * w down to fp16's smallest step.  K a multiple of 8, w and y 16-byte
+ * aligned. */
+EBH_API int ebh_op_to_pair_rest(const float* w, uint32_t* y, int32_t N, int32_t K, float scale, void* stream);
 
 /* Masked multi-head attention (src/lib.rs:700-730 with 851-956) over packed
  * sequences: qkv [T, 3*hidden] rows (q | k | v), sequence b = rows

@@ -32,6 +32,12 @@ def to_pair(torch, N, L, x, scale, s):
     return y
 
 
+def to_pair_rest(torch, N, L, w, scale, s):
+    y = torch.empty(w.shape[0], w.shape[1] * 3 // 2, device="cuda")
+    N.check(L.ebh_op_to_pair_rest(vp(w), vp(y), w.shape[0], w.shape[1], scale, s))
+    return y
+
+
 def unpair(torch, y, scale):
     h = y.view(torch.float16).view(y.shape[0], -1, 2, 8).double()
     return ((h[:, :, 0] + h[:, :, 1]) / scale).reshape(y.shape[0], -1)
@@ -111,25 +117,77 @@ def test_gemm_pair(env, M, Nn, K, S, tile):
     assert padding_kept(D)
 
 
+# K: two, three and twelve pairs of the rest's k-tiles, split and not
+@pytest.mark.parametrize("K,S", [(128, 1), (256, 2), (384, 1), (384, 3), (1536, 4)])
+def test_rest_makes_weights_exact(env, K, S):
+    """Rows of the identity pick out the weights: with the rest every one of them
+    comes back as it is, at every k, on every tile; without it, a quarter do not."""
+    torch, eb, N, L = env
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator(device="cuda").manual_seed(K)
+    W = 0.04 * torch.randn(200, K, device="cuda", generator=g)
+    sw = 2.0 ** 16
+    A = to_pair(torch, N, L, torch.eye(K, device="cuda"), 1.0, s)
+    Wr = to_pair_rest(torch, N, L, W, sw, s)
+    halves = Wr[:, K:].contiguous().view(torch.float16).double()
+    # below 1/2 (scaled) a value's 24th bit is less than fp16's smallest step, 2^-24
+    exact = W.abs() * sw >= 0.5
+    assert exact.float().mean().item() > 0.999
+    assert torch.equal((unpair(torch, Wr[:, :K].contiguous(), sw) + halves / sw)[exact], W.double()[exact])
+
+    def product(f, W, ldw, tile):
+        C = torch.empty(S, K, 200, device="cuda")
+        N.check(f(vp(A), K, vp(W), ldw, 1 / sw, None, vp(C), 200, 0.0, K, 200, K, EPI_NONE, S, K * 200, tile, s))
+        return C.sum(0).t()            # one split holds the value, the others zeros
+
+    for tile in range(-1, 8):
+        assert torch.equal(product(L.ebh_op_gemm_pair_rest, Wr, K * 3 // 2, tile)[exact], W[exact])
+    off = product(L.ebh_op_gemm_pair, Wr, K * 3 // 2, -1) != W
+    assert 0.2 < off.float().mean().item() < 0.3
+    assert L.ebh_op_gemm_pair_rest(vp(A), K, vp(Wr), K, 1 / sw, None, vp(Wr), 200, 0.0, K, 200, K, EPI_NONE, 1, 0, -1,
+                                   s) == N.EBH_ERR_INVALID_ARG      # rows without room for the rest
+    assert L.ebh_op_gemm_pair_rest(vp(A), K, vp(Wr), K * 3 // 2, 1 / sw, None, vp(Wr), 200, 0.0, K, 200, 64, EPI_NONE, 1,
+                                   0, -1, s) == N.EBH_ERR_INVALID_ARG
+
+
+def test_products_by_length_and_depth(env, weights_for):
+    """Where fp32 models take pairs, pairs with the rest and fp32 MFMA products."""
+    torch, eb, N, L = env
+    mfma, pair, rest = 0, 1, 2
+    wide = dict(vocab_size=50, max_position_embeddings=512, layer_norm_eps=1e-12)
+    deep = eb.BertConfig(hidden_size=128, num_attention_heads=4, num_hidden_layers=12, intermediate_size=256, **wide)
+    narrow = eb.BertConfig(hidden_size=64, num_attention_heads=2, num_hidden_layers=2, intermediate_size=256, **wide)
+    for cfg, want in ((eb.MINILM_L6, {(1, 64): mfma, (1, 65): pair, (300, 128): pair, (1, 129): rest, (8, 512): rest}),
+                      (narrow, {(30, 128): pair, (30, 129): mfma}),       # K = 64: no rest
+                      (deep, {(2, 64): pair, (2, 65): rest, (2, 192): rest, (2, 193): mfma, (1, 64): mfma})):
+        m = eb.Model.from_weights(weights_for(cfg), cfg, "fp32")
+        try:
+            got = {k: L.ebh_op_products(m._h, *k) for k in want}
+        finally:
+            m.close()
+        assert got == want
+
+
 # at least three items for every workgroup on every tile, in whole rounds of
 # 256 x 256 tiles and not, rows and columns ending inside a tile; tiles of two
 # k-tiles, of four and of more.  The columns of a workgroup's items differ, and so
 # do their biases.
 @pytest.mark.parametrize("M,Nn", [(8187, 6136), (8450, 6392)])
-@pytest.mark.parametrize("K,S", [(64, 1), (128, 2), (384, 3)])
-def test_gemm_pair_many_tiles(env, M, Nn, K, S):
+@pytest.mark.parametrize("K,S,rest", [(64, 1, False), (128, 2, False), (384, 3, False), (128, 1, True), (384, 3, True)])
+def test_gemm_pair_many_tiles(env, M, Nn, K, S, rest):
     torch, eb, N, L = env
     s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     g = torch.Generator(device="cuda").manual_seed(M + K)
     A, W = torch.randn(M, K, device="cuda", generator=g), 0.04 * torch.randn(Nn, K, device="cuda", generator=g)
     b = 3 * torch.randn(Nn, device="cuda", generator=g)
     sa, sw, sc = 2.0 ** 8, 2.0 ** 14, 2.0 ** 4
-    Ap, Wp = to_pair(torch, N, L, A, sa, s), to_pair(torch, N, L, W, sw, s)
+    Ap, Wp = to_pair(torch, N, L, A, sa, s), (to_pair_rest if rest else to_pair)(torch, N, L, W, sw, s)
+    product = L.ebh_op_gemm_pair_rest if rest else L.ebh_op_gemm_pair
 
     def run(tile, epi, splits=1):
         C = torch.empty(splits, M, Nn, device="cuda")
-        N.check(L.ebh_op_gemm_pair(vp(Ap), K, vp(Wp), K, 1 / (sa * sw), vp(b) if epi != EPI_NONE else None, vp(C), Nn,
-                                   sc if epi != EPI_NONE else 0.0, M, Nn, K, epi, splits, M * Nn, tile, s))
+        N.check(product(vp(Ap), K, vp(Wp), Wp.shape[1], 1 / (sa * sw), vp(b) if epi != EPI_NONE else None, vp(C), Nn,
+                        sc if epi != EPI_NONE else 0.0, M, Nn, K, epi, splits, M * Nn, tile, s))
         return C
 
     ref = A.double() @ W.double().t()

@@ -290,10 +290,11 @@ size_t layout_workspace(const ebh_model* m, int64_t tcap, int bcap, char* base, 
     const size_t H = c.hidden_size, I = c.intermediate_size;
     const bool b16 = m->dtype == EBH_DTYPE_BF16;
     int64_t yparts = y_parts_for(m, tcap);
-    // Split counts fall at whole 64-row tiles; partials may run on into QKV's
-    // three rows a position (enqueue_pair_layers).
+    // Split counts fall at whole 64-row tiles.  (Pair forwards' partials may
+    // also run on into QKV's three rows a position, enqueue_pair_layers; the
+    // others', the few-token ones among them, have Y alone.)
     for (int64_t T = 64; any_fewer && T < tcap; T += 64)
-        yparts = std::max(yparts, ((int64_t)(y_parts_for(m, T) + 3) * T + tcap - 1) / tcap - 3);
+        yparts = std::max(yparts, ((int64_t)y_parts_for(m, T) * T + tcap - 1) / tcap);
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off += align_up(std::max<size_t>(bytes, 1)); return o; };
     const size_t oErr = take(4), oX = take(b16 ? 0 : tcap * H * 4), oX16 = take(b16 ? tcap * H * 2 : 0),

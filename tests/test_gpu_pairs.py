@@ -379,8 +379,13 @@ def test_models_at_the_ends_of_the_range(env, weights_for, how):
     assert np.abs(got - want).max() <= 1e-5
 
 
-@pytest.mark.parametrize("B,S,after", [(3, 22, (6, 60)), (5, 128, (20, 67)), (40, 50, (43, 64)), (63, 128, (65, 128))])
-def test_vectors_do_not_depend_on_earlier_batches(env, weights_for, B, S, after):
+# pairs; pairs with the rest; the few-token kernels (a partial per head) at the
+# workspace sizes just above their own; products whose operands are not pairs
+@pytest.mark.parametrize("dtype,B,S,after", [
+    ("fp32", 3, 22, (6, 60)), ("fp32", 5, 128, (20, 67)), ("fp32", 40, 50, (43, 64)), ("fp32", 63, 128, (65, 128)),
+    ("fp32", 5, 140, (4, 201)), ("fp32", 4, 16, (5, 16)), ("fp32", 1, 64, (1, 95)), ("fp32", 2, 31, (3, 31)),
+    ("fp32-bf16x6", 4, 16, (5, 16)), ("fp32-bf16x6", 21, 64, (26, 64)), ("fp32-bf16x6", 3, 64, (67, 128))])
+def test_vectors_do_not_depend_on_earlier_batches(env, weights_for, dtype, B, S, after):
     """A batch gives the same bits in a fresh model and in one whose workspace a
     larger batch has grown (a product's split count goes by the batch alone)."""
     torch, eb, N, L = env
@@ -392,7 +397,7 @@ def test_vectors_do_not_depend_on_earlier_batches(env, weights_for, B, S, after)
         return rng.integers(10, cfg.vocab_size, (b, s)).astype(np.uint32), np.ones((b, s), np.uint32)
 
     ids, mask = batch(B, S)
-    fresh, grown = eb.Model.from_weights(w, cfg, "fp32"), eb.Model.from_weights(w, cfg, "fp32")
+    fresh, grown = eb.Model.from_weights(w, cfg, dtype), eb.Model.from_weights(w, cfg, dtype)
     try:
         want = fresh.encode_ids(ids, mask)
         grown.encode_ids(*batch(*after))

@@ -1098,16 +1098,23 @@ static int prepare_pairs(ebh_model* m) {
         if (!std::isfinite(ss)) return Norm{NAN, NAN, NAN};   // std::max loses a NaN
         return Norm{mx, median(std::move(size)), gm * root + std::sqrt(bb)};
     };
-    // Bound and typical size of the rows of x . w^T + b.
-    auto out_scale = [&](const float* n2, const float* b, size_t n, const Norm& x) {
-        double mx = 0, ss = 0;
-        std::vector<double> size(n);
-        for (size_t i = 0; i < n; ++i) {
-            const double w = std::sqrt((double)n2[i]), bi = std::fabs((double)b[i]);
-            mx = std::max(mx, w * x.norm + bi);
-            ss += size[i] = w * x.typ + bi;
+    // Bound and typical size of the rows of x . w^T + b.  parts: that many equal
+    // runs of rows share the scale (q, k and v), and the typical size is the
+    // smallest of theirs.
+    auto out_scale = [&](const float* n2, const float* b, size_t n, const Norm& x, size_t parts = 1) {
+        double mx = 0, ss = 0, typ = 1e300;
+        for (size_t part = 0; part < parts; ++part) {
+            std::vector<double> size(n / parts);
+            for (size_t i = 0; i < size.size(); ++i) {
+                const size_t row = part * size.size() + i;
+                const double w = std::sqrt((double)n2[row]), bi = std::fabs((double)b[row]);
+                mx = std::max(mx, w * x.norm + bi);
+                ss += size[i] = w * x.typ + bi;
+            }
+            if (!std::isfinite(ss)) return 0.0f;
+            typ = std::min(typ, median(std::move(size)));
         }
-        return std::isfinite(ss) ? pair_scale(mx, median(std::move(size)), kActLimit) : 0.0f;
+        return pair_scale(mx, typ, kActLimit);
     };
     auto weight_scale = [&](const float* n2, const float* am, size_t n) {
         double mx = 0, mn = 1e300, sum = 0;
@@ -1126,7 +1133,7 @@ static int prepare_pairs(ebh_model* m) {
         const Norm mid = norm_of(p, p + H);
         PairScales& q = sc[l];
         q.x = pair_scale(in.max, in.typ, kActLimit);
-        q.qkv = out_scale(n2, p + 4 * H, 3 * H, in);
+        q.qkv = out_scale(n2, p + 4 * H, 3 * H, in, 3);
         q.ctx = out_scale(n2 + 2 * H, p + 6 * H, H, in);
         q.mid = pair_scale(mid.max, mid.typ, kActLimit);
         q.f = out_scale(n2 + 4 * H, p + 7 * H, I, mid);

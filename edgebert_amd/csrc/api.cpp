@@ -1043,11 +1043,14 @@ static float pair_scale(double bound, double typ, double limit) {
 // |w| |x| + |b|; the context is a mean of v rows, and |gelu(u)| <= |u|.  So no
 // input can overflow an operand.  Where a scale would leave the range in which
 // pairs are as exact as fp32 products (pair_scale), or a shape is not whole
-// 64-wide k-tiles, the model keeps the fp32 kernels throughout.
+// 64-wide k-tiles or has rows too long for the pair products, the model keeps
+// the fp32 kernels throughout.
 static int prepare_pairs(ebh_model* m) {
     const ebh_config& c = m->cfg;
     const size_t H = c.hidden_size, I = c.intermediate_size, L = m->layers.size();
-    if (H % 64 || I % 64 || L == 0 || !ebh::row4_shape_ok((int)H)) return EBH_OK;
+    if (H % 64 || I % 64 || L == 0 || !ebh::row4_shape_ok((int)H) ||
+        !ebh::gemm_offsets_fit32((int64_t)std::max(H, I) * 3 / 2, (int64_t)std::max(H, I) * 3 / 2, 4))
+        return EBH_OK;
     hipStream_t st = m->stream;
     const size_t rows = 3 * H + H + I + H;               // weight rows of a layer
     float* d_stats = nullptr;

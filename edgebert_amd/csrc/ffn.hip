@@ -268,11 +268,13 @@ __global__ __launch_bounds__(512, 2) void ffn_pair_kernel(FfnPairArgs p) {
 
 }  // namespace
 
-bool ffn_pair_shape_ok(int H, int I) { return H == FH && I > 0 && I % FBC == 0; }
+constexpr int FFN_MAX_I = (1 << 20) / 4;   // 384 rows of W2, 6 bytes an element, below 2^32 bytes
+
+bool ffn_pair_shape_ok(int H, int I) { return H == FH && I > 0 && I % FBC == 0 && I <= FFN_MAX_I; }
 
 hipError_t launch_ffn_pair(const FfnPairArgs& a, hipStream_t s) {
     auto al16 = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
-    if (a.M_max < 0 || a.I <= 0 || a.I % FBC || a.splits < 1 || (a.I / FBC) % a.splits || a.I > (1 << 20) / 4 ||
+    if (a.M_max < 0 || a.I <= 0 || a.I % FBC || a.splits < 1 || (a.I / FBC) % a.splits || a.I > FFN_MAX_I ||
         a.ldw1 < FH || a.ldw2 < a.I || a.ldw1 % 4 || a.ldw2 % 4 || a.ldw1 > (1 << 20) || a.ldw2 > (1 << 20) ||
         !al16(a.X) || !al16(a.W1) || !al16(a.W2) || !al16(a.b1) || !al16(a.Y) || a.split_stride % 4)
         return hipErrorInvalidValue;

@@ -385,6 +385,38 @@ def test_models_at_the_ends_of_the_range(env, weights_for, how, products):
     assert np.abs(got - want).max() <= (5e-6 if how == "outlier_gain" else 5e-7)
 
 
+def test_rows_too_long_for_the_pair_products(env):
+    """An FFN of 1.9 million columns is beyond the pair products' 32-bit row offsets:
+    the model keeps the fp32 kernels."""
+    torch, eb, N, L = env
+    cfg = eb.BertConfig(hidden_size=64, num_attention_heads=2, num_hidden_layers=1, intermediate_size=1_900_032,
+                        vocab_size=50, max_position_embeddings=32, layer_norm_eps=1e-12)
+    r = np.random.default_rng(1)
+    shapes = {"embeddings.word_embeddings.weight": (50, 64), "embeddings.position_embeddings.weight": (32, 64),
+              "embeddings.token_type_embeddings.weight": (2, 64)}
+    w = {k: r.standard_normal(s).astype(np.float32) for k, s in shapes.items()}
+    for k in ("embeddings.", "encoder.layer.0.attention.output.", "encoder.layer.0.output."):
+        w[k + "LayerNorm.weight"], w[k + "LayerNorm.bias"] = np.ones(64, np.float32), np.zeros(64, np.float32)
+    for k, n, m in (("attention.self.query", 64, 64), ("attention.self.key", 64, 64), ("attention.self.value", 64, 64),
+                    ("attention.output.dense", 64, 64), ("intermediate.dense", cfg.intermediate_size, 64),
+                    ("output.dense", 64, cfg.intermediate_size)):
+        w["encoder.layer.0." + k + ".weight"] = np.float32(0.04) * r.standard_normal((n, m), dtype=np.float32)
+        w["encoder.layer.0." + k + ".bias"] = np.zeros(n, np.float32)
+    ids, mask = r.integers(0, 50, (5, 20)).astype(np.uint32), np.ones((5, 20), np.uint32)
+    got = []
+    for dtype in ("fp32", "fp32-bf16x6"):
+        m = eb.Model.from_weights(w, cfg, dtype)
+        try:
+            got.append(m.encode_ids(ids, mask))
+        finally:
+            m.close()
+    # Sums of n = 1.9 million terms of random signs in two orders: a partial sum S_k
+    # is rounded by up to 2^-24 |S_k|, and |S_k|^2 grows as k, so each order is off
+    # by some sqrt(n / 2) 2^-24 / sqrt(3) = 3e-5 of the sum's norm, at most the unit
+    # vector's, and both by twice that at most
+    assert np.isfinite(got[0]).all() and np.linalg.norm(got[0] - got[1], axis=1).max() <= 7e-5
+
+
 # pairs; pairs with the rest; the few-token kernels (a partial per head) at the
 # workspace sizes just above their own; products whose operands are not pairs
 @pytest.mark.parametrize("dtype,B,S,after", [

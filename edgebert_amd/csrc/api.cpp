@@ -1054,7 +1054,10 @@ static int prepare_pairs(ebh_model* m) {
     hipStream_t st = m->stream;
     const size_t rows = 3 * H + H + I + H;               // weight rows of a layer
     float* d_stats = nullptr;
-    HIP_TRY(hipMalloc((void**)&d_stats, L * rows * 2 * sizeof(float)));
+    if (hipMalloc((void**)&d_stats, L * rows * 2 * sizeof(float)) != hipSuccess) {   // no room: the fp32 kernels need none
+        (void)hipGetLastError();
+        return EBH_OK;
+    }
     std::unique_ptr<void, hipError_t (*)(void*)> stats_guard(d_stats, hipFree);
     std::vector<float> stats(L * rows * 2);
     for (size_t l = 0; l < L; ++l) {
@@ -1149,7 +1152,7 @@ static int prepare_pairs(ebh_model* m) {
         in = norm_of(p + 2 * H, p + 3 * H);
     }
     const size_t words = (4 * H * H + 2 * H * I) * 3 / 2;   // pair weights of a layer, with their rests
-    if (hipMalloc(&m->wpair, L * words * 4) != hipSuccess) {   // no room: the fp32 kernels need none
+    if (hipMalloc(&m->wpair, L * words * 4) != hipSuccess) {   // as above
         (void)hipGetLastError();
         m->wpair = nullptr;
         return EBH_OK;

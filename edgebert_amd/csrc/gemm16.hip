@@ -82,7 +82,9 @@ hipError_t launch_row_stats(const float* W, int N, int K, float* norm2, float* a
 // ---------------------------------------------------------------------------
 // Family and tile choice: the cost model of gemm16.hpp with constants fitted to
 // a sweep on MI355X of the four products of MiniLM and BERT-base at 96 ..
-// 40,000 rows (bf16: .. 131,072) and 1 .. 6 splits (rms error of a fit 5-10%).
+// 40,000 rows (bf16: .. 131,072) and 1 .. 6 splits (rms error of a fit 5-10%;
+// least where operands come from a cache: MiniLM's two FFN products at 32,768
+// rows take 205 us, 172 by the tables).
 // What the numbers say: a 256-wide tile runs its k-loop fastest but pays a long
 // epilogue (its C is all of a CU's stores), so it wins on many rounds or a long
 // K; small tiles, two workgroups per CU, keep a small job on all CUs.  Each split
@@ -174,10 +176,14 @@ Gemm16Plan gemm16_pair_plan(int M, bool exact, int N, int K, bool gelu, int min_
 
 // ffn_pair_kernel: rounds of one workgroup per CU; a chunk of 128 intermediate
 // columns takes 12.6 us with up to half of the CUs at work and 16.6 us with all
-// (measured at 256 .. 40,000 rows, 1 .. 12 splits; 14,355 rows: 105 us in 2
-// splits, the two products 108 on their best tiles).  The estimate is weighed
-// at 0.95: in a forward the products lose more against these back-to-back
-// timings than this kernel does (32,768 rows: 203 -> 233 us against 201 -> 224).
+// (measured at 256 .. 40,000 rows, 1 .. 12 splits).  Back to back the two forms
+// are within 10% of one another from 6,000 to 33,000 rows of I = 1536 (us, fused
+// in its best splits against the products: 6,124 rows 50.7 / 55.4, 10,000 73.6 /
+// 77.6, 14,313 102.0 / 102.3, 32,768 206 / 205).  The estimate is weighed at
+// 0.95, which decides between forms that close.  In forwards, against no weight:
+// full batches of 6,144 and 8,192 rows 1-2% faster, ragged ones of 60-85% of them
+// 2-6% slower (649 against 611 us at 3,817 of 6,144), and, since this kernel then
+// runs in more splits than the products would, vectors 3% closer to float64.
 static double ffn_us(int M, int I, int S) {
     const int cus = device_cu_count();
     const int64_t items = (int64_t)((M + 127) / 128) * S;
@@ -254,8 +260,8 @@ bool launch_gemm16_bf16(const GemmArgs& g, int epi, hipStream_t s, hipError_t* e
     const bool exact = g.M_dev == nullptr, gelu = epi == EPI_BIAS_GELU;
     int best = -1;
     // The ring kernel's estimate is weighed at 0.92: its three A stages hide what
-    // a forward's cold operands cost the others (131,072 rows, FFN down: 481 us
-    // against 523, where back to back they are within 2%).
+    // a forward's cold operands cost the others (measured at one shape: 131,072
+    // rows, FFN down, 481 us against 523, where back to back they are within 2%).
     const TileChoice ring = choice_for(kBf16Ring, g.N, g.K / 64, gelu, 1, false);
     double best_us = 0.92 * over_fills(g.M_max, exact, [&](int m) { return (double)choice_us(ring, 0, m); });
     for (int i = 0; i < FAMILIES; ++i) {

@@ -261,7 +261,11 @@ EBH_API int ebh_model_info(const ebh_model* m, ebh_config* cfg_out, int32_t* dty
 /* Time one kernel family with HIP events during forwards, on the stream the
  * kernels are launched on.  kernel: one of EBH_PROF_* (EBH_PROF_NONE = off).
  * ebh_profile_read returns the accumulated launch count and total ms since the
- * last ebh_profile_enable, after waiting for the model's work. */
+ * last ebh_profile_enable, after waiting for the model's work.  A launch that
+ * does two families' work counts as one of them: FFN up, GELU and FFN down in one
+ * (some fp32 batches of hidden size 384) as GEMM_FFN_DOWN, attention with the
+ * output projection (at most 64 positions) as ATTENTION; the other then has no
+ * launches. */
 #define EBH_PROF_NONE 0
 #define EBH_PROF_GEMM_QKV 1
 #define EBH_PROF_ATTENTION 2

@@ -57,9 +57,9 @@ enum Out16 : int { OUT_F32 = 0, OUT_PAIR = 1, OUT_BF16 = 2 };
 // Lane group q's operands are chunks 2q and 2q + 1 of a row (pairs: h and l of
 // k = 8q .. 8q + 7), or q and q + 4 (bf16: two 32-deep slices of k, in order).
 // bf16 sums start at the bias and run over the slices, as the ring kernel's
-// (gemm.hip) do, so every tile there is gives a row the same bits and a bf16
-// vector does not depend on the batch it is in.  Pairs add the bias last: their
-// sums hold a scale of their own.  The MFMAs take W
+// (gemm.hip) do, so every tile there is gives a row the same bits, and the tile
+// that a batch's size picks does not show in its vectors.  Pairs add the bias
+// last: their sums hold a scale of their own.  The MFMAs take W
 // as their first operand, so lane (r, q) of a 16 x 16 block holds C row r and
 // the block's W rows 4q .. 4q + 3.  W rows are permuted on their way into LDS
 // (within each 32, LDS row 16 jj + 4q + e holds column 8q + 4 jj + e), so a lane

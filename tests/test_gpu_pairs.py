@@ -1,8 +1,10 @@
-"""fp32 products from fp16 pairs (ebh_op_to_pair, ebh_op_gemm_pair) against float64
-on every tile, at tile edges and remainders; bf16 products at the sizes between
-which their tile changes; and models whose weights lie at
-the ends of the range the pair operands' scales are taken from, or outside it
-(those keep the fp32 kernels), against the CPU oracle."""
+"""fp32 products from fp16 pairs, with and without the weights' rest
+(ebh_op_to_pair, ebh_op_gemm_pair and their _rest forms), against float64 on every
+tile, at tile edges and remainders and over several tiles a workgroup; bf16
+products at the sizes between which their tile changes, bit for bit against the
+ring kernel's; which products a model takes for a batch's shape; and models whose
+weights lie at the ends of the range the pair operands' scales are taken from, or
+outside it (those keep the fp32 kernels), against the CPU oracle."""
 import ctypes
 
 import numpy as np
